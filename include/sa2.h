@@ -121,6 +121,17 @@ int sa2_fwd(const sa2_problem *prob,
             const sa2_tensor *out, const sa2_tensor *out_residual, float *lse,
             const sa2_saved *saved, void *hip_stream);
 
+/* The same with scratch memory: small grids (few rows and heads) are shared by more workgroups, each walking a part of
+ * a query tile's offsets, and a second kernel merges their fp32 results.  workspace may be NULL (or smaller than
+ * sa2_fwd_workspace_bytes(), which is 0 where nothing is gained): the call is then sa2_fwd.  16-byte aligned, needs no
+ * clearing.  Results agree with sa2_fwd's to the order of fp32 sums. */
+int64_t sa2_fwd_workspace_bytes(const sa2_problem *prob);   /* -1 if the problem is invalid */
+int sa2_fwd_ws(const sa2_problem *prob,
+               const sa2_tensor *q, const sa2_tensor *k1, const sa2_tensor *k2,
+               const sa2_tensor *v1, const sa2_tensor *v2,
+               const sa2_tensor *out, const sa2_tensor *out_residual, float *lse,
+               const sa2_saved *saved, void *workspace, int64_t workspace_bytes, void *hip_stream);
+
 /* delta[b,h,n] = sum_d (out + out_residual) * dout; out_residual may be NULL.
  * Replaces backward_preprocess_do_o_dot
  * (triton_two_simplicial_attention.py:834-849; kernel :230-286). */
@@ -173,6 +184,19 @@ int sa2_bwd(const sa2_problem *prob,
             const sa2_tensor *dq, const sa2_tensor *dk1, const sa2_tensor *dk2,
             const sa2_tensor *dv1, const sa2_tensor *dv2,
             void *workspace, int64_t workspace_bytes, void *hip_stream);
+
+/* The same for callers that give scratch memory freely: small grids (few rows and heads) are shared by as many
+ * workgroups as pays, which leave fp32 partial results in the workspace.  workspace: sa2_bwd_split_workspace_bytes(prob,
+ * whether saved is given) bytes.  Results agree with sa2_bwd's to the order of fp32 sums. */
+int64_t sa2_bwd_split_workspace_bytes(const sa2_problem *prob, int with_saved);   /* -1 if the problem is invalid */
+int sa2_bwd_split(const sa2_problem *prob,
+                  const sa2_tensor *q, const sa2_tensor *k1, const sa2_tensor *k2,
+                  const sa2_tensor *v1, const sa2_tensor *v2,
+                  const sa2_tensor *out, const sa2_tensor *out_residual, const sa2_tensor *dout,
+                  const float *lse, const sa2_saved *saved, float *delta_ws,
+                  const sa2_tensor *dq, const sa2_tensor *dk1, const sa2_tensor *dk2,
+                  const sa2_tensor *dv1, const sa2_tensor *dv2,
+                  void *workspace, int64_t workspace_bytes, void *hip_stream);
 
 /* Whole backward for callers that cannot allocate (code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc): sa2_bwd without the delta_ws and workspace arguments.

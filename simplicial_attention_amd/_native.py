@@ -25,8 +25,9 @@ STATUS_NAMES = {
     5: 'SA2_ERR_LAUNCH',
 }
 
-EXPORTS = ('sa2_version', 'sa2_last_error', 'sa2_supported', 'sa2_saved_t_bytes', 'sa2_saved_m_bytes', 'sa2_fwd',
-           'sa2_bwd_delta', 'sa2_bwd_workspace_bytes', 'sa2_bwd_workspace_bytes_with_saved', 'sa2_bwd_dq_dkv2', 'sa2_bwd_dkv1', 'sa2_bwd',
+EXPORTS = ('sa2_version', 'sa2_last_error', 'sa2_supported', 'sa2_saved_t_bytes', 'sa2_saved_m_bytes', 'sa2_fwd', 'sa2_fwd_ws', 'sa2_fwd_workspace_bytes',
+           'sa2_bwd_delta', 'sa2_bwd_workspace_bytes', 'sa2_bwd_workspace_bytes_with_saved',
+           'sa2_bwd_split', 'sa2_bwd_split_workspace_bytes', 'sa2_bwd_dq_dkv2', 'sa2_bwd_dkv1', 'sa2_bwd',
            'sa2_bwd_noalloc_scratch_bytes', 'sa2_bwd_noalloc',
            'sa2_qkv_norm_fwd', 'sa2_qkv_norm_bwd_workspace_bytes', 'sa2_qkv_norm_bwd')
 
@@ -71,7 +72,7 @@ def _declare(lib: ctypes.CDLL) -> ctypes.CDLL:
     S = ctypes.POINTER(Saved)
     I64 = ctypes.c_int64
     for name in ('sa2_saved_t_bytes', 'sa2_saved_m_bytes', 'sa2_bwd_workspace_bytes', 'sa2_bwd_workspace_bytes_with_saved', 'sa2_qkv_norm_bwd_workspace_bytes',
-                 'sa2_bwd_noalloc_scratch_bytes'):
+                 'sa2_bwd_noalloc_scratch_bytes', 'sa2_fwd_workspace_bytes'):
         getattr(lib, name).restype = I64
         getattr(lib, name).argtypes = [P]
     lib.sa2_version.restype = ctypes.c_int
@@ -82,6 +83,10 @@ def _declare(lib: ctypes.CDLL) -> ctypes.CDLL:
     lib.sa2_supported.argtypes = [ctypes.c_int32] * 4
     lib.sa2_fwd.restype = ctypes.c_int
     lib.sa2_fwd.argtypes = [P, T, T, T, T, T, T, T, F, S, V]
+    lib.sa2_fwd_ws.restype = ctypes.c_int
+    lib.sa2_fwd_ws.argtypes = [P, T, T, T, T, T, T, T, F, S, V, I64, V]
+    lib.sa2_bwd_split_workspace_bytes.restype = I64
+    lib.sa2_bwd_split_workspace_bytes.argtypes = [P, ctypes.c_int]
     lib.sa2_bwd_delta.restype = ctypes.c_int
     lib.sa2_bwd_delta.argtypes = [P, T, T, T, F, V]
     lib.sa2_bwd_dq_dkv2.restype = ctypes.c_int
@@ -90,6 +95,8 @@ def _declare(lib: ctypes.CDLL) -> ctypes.CDLL:
     lib.sa2_bwd_dkv1.argtypes = [P, T, T, T, T, T, T, F, F, T, T, V]
     lib.sa2_bwd.restype = ctypes.c_int
     lib.sa2_bwd.argtypes = [P, T, T, T, T, T, T, T, T, F, S, F, T, T, T, T, T, V, I64, V]
+    lib.sa2_bwd_split.restype = ctypes.c_int
+    lib.sa2_bwd_split.argtypes = lib.sa2_bwd.argtypes
     lib.sa2_bwd_noalloc.restype = ctypes.c_int
     lib.sa2_bwd_noalloc.argtypes = [P, T, T, T, T, T, T, T, T, F, S, T, T, T, T, T, V]
     lib.sa2_qkv_norm_fwd.restype = ctypes.c_int

@@ -81,6 +81,7 @@ sa2::KParams base_params(const sa2_problem *p) {
     k.w2 = p->w2;
     k.scale = p->scale;
     k.scale_log2e = p->scale * sa2::kLog2e;
+    k.q_splits = 1;
     return k;
 }
 
@@ -185,9 +186,74 @@ int64_t sa2_saved_m_bytes(const sa2_problem *prob) {
     return (int64_t)prob->batch * prob->heads * prob->w2 * prob->seq_len * 4;
 }
 
-int sa2_fwd(const sa2_problem *prob, const sa2_tensor *q, const sa2_tensor *k1, const sa2_tensor *k2,
-            const sa2_tensor *v1, const sa2_tensor *v2, const sa2_tensor *out, const sa2_tensor *out_residual,
-            float *lse, const sa2_saved *saved, void *hip_stream) {
+// ---- splitting the work of small grids.  The rules are functions of the problem alone (the library is built for this one
+// chip), so workspace sizes and the kernels that run do not depend on the device or on which thread asked first.
+static constexpr int kComputeUnits = 256;
+
+// Estimated finish time of `groups` workgroups of at most `longest` units each (their sum: `total`) that the CUs take one
+// at a time: one round of the longest while they fit the chip, else an even share and a ragged end, but hardly less than
+// the whole rounds that workgroups of equal length would take (list schedules of the shapes of the tests and the benchmark
+// end within 5 % of this).
+static double finish_time(double groups, double longest, double total) {
+    if (groups <= kComputeUnits) return longest;
+    const double full = std::ceil(groups / kComputeUnits) * longest, even = total / kComputeUnits + 0.2 * longest;
+    return full * 0.95 > even ? full * 0.95 : even;
+}
+
+// Query-stationary kernels: the rounds (eight offsets each) of a query tile over several workgroups.  A unit is one step
+// (a K1/V1 tile of one round, 0.7 us); a round end takes kRoundEnd of them, a workgroup's start and end kQueryCost, and
+// the partial rows are written and read once.  Two sequences of 128 rows and 4 heads at D = 64 (32 workgroups of 4 rounds)
+// took 29 us unsplit.
+static constexpr int kRoundEnd = 3, kQueryCost = 6;
+static constexpr int64_t kQueryPartBytes = 128ll << 20;
+
+static int64_t q_parts_bytes(const sa2_problem *prob, int splits) {
+    return (int64_t)splits * prob->batch * prob->heads * prob->seq_len * prob->dim_head * 4;
+}
+
+static int q_splits(const sa2_problem *prob, int merge_cost) {
+    if (prob->dim_head == kWideDimHead) return 1;
+    const int ntile = (prob->seq_len + 31) / 32;
+    const int64_t heads = (int64_t)prob->batch * prob->heads;
+    const int64_t items = heads * ntile;
+    // (rows of 128 lanes and up fill the chip many times over: nothing to gain)
+    if (items > 8 * kComputeUnits) return 1;
+    const int rounds = sa2::fwd_rounds(ntile - 1, prob->w2);
+    int best = 1;
+    double best_cost = 0;
+    for (int splits = 1; splits <= rounds; ++splits) {
+        if (splits > 1 && q_parts_bytes(prob, splits) > kQueryPartBytes) break;
+        double total = 0, longest = 0, groups = 0;
+        for (int t = 0; t < ntile; ++t) {
+            const int lo = 32 * t - prob->w1 + 1 > 0 ? (32 * t - prob->w1 + 1) / 32 : 0;
+            const int r = sa2::fwd_rounds(t, prob->w2), n = splits < r ? splits : r;
+            const double step = t - lo + 1 + kRoundEnd;
+            const double one = (r + n - 1) / n * step + kQueryCost;
+            longest = one > longest ? one : longest;
+            total += r * step + n * kQueryCost;
+            groups += n;
+        }
+        const double merge = splits > 1 ? merge_cost + 2.0 * (double)q_parts_bytes(prob, splits) / 3.5e6 : 0;
+        const double cost = finish_time(groups * heads, longest, total * heads) + merge;
+        if (splits == 1 || cost < 0.95 * best_cost) {
+            best = splits;
+            best_cost = cost;
+        }
+    }
+    return best;
+}
+
+static constexpr int kFwdMergeCost = 8, kBwdMergeCost = 2;        // (the forward's merge is a launch of its own)
+
+int64_t sa2_fwd_workspace_bytes(const sa2_problem *prob) {
+    if (check_problem(prob) != SA2_OK) return -1;
+    const int splits = q_splits(prob, kFwdMergeCost);
+    return splits > 1 ? q_parts_bytes(prob, splits) + 8ll * splits * prob->batch * prob->heads * prob->seq_len : 0;
+}
+
+int sa2_fwd_ws(const sa2_problem *prob, const sa2_tensor *q, const sa2_tensor *k1, const sa2_tensor *k2,
+               const sa2_tensor *v1, const sa2_tensor *v2, const sa2_tensor *out, const sa2_tensor *out_residual,
+               float *lse, const sa2_saved *saved, void *workspace, int64_t workspace_bytes, void *hip_stream) {
     SA2_TRY(check_problem(prob));
     if (out_residual) SA2_TRY(check_tensor(out_residual, "out_residual"));
     SA2_TRY(check_tensor(q, "q"));
@@ -197,6 +263,7 @@ int sa2_fwd(const sa2_problem *prob, const sa2_tensor *q, const sa2_tensor *k1, 
     SA2_TRY(check_tensor(v2, "v2"));
     SA2_TRY(check_tensor(out, "out"));
     if (!lse) return fail(SA2_ERR_NULL_POINTER, "lse is NULL");
+    if ((reinterpret_cast<uintptr_t>(workspace) & 15) != 0) return fail(SA2_ERR_ALIGNMENT, "workspace must be 16-byte aligned");
     sa2::KParams k = base_params(prob);
     k.q = dev(q);
     k.k1 = dev(k1);
@@ -216,10 +283,28 @@ int sa2_fwd(const sa2_problem *prob, const sa2_tensor *q, const sa2_tensor *k1, 
     if (prob->dim_head == kWideDimHead) {
         const int wgrid = prob->batch * prob->heads * ((prob->seq_len + 127) / 128);
         hipLaunchKernelGGL(sa2::fwd_wide_kernel<kWideDimHead>, dim3(wgrid), dim3(256), 0, s, k);
+        return after_launch("forward");
     }
-    else
+    const int64_t need = workspace ? sa2_fwd_workspace_bytes(prob) : 0;
+    if (need == 0 || workspace_bytes < need) {
         SA2_FOR_DIM_HEAD(prob->dim_head, hipLaunchKernelGGL(sa2::fwd_kernel<DH>, dim3(grid), dim3(512), 0, s, k));
-    return after_launch("forward");
+        return after_launch("forward");
+    }
+    k.q_splits = q_splits(prob, kFwdMergeCost);
+    k.q_parts = static_cast<float *>(workspace);
+    SA2_FOR_DIM_HEAD(prob->dim_head, hipLaunchKernelGGL((sa2::fwd_kernel<DH, true>), dim3(k.q_splits * grid), dim3(512), 0, s, k));
+    SA2_TRY(after_launch("forward in splits"));
+    const int64_t rows = (int64_t)prob->batch * prob->heads * prob->seq_len;
+    const int rows_per_block = 256 / (prob->dim_head / 8);
+    const int cgrid = (int)((rows + rows_per_block - 1) / rows_per_block);
+    SA2_FOR_DIM_HEAD(prob->dim_head, hipLaunchKernelGGL(sa2::fwd_combine_kernel<DH>, dim3(cgrid), dim3(256), 0, s, k));
+    return after_launch("forward combine");
+}
+
+int sa2_fwd(const sa2_problem *prob, const sa2_tensor *q, const sa2_tensor *k1, const sa2_tensor *k2,
+            const sa2_tensor *v1, const sa2_tensor *v2, const sa2_tensor *out, const sa2_tensor *out_residual,
+            float *lse, const sa2_saved *saved, void *hip_stream) {
+    return sa2_fwd_ws(prob, q, k1, k2, v1, v2, out, out_residual, lse, saved, nullptr, 0, hip_stream);
 }
 
 int sa2_bwd_delta(const sa2_problem *prob, const sa2_tensor *out, const sa2_tensor *out_residual,
@@ -286,39 +371,93 @@ static int64_t partial_rows_bytes(const sa2_problem *prob) {
     return sa2::qk2_ws_floats(prob->batch, prob->heads, prob->seq_len, prob->dim_head, 32 + q_halo(prob->w2)) * 4;
 }
 
-// dK1/dV1 with the key slabs' work split over two workgroups each (fp32 partial results, summed by a second kernel):
-// for grids of one to four workgroups per CU on short sequences, where the slabs at the sequence's end (those within
-// w1 + 128 rows of it) meet fewer query tiles than the others and whole workgroups of unequal length leave many CUs
-// idle at the end.  Measured on the 256 CUs of an MI355X, whole backward: - 3 % and - 8 % at 512 and 896 workgroups of
-// N = 2048, D = 64; - 1 to - 2 % at 512 and 768 of D = 128; + 1 to + 2 % at 256 workgroups and at N = 8192, which the rule
-// leaves alone.  The rule is a function of the problem alone (the library is built for this one chip), so workspace sizes
-// and the kernels that run do not depend on the device or on which thread asked first.
-static constexpr int kComputeUnits = 256;
-static int cu_count() { return kComputeUnits; }
-
-static bool dkv1_in_parts(const sa2_problem *prob) {
-    if (prob->dim_head == kWideDimHead) return false;
-    const int ntile = (prob->seq_len + 127) / 128;
-    const int64_t grid = (int64_t)prob->batch * prob->kv_heads * ntile;
-    const int64_t ragged = (prob->w1 + 127) / 128 + 1;          // slabs per sequence with a shortened range of query tiles
-    return grid > cu_count() && grid < 4 * cu_count() && 8 * ragged >= ntile;
-}
-
-static int64_t dkv1_parts_bytes(const sa2_problem *prob) {
-    if (!dkv1_in_parts(prob)) return 0;
-    return 2ll * 2 * prob->batch * prob->kv_heads * prob->seq_len * prob->dim_head * 4;
-}
-
 static int64_t max64(int64_t a, int64_t b) { return a > b ? a : b; }
+
+// dK1/dV1 with the walk of a key slab split over several workgroups (fp32 partial results, summed by a second kernel).
+// One workgroup runs per CU, so a small grid leaves CUs idle (at 1 sequence of 1000 rows and 4 key/value heads 32
+// workgroups took 695 us where the work of 256 CUs is 60 us) and a middle one ends on a ragged tail (512 workgroups of
+// unequal length at 8 sequences of 2048 rows).  The rule estimates the finish time of every part count in units of one
+// pair (a query tile and two offsets, 1.3 us at D = 64, 1.9 us at D = 128); a part costs kPartCost pairs on top of its share
+// (its K1/V1 rows, the first rows and operand tiles, 2 * 128 * D fp32 values written and read again).
+static constexpr int kPartCost = 8;
+static constexpr int kMaxParts = 64;
+
+struct Kv8Plan {
+    int chunk, parts;      // parts == 1: one workgroup per slab, no partial results
+};
+
+static int64_t kv_part_bytes(const sa2_problem *prob) {
+    return 2ll * prob->batch * prob->kv_heads * prob->seq_len * prob->dim_head * 4;
+}
+
+// Partial results of dK1/dV1 may take what the scatter rows of dK2 and dV2 take, or this much where those are small.
+static constexpr int64_t kPartBytes = 192ll << 20;
+
+static Kv8Plan kv8_plan(const sa2_problem *prob) {
+    if (prob->dim_head == kWideDimHead) return {0, 1};
+    const int nslab = (prob->seq_len + 127) / 128, G = prob->heads / prob->kv_heads;
+    const int64_t heads = (int64_t)prob->batch * prob->kv_heads;
+    const int64_t budget = max64(kPartBytes, partial_rows_bytes(prob));
+    int64_t longest = 0, total = 0;
+    for (int t = 0; t < nslab; ++t) {
+        const int64_t n = (int64_t)sa2::kv8_walk_pairs(t, prob->seq_len, prob->w1, prob->w2) * G;
+        longest = n > longest ? n : longest;
+        total += n;
+    }
+    total *= heads;
+    Kv8Plan best = {0, 1};
+    double best_cost = 0;
+    for (int parts = 1; parts <= kMaxParts && parts <= longest && (parts == 1 || parts * kv_part_bytes(prob) <= budget); ++parts) {
+        const int64_t chunk = (longest + parts - 1) / parts;
+        const double extra = parts > 1 ? kPartCost : 0;
+        const double groups = parts == 1 ? (double)heads * nslab : (double)total / chunk;      // of about equal length
+        const double cost = finish_time(groups, chunk + extra, (double)total + extra * groups);
+        // (a second launch has to pay for itself)
+        if (parts == 1 || cost < 0.98 * best_cost) {
+            best = {(int)chunk, parts};
+            best_cost = cost;
+        }
+    }
+    return best;
+}
+
+// The plan of sa2_bwd, whose workspace leaves room for two parts: for grids of one to four workgroups per CU on short
+// sequences, where the slabs at the sequence's end (those within w1 + 128 rows of it) meet fewer query tiles than the others.
+static Kv8Plan two_part_plan(const sa2_problem *prob) {
+    if (prob->dim_head == kWideDimHead) return {0, 1};
+    const int nslab = (prob->seq_len + 127) / 128;
+    const int64_t grid = (int64_t)prob->batch * prob->kv_heads * nslab;
+    const int64_t ragged = (prob->w1 + 127) / 128 + 1;          // slabs per sequence with a shortened range of query tiles
+    if (grid <= kComputeUnits || grid >= 4 * kComputeUnits || 8 * ragged < nslab) return {0, 1};
+    int64_t longest = 0;
+    for (int t = 0; t < nslab; ++t)
+        longest = max64(longest, (int64_t)sa2::kv8_walk_pairs(t, prob->seq_len, prob->w1, prob->w2) * (prob->heads / prob->kv_heads));
+    return {(int)((longest + 1) / 2), 2};
+}
+
+static int64_t two_parts_bytes(const sa2_problem *prob) { return two_part_plan(prob).parts > 1 ? 2 * kv_part_bytes(prob) : 0; }
 
 int64_t sa2_bwd_workspace_bytes(const sa2_problem *prob) {
     if (check_problem(prob) != SA2_OK) return -1;
-    return max64(partial_rows_bytes(prob), dkv1_parts_bytes(prob));
+    return max64(partial_rows_bytes(prob), two_parts_bytes(prob));
 }
 
 int64_t sa2_bwd_workspace_bytes_with_saved(const sa2_problem *prob) {
     if (check_problem(prob) != SA2_OK) return -1;
-    return max64(partial_rows_bytes(prob) / 2, dkv1_parts_bytes(prob));
+    return max64(partial_rows_bytes(prob) / 2, two_parts_bytes(prob));
+}
+
+// workspace of the dQ/dK2/dV2 pass in `splits`: scatter rows per split, fp32 dq rows per split behind them
+static int64_t q_workspace_bytes(const sa2_problem *prob, int splits, bool with_saved) {
+    const int64_t scatter = partial_rows_bytes(prob) / (with_saved ? 2 : 1);
+    return splits > 1 ? splits * scatter + q_parts_bytes(prob, splits) : scatter;
+}
+
+int64_t sa2_bwd_split_workspace_bytes(const sa2_problem *prob, int with_saved) {
+    if (check_problem(prob) != SA2_OK) return -1;
+    const Kv8Plan plan = kv8_plan(prob);
+    const int64_t parts = plan.parts > 1 ? plan.parts * kv_part_bytes(prob) : 0;
+    return max64(q_workspace_bytes(prob, q_splits(prob, kBwdMergeCost), with_saved != 0), parts);
 }
 
 // The launches behind sa2_bwd_dq_dkv2: the MFMA kernel(s) on stream `s`; the kernel that streams the forward's saved
@@ -334,7 +473,7 @@ struct QLaunch {
 static int prepare_dq_dkv2(const sa2_problem *prob, const sa2_tensor *q, const sa2_tensor *k1, const sa2_tensor *k2,
                            const sa2_tensor *v1, const sa2_tensor *v2, const sa2_tensor *dout, const float *lse,
                            const float *delta, const sa2_saved *saved, const sa2_tensor *dq, const sa2_tensor *dk2,
-                           const sa2_tensor *dv2, void *workspace, int64_t workspace_bytes, QLaunch *out) {
+                           const sa2_tensor *dv2, void *workspace, int64_t workspace_bytes, bool may_split, QLaunch *out) {
     sa2::KParams &k = out->k;
     SA2_TRY(bwd_common(prob, q, k1, k2, v1, v2, dout, lse, delta, &k));
     SA2_TRY(check_tensor(dq, "dq"));
@@ -345,10 +484,11 @@ static int prepare_dq_dkv2(const sa2_problem *prob, const sa2_tensor *q, const s
     // the dK2 partial rows are the first half of the workspace, the dV2 partial rows the second: with saved
     // forward partials dV2 needs none
     const bool saved_given = saved != nullptr;
-    const int64_t need = partial_rows_bytes(prob) / (saved_given ? 2 : 1);
+    const int splits = may_split ? q_splits(prob, kBwdMergeCost) : 1;
+    const int64_t need = q_workspace_bytes(prob, splits, saved_given);
     if (workspace_bytes < need)
-        return fail(SA2_ERR_BAD_SHAPE, "workspace of %lld bytes is smaller than the %lld bytes this call needs (sa2_bwd_workspace_bytes%s())",
-                    (long long)workspace_bytes, (long long)need, saved_given ? "_with_saved" : "");
+        return fail(SA2_ERR_BAD_SHAPE, "workspace of %lld bytes is smaller than the %lld bytes this call needs (sa2_bwd_%sworkspace_bytes%s())",
+                    (long long)workspace_bytes, (long long)need, may_split ? "split_" : "", saved_given && !may_split ? "_with_saved" : "");
     k.dq = dev(dq);
     k.dk2 = dev(dk2);
     k.dv2 = dev(dv2);
@@ -358,6 +498,11 @@ static int prepare_dq_dkv2(const sa2_problem *prob, const sa2_tensor *q, const s
     // with the forward's saved per-offset T the dv2 pass (a recomputation of S and T) is
     // replaced by a kernel that streams T once
     out->use_saved = saved_given;
+    out->k.q_ws_stride = partial_rows_bytes(prob) / (saved_given ? 2 : 1) / 4;
+    if (splits > 1) {
+        k.q_splits = splits;
+        k.q_parts = out->ws + splits * k.q_ws_stride;
+    }
     if (saved) {
         SA2_TRY(check_saved(prob, saved));
         k.t_save = static_cast<char *>(saved->t);
@@ -372,6 +517,13 @@ static int launch_q_mfma(const sa2_problem *prob, const QLaunch &L, int pass, hi
         hipLaunchKernelGGL(sa2::bwd_wide_q_kernel<kWideDimHead>, dim3(L.grid), dim3(256), 0, s, L.k, L.ws, L.halo);
         return after_launch("dq/dk2/dv2");
     }
+    if (L.k.q_splits > 1) {
+        const dim3 sgrid(L.k.q_splits * L.grid);
+        SA2_FOR_DIM_HEAD(prob->dim_head, hipLaunchKernelGGL((sa2::bwd_q_kernel<DH, true, true>), sgrid, dim3(512), 0, s, L.k, L.ws, L.halo));
+        if (!L.use_saved)
+            SA2_FOR_DIM_HEAD(prob->dim_head, hipLaunchKernelGGL((sa2::bwd_q_kernel<DH, false, true>), sgrid, dim3(512), 0, s, L.k, L.ws, L.halo));
+        return after_launch("dq/dk2/dv2 in splits");
+    }
     SA2_FOR_DIM_HEAD(prob->dim_head, hipLaunchKernelGGL((sa2::bwd_q_kernel<DH, true>), dim3(L.grid), dim3(512), 0, s, L.k, L.ws, L.halo));
     if (pass != 1 && !L.use_saved)
         SA2_FOR_DIM_HEAD(prob->dim_head, hipLaunchKernelGGL((sa2::bwd_q_kernel<DH, false>), dim3(L.grid), dim3(512), 0, s, L.k, L.ws, L.halo));
@@ -385,11 +537,13 @@ static int launch_dv2_from_saved(const sa2_problem *prob, const QLaunch &L, hipS
 }
 
 static int launch_q_combine(const sa2_problem *prob, const QLaunch &L, hipStream_t s) {
-    const int64_t rows = (int64_t)prob->batch * prob->kv_heads * prob->seq_len;
+    // (split query tiles: a second grid row forms dq)
+    const bool dq_too = L.k.q_splits > 1;
+    const int64_t rows = (int64_t)prob->batch * (dq_too ? prob->heads : prob->kv_heads) * prob->seq_len;
     const int rows_per_block = 256 / (prob->dim_head / 8);
     const int cgrid = (int)((rows + rows_per_block - 1) / rows_per_block);
     const int with_dv2 = L.use_saved ? 0 : 1;
-    SA2_FOR_ANY_DIM_HEAD(prob->dim_head, hipLaunchKernelGGL(sa2::dk2_dv2_combine_kernel<DH>, dim3(cgrid), dim3(256), 0, s, L.k, L.ws, 32 + L.halo, with_dv2));
+    SA2_FOR_ANY_DIM_HEAD(prob->dim_head, hipLaunchKernelGGL(sa2::dk2_dv2_combine_kernel<DH>, dim3(cgrid, dq_too ? 2 : 1), dim3(256), 0, s, L.k, L.ws, 32 + L.halo, with_dv2));
     return after_launch("dk2/dv2 combine");
 }
 
@@ -398,7 +552,7 @@ int sa2_bwd_dq_dkv2(const sa2_problem *prob, const sa2_tensor *q, const sa2_tens
                     const float *delta, const sa2_saved *saved, const sa2_tensor *dq, const sa2_tensor *dk2,
                     const sa2_tensor *dv2, void *workspace, int64_t workspace_bytes, void *hip_stream) {
     QLaunch L;
-    SA2_TRY(prepare_dq_dkv2(prob, q, k1, k2, v1, v2, dout, lse, delta, saved, dq, dk2, dv2, workspace, workspace_bytes, &L));
+    SA2_TRY(prepare_dq_dkv2(prob, q, k1, k2, v1, v2, dout, lse, delta, saved, dq, dk2, dv2, workspace, workspace_bytes, false, &L));
     hipStream_t s = static_cast<hipStream_t>(hip_stream);
     const int pass = bwd_pass_filter();
     SA2_TRY(launch_q_mfma(prob, L, pass, s));
@@ -409,7 +563,7 @@ int sa2_bwd_dq_dkv2(const sa2_problem *prob, const sa2_tensor *q, const sa2_tens
 
 static int launch_dkv1(const sa2_problem *prob, const sa2_tensor *q, const sa2_tensor *k1, const sa2_tensor *k2,
                        const sa2_tensor *v1, const sa2_tensor *v2, const sa2_tensor *dout, const float *lse,
-                       const float *delta, const sa2_tensor *dk1, const sa2_tensor *dv1, float *parts, void *hip_stream) {
+                       const float *delta, const sa2_tensor *dk1, const sa2_tensor *dv1, const Kv8Plan &plan, float *parts, void *hip_stream) {
     sa2::KParams k;
     SA2_TRY(bwd_common(prob, q, k1, k2, v1, v2, dout, lse, delta, &k));
     SA2_TRY(check_tensor(dk1, "dk1"));
@@ -417,6 +571,8 @@ static int launch_dkv1(const sa2_problem *prob, const sa2_tensor *q, const sa2_t
     k.dk1 = dev(dk1);
     k.dv1 = dev(dv1);
     k.kv_parts = parts;
+    k.kv_chunk = plan.chunk;
+    k.kv_max_parts = plan.parts;
     hipStream_t s = static_cast<hipStream_t>(hip_stream);
     if (prob->dim_head == kWideDimHead) {
         const int wgrid = prob->batch * prob->kv_heads * ((prob->seq_len + 31) / 32);
@@ -425,18 +581,18 @@ static int launch_dkv1(const sa2_problem *prob, const sa2_tensor *q, const sa2_t
     }
     const int grid = prob->batch * prob->kv_heads * ((prob->seq_len + 127) / 128);
     // dim_head 128: the two waves of a slab split the contractions; dim_head 64 and 32: each wave forms both outputs
-    if (parts) {
+    if (plan.parts > 1) {
         if (prob->dim_head == 128)
-            hipLaunchKernelGGL((sa2::bwd_kv8_kernel<128, sa2::kKvSplit, true>), dim3(2 * grid), dim3(512), 0, s, k);
+            hipLaunchKernelGGL((sa2::bwd_kv8_kernel<128, sa2::kKvSplit, true>), dim3(plan.parts * grid), dim3(512), 0, s, k);
         else if (prob->dim_head == 64)
-            hipLaunchKernelGGL((sa2::bwd_kv8_kernel<64, sa2::kKvBoth, true>), dim3(2 * grid), dim3(512), 0, s, k);
+            hipLaunchKernelGGL((sa2::bwd_kv8_kernel<64, sa2::kKvBoth, true>), dim3(plan.parts * grid), dim3(512), 0, s, k);
         else
-            hipLaunchKernelGGL((sa2::bwd_kv8_kernel<32, sa2::kKvBoth, true>), dim3(2 * grid), dim3(512), 0, s, k);
+            hipLaunchKernelGGL((sa2::bwd_kv8_kernel<32, sa2::kKvBoth, true>), dim3(plan.parts * grid), dim3(512), 0, s, k);
         SA2_TRY(after_launch("dk1/dv1 in parts"));
         const int64_t rows = (int64_t)prob->batch * prob->kv_heads * prob->seq_len;
         const int rows_per_block = 256 / (prob->dim_head / 8);
         const int cgrid = (int)((rows + rows_per_block - 1) / rows_per_block);
-        SA2_FOR_DIM_HEAD(prob->dim_head, hipLaunchKernelGGL(sa2::dkv1_parts_combine_kernel<DH>, dim3(cgrid), dim3(256), 0, s, k));
+        SA2_FOR_DIM_HEAD(prob->dim_head, hipLaunchKernelGGL(sa2::dkv1_parts_combine_kernel<DH>, dim3(cgrid, 2), dim3(256), 0, s, k));
         return after_launch("dk1/dv1 parts combine");
     }
     if (prob->dim_head == 128)
@@ -451,7 +607,35 @@ static int launch_dkv1(const sa2_problem *prob, const sa2_tensor *q, const sa2_t
 int sa2_bwd_dkv1(const sa2_problem *prob, const sa2_tensor *q, const sa2_tensor *k1, const sa2_tensor *k2,
                  const sa2_tensor *v1, const sa2_tensor *v2, const sa2_tensor *dout, const float *lse,
                  const float *delta, const sa2_tensor *dk1, const sa2_tensor *dv1, void *hip_stream) {
-    return launch_dkv1(prob, q, k1, k2, v1, v2, dout, lse, delta, dk1, dv1, nullptr, hip_stream);
+    return launch_dkv1(prob, q, k1, k2, v1, v2, dout, lse, delta, dk1, dv1, Kv8Plan{0, 1}, nullptr, hip_stream);
+}
+
+static int bwd_all(bool split, const sa2_problem *prob, const sa2_tensor *q, const sa2_tensor *k1, const sa2_tensor *k2,
+            const sa2_tensor *v1, const sa2_tensor *v2, const sa2_tensor *out, const sa2_tensor *out_residual,
+            const sa2_tensor *dout, const float *lse, const sa2_saved *saved, float *delta_ws, const sa2_tensor *dq,
+            const sa2_tensor *dk1, const sa2_tensor *dk2, const sa2_tensor *dv1, const sa2_tensor *dv2, void *workspace,
+            int64_t workspace_bytes, void *hip_stream) {
+    SA2_TRY(check_problem(prob));
+    // every size and pointer is checked before the first launch: a call that fails has written nothing
+    const Kv8Plan plan = split ? kv8_plan(prob) : two_part_plan(prob);
+    const int64_t need = plan.parts > 1 ? plan.parts * kv_part_bytes(prob) : 0;
+    if (workspace_bytes < need)
+        return fail(SA2_ERR_BAD_SHAPE, "workspace of %lld bytes is smaller than the %lld bytes this problem's dk1/dv1 pass needs (sa2_bwd_%s())",
+                    (long long)workspace_bytes, (long long)need, split ? "split_workspace_bytes" : "workspace_bytes");
+    if (!delta_ws) return fail(SA2_ERR_NULL_POINTER, "delta is NULL");
+    SA2_TRY(check_tensor(out, "out"));
+    if (out_residual) SA2_TRY(check_tensor(out_residual, "out_residual"));
+    SA2_TRY(check_tensor(dk1, "dk1"));
+    SA2_TRY(check_tensor(dv1, "dv1"));
+    QLaunch L;
+    SA2_TRY(prepare_dq_dkv2(prob, q, k1, k2, v1, v2, dout, lse, delta_ws, saved, dq, dk2, dv2, workspace, workspace_bytes, split, &L));
+    hipStream_t s = static_cast<hipStream_t>(hip_stream);
+    SA2_TRY(sa2_bwd_delta(prob, out, out_residual, dout, delta_ws, hip_stream));
+    SA2_TRY(launch_q_mfma(prob, L, 0, s));
+    if (L.use_saved) SA2_TRY(launch_dv2_from_saved(prob, L, s));
+    SA2_TRY(launch_q_combine(prob, L, s));
+    // the partial rows of dK2/dV2 are spent by now: the partial results of split key slabs reuse the workspace
+    return launch_dkv1(prob, q, k1, k2, v1, v2, dout, lse, delta_ws, dk1, dv1, plan, static_cast<float *>(workspace), hip_stream);
 }
 
 int sa2_bwd(const sa2_problem *prob, const sa2_tensor *q, const sa2_tensor *k1, const sa2_tensor *k2,
@@ -459,27 +643,17 @@ int sa2_bwd(const sa2_problem *prob, const sa2_tensor *q, const sa2_tensor *k1, 
             const sa2_tensor *dout, const float *lse, const sa2_saved *saved, float *delta_ws, const sa2_tensor *dq,
             const sa2_tensor *dk1, const sa2_tensor *dk2, const sa2_tensor *dv1, const sa2_tensor *dv2, void *workspace,
             int64_t workspace_bytes, void *hip_stream) {
-    SA2_TRY(check_problem(prob));
-    // every size and pointer is checked before the first launch: a call that fails has written nothing
-    const bool parts_wanted = dkv1_in_parts(prob);
-    if (parts_wanted && workspace_bytes < dkv1_parts_bytes(prob))
-        return fail(SA2_ERR_BAD_SHAPE, "workspace of %lld bytes is smaller than the %lld bytes this problem's dk1/dv1 pass needs (sa2_bwd_workspace_bytes())",
-                    (long long)workspace_bytes, (long long)dkv1_parts_bytes(prob));
-    if (!delta_ws) return fail(SA2_ERR_NULL_POINTER, "delta is NULL");
-    SA2_TRY(check_tensor(out, "out"));
-    if (out_residual) SA2_TRY(check_tensor(out_residual, "out_residual"));
-    SA2_TRY(check_tensor(dk1, "dk1"));
-    SA2_TRY(check_tensor(dv1, "dv1"));
-    QLaunch L;
-    SA2_TRY(prepare_dq_dkv2(prob, q, k1, k2, v1, v2, dout, lse, delta_ws, saved, dq, dk2, dv2, workspace, workspace_bytes, &L));
-    hipStream_t s = static_cast<hipStream_t>(hip_stream);
-    SA2_TRY(sa2_bwd_delta(prob, out, out_residual, dout, delta_ws, hip_stream));
-    SA2_TRY(launch_q_mfma(prob, L, 0, s));
-    if (L.use_saved) SA2_TRY(launch_dv2_from_saved(prob, L, s));
-    SA2_TRY(launch_q_combine(prob, L, s));
-    // the partial rows of dK2/dV2 are spent by now: the partial results of split key slabs reuse the workspace
-    float *parts = parts_wanted ? static_cast<float *>(workspace) : nullptr;
-    return launch_dkv1(prob, q, k1, k2, v1, v2, dout, lse, delta_ws, dk1, dv1, parts, hip_stream);
+    return bwd_all(false, prob, q, k1, k2, v1, v2, out, out_residual, dout, lse, saved, delta_ws, dq, dk1, dk2, dv1, dv2, workspace,
+                   workspace_bytes, hip_stream);
+}
+
+int sa2_bwd_split(const sa2_problem *prob, const sa2_tensor *q, const sa2_tensor *k1, const sa2_tensor *k2,
+                  const sa2_tensor *v1, const sa2_tensor *v2, const sa2_tensor *out, const sa2_tensor *out_residual,
+                  const sa2_tensor *dout, const float *lse, const sa2_saved *saved, float *delta_ws, const sa2_tensor *dq,
+                  const sa2_tensor *dk1, const sa2_tensor *dk2, const sa2_tensor *dv1, const sa2_tensor *dv2, void *workspace,
+                  int64_t workspace_bytes, void *hip_stream) {
+    return bwd_all(true, prob, q, k1, k2, v1, v2, out, out_residual, dout, lse, saved, delta_ws, dq, dk1, dk2, dv1, dv2, workspace,
+                   workspace_bytes, hip_stream);
 }
 
 static int64_t align256(int64_t x) { return (x + 255) & ~int64_t(255); }

@@ -72,8 +72,36 @@ struct Kv8Cfg {
     static_assert((MODE == kKvBoth ? 2 : 1) * RED <= LDS, "final reduction must fit (everything else is dead by then)");
 };
 
-// PARTS: two workgroups per key slab, each walks half of the slab's query tiles and leaves fp32 partial rows in
-// p.kv_parts (for grids that would otherwise put one or two long workgroups on every CU and end on a ragged tail)
+// The walk of a 128-row key slab: its pairs in order (query head of the group, query tile, pair of offsets).  A query
+// tile holds min(ceil(w2 / 2), 16 (it + 1)) pairs (offsets 0 .. min(w2 - 1, 32 it + 31)); kv8_pairs_below is the prefix
+// sum over the tiles 0 .. it - 1.
+__host__ __device__ inline int kv8_pairs_of(int it, int w2) {
+    const int c = (w2 + 1) / 2, ramp = 16 * (it + 1);
+    return c < ramp ? c : ramp;
+}
+__host__ __device__ inline int64_t kv8_pairs_below(int it, int w2) {
+    const int c = (w2 + 1) / 2;
+    const int64_t m = it < c / 16 ? it : c / 16;      // tiles on the ramp
+    return 8 * m * (m + 1) + (it - m) * c;
+}
+// last query tile that reaches the slab
+__host__ __device__ inline int kv8_last_tile(int slab, int N, int w1) {
+    const int64_t last_i = 128ll * slab + 127 + w1 - 1;
+    return (int)((last_i < N - 1 ? last_i : N - 1) / 32);
+}
+// pairs of one query head's walk
+__host__ __device__ inline int kv8_walk_pairs(int slab, int N, int w1, int w2) {
+    return (int)(kv8_pairs_below(kv8_last_tile(slab, N, w1) + 1, w2) - kv8_pairs_below(4 * slab, w2));
+}
+// workgroups that share a slab of `pairs` pairs when a part holds about `chunk` of them (at most max_parts: the grid)
+__host__ __device__ inline int kv8_parts_of(int64_t pairs, int chunk, int max_parts) {
+    const int64_t n = (pairs + chunk - 1) / chunk;
+    return n < 1 ? 1 : (n < max_parts ? (int)n : max_parts);
+}
+
+// PARTS: several workgroups per key slab (p.kv_max_parts of them in the grid), each walks an equal share of the slab's
+// pairs and leaves fp32 partial rows in p.kv_parts.  For grids that would otherwise leave CUs without a workgroup or
+// end on a ragged tail (kv8_plan in sa2_api.hip has the rule).
 template <int D, int MODE, bool PARTS = false>
 __global__ __launch_bounds__(512) void bwd_kv8_kernel(KParams p) {
     constexpr int KS = D / 16, DT = D / 32, PPR = D / 8;
@@ -85,10 +113,21 @@ __global__ __launch_bounds__(512) void bwd_kv8_kernel(KParams p) {
     const int N = p.N;
     const int ntile = (N + 127) / 128;
     const int item_all = xcd_contiguous(blockIdx.x, gridDim.x);
-    const int part = PARTS ? item_all & 1 : 0;
-    const int item = PARTS ? item_all >> 1 : item_all;
+    const int item = PARTS ? uniform(item_all / p.kv_max_parts) : item_all;
+    const int part = PARTS ? item_all - item * p.kv_max_parts : 0;
     const int tile = item % ntile;
     const int bh = item / ntile;
+    // this workgroup's share of the slab's walk: pairs pair0 .. pair0 + npairs - 1
+    const int head_pairs = kv8_walk_pairs(tile, N, p.w1, p.w2);
+    int pair0 = 0;
+    int npairs = head_pairs * p.G;
+    if constexpr (PARTS) {
+        const int64_t all = (int64_t)head_pairs * p.G;
+        const int parts = uniform(kv8_parts_of(all, p.kv_chunk, p.kv_max_parts));
+        if (part >= parts) return;                    // (a slab with a short walk: the combine kernel knows)
+        pair0 = uniform((int)(all * part / parts));
+        npairs = uniform((int)(all * (part + 1) / parts)) - pair0;
+    }
     const int hk = bh % p.HK, b = bh / p.HK;
 
     const int tid = threadIdx.x;
@@ -126,29 +165,12 @@ __global__ __launch_bounds__(512) void bwd_kv8_kernel(KParams p) {
 #pragma unroll
     for (int dt = 0; dt < (TWO ? DT : 1); ++dt) acc2[dt] = zero16();
 
-    const int last_i = (j0 + 127 + p.w1 - 1 < N - 1) ? j0 + 127 + p.w1 - 1 : N - 1;
-    const int it_first = j0 / 32, it_last = last_i / 32;          // the query tiles that reach the slab
-    const int it_half = (it_last - it_first + 2) / 2;             // PARTS: the first part takes the larger half
-    const int it_begin = PARTS && part ? it_first + it_half : it_first;
-    const int it_end = PARTS && !part ? it_first + it_half - 1 : it_last;
+    const int it_begin = j0 / 32, it_end = kv8_last_tile(tile, N, p.w1);      // the query tiles that reach the slab
     // where a lane's row of a partial result goes (PARTS)
     auto part_row = [&](int which) {
         const int64_t rows = (int64_t)p.B * p.HK * N;
         return p.kv_parts + ((int64_t)(2 * part + which) * rows + ((int64_t)b * p.HK + hk) * N + j) * D + 16 * hf;
     };
-    if constexpr (PARTS) {
-        if (it_begin > it_end) {
-            // (a slab with a single query tile: nothing for the second part but its zeros)
-            f32x16 z[DT];
-#pragma unroll
-            for (int dt = 0; dt < DT; ++dt) z[dt] = zero16();
-            if (j_ok && wave < 4) {
-                store_row_f32<DT>(part_row(0), z, 0.f);
-                store_row_f32<DT>(part_row(1), z, 0.f);
-            }
-            return;
-        }
-    }
     const bool wave_active = jw < N;
     const int wit_lo = jw / 32;
     const int wit_hi = ((jw + 31 + p.w1 - 1 < N - 1) ? jw + 31 + p.w1 - 1 : N - 1) / 32;
@@ -180,11 +202,6 @@ __global__ __launch_bounds__(512) void bwd_kv8_kernel(KParams p) {
     auto next_pair = [&](Pair &s) {
         if (2 * (++s.m) > dmax_of(s.it, s.blk)) next_unit(s);
     };
-    int npairs = 0;
-    for (int it = it_begin; it <= it_end; ++it)
-        for (int blk = 0; 32 * blk <= dtop_of(it); ++blk) npairs += dmax_of(it, blk) / 2 + 1;
-    npairs *= p.G;
-
     // ---- row staging: per (query head, query tile) the q/do rows and the k2/v2 rows go
     // global -> registers (a whole tile ahead) -> LDS
     u32x4 rows[L::RPT];
@@ -302,8 +319,15 @@ __global__ __launch_bounds__(512) void bwd_kv8_kernel(KParams p) {
         }
     };
     Pair nb = {0, it_begin, 0, 0};   // next pair to build
-    Pair cur = {0, it_begin, 0, 0};  // pair being computed
-    Pair rw = {0, it_begin, 0, 0};   // staging unit whose rows are loaded next
+    if constexpr (PARTS) {
+        nb.g = uniform(pair0 / head_pairs);
+        int left = pair0 - nb.g * head_pairs;
+        for (int n; left >= (n = kv8_pairs_of(nb.it, p.w2)); ++nb.it) left -= n;
+        nb.blk = left / 16;
+        nb.m = left % 16;
+    }
+    Pair cur = nb;                   // pair being computed
+    Pair rw = nb;                    // staging unit whose rows are loaded next
     issue_rows(rw);
     next_unit(rw);
     write_rows();
@@ -667,28 +691,37 @@ __global__ __launch_bounds__(512) void bwd_kv8_kernel(KParams p) {
     }
 }
 
-// dK1 and dV1 from the two partial results of the split slabs: a thread sums 8 d of one row
+// dK1 and dV1 from the partial results of the split slabs, added in part order: a thread sums 8 d of one row of one of them
 template <int D>
 __global__ __launch_bounds__(256) void dkv1_parts_combine_kernel(KParams p) {
     constexpr int LP = D / 8;
     const int64_t rows = (int64_t)p.B * p.HK * p.N;
     const int64_t row = (int64_t)blockIdx.x * (256 / LP) + threadIdx.x / LP;
     if (row >= rows) return;
+    const int which = blockIdx.y;
     const int piece = threadIdx.x % LP;
     const int j = (int)(row % p.N);
     const int hk = (int)((row / p.N) % p.HK);
     const int b = (int)(row / ((int64_t)p.N * p.HK));
-#pragma unroll
-    for (int which = 0; which < 2; ++which) {
-        const float *a = p.kv_parts + ((int64_t)which * rows + row) * D + piece * 8;
-        const float *c = a + 2 * rows * D;
-        const float4 a0 = *reinterpret_cast<const float4 *>(a), a1 = *reinterpret_cast<const float4 *>(a + 4);
-        const float4 c0 = *reinterpret_cast<const float4 *>(c), c1 = *reinterpret_cast<const float4 *>(c + 4);
-        const u32x4 o = {pack_bf16(a0.x + c0.x, a0.y + c0.y), pack_bf16(a0.z + c0.z, a0.w + c0.w),
-                         pack_bf16(a1.x + c1.x, a1.y + c1.y), pack_bf16(a1.z + c1.z, a1.w + c1.w)};
-        const DevTensor &t = which ? p.dv1 : p.dk1;
-        st_global16(t.ptr + b * t.sb + (int64_t)j * t.sn + hk * t.sh + piece * 16, o);
+    const int parts = kv8_parts_of((int64_t)kv8_walk_pairs(j / 128, p.N, p.w1, p.w2) * p.G, p.kv_chunk, p.kv_max_parts);
+    const float *src = p.kv_parts + ((int64_t)which * rows + row) * D + piece * 8;
+    const int64_t step = 2 * rows * D;
+    float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+    for (int x = 0; x < parts; ++x, src += step) {
+        const float4 a0 = *reinterpret_cast<const float4 *>(src), a1 = *reinterpret_cast<const float4 *>(src + 4);
+        s[0] += a0.x;
+        s[1] += a0.y;
+        s[2] += a0.z;
+        s[3] += a0.w;
+        s[4] += a1.x;
+        s[5] += a1.y;
+        s[6] += a1.z;
+        s[7] += a1.w;
     }
+    const u32x4 o = {pack_bf16(s[0], s[1]), pack_bf16(s[2], s[3]), pack_bf16(s[4], s[5]), pack_bf16(s[6], s[7])};
+    const DevTensor &t = which ? p.dv1 : p.dk1;
+    st_global16(t.ptr + b * t.sb + (int64_t)j * t.sn + hk * t.sh + piece * 16, o);
 }
 
 }  // namespace sa2

@@ -28,6 +28,7 @@
 #include <type_traits>
 
 #include "sa2_common.hpp"
+#include "sa2_fwd.hpp"
 #include "sa2_lds.hpp"
 
 namespace sa2 {
@@ -58,12 +59,15 @@ struct QCfg {
     static constexpr int PIECES = 32 * PPR;           // ... per tile
 };
 
-// workspace layout (floats): [tensor 0: dk2, 1: dv2][b][h][tile][srows][D], srows = 32 + halo
-__host__ __device__ inline int64_t qk2_ws_floats(int B, int H, int N, int D, int srows) {
+// SPLIT: the rounds of a query tile are shared by p.q_splits workgroups (fwd_split_round); each leaves its dq rows in
+// p.q_parts as fp32 and its scatter rows in a workspace block of its own, which the combine kernel adds in split order.
+//
+// workspace layout (floats): [split][tensor 0: dk2, 1: dv2 (not with saved forward partials)][b][h][tile][srows][D], srows = 32 + halo
+__host__ __device__ inline int64_t qk2_ws_floats(int B, int H, int N, int D, int srows) {   // of one split
     return 2ll * B * H * ((N + 31) / 32) * srows * D;
 }
 
-template <int D, bool DQ>
+template <int D, bool DQ, bool SPLIT = false>
 __global__ __launch_bounds__(512) void bwd_q_kernel(KParams p, float *ws, int halo) {
     using C = QCfg<D, DQ>;
     constexpr int KS = C::KS, DT = C::DT, PPR = C::PPR, PITCH = C::PITCH;
@@ -71,11 +75,18 @@ __global__ __launch_bounds__(512) void bwd_q_kernel(KParams p, float *ws, int ha
 
     const int N = p.N;
     const int ntile = (N + 31) / 32;
-    const int item = xcd_contiguous(blockIdx.x, gridDim.x);
-    const int tile = ntile - 1 - item % ntile;
-    const int bh = item / ntile;
-    const int h = bh % p.H, b = bh / p.H;
-    const int hk = h / p.G;
+    const int item_all = xcd_contiguous(blockIdx.x, gridDim.x);
+    const int item = SPLIT ? uniform(item_all / p.q_splits) : item_all;
+    const int split = SPLIT ? item_all - item * p.q_splits : 0;
+    const int bh = uniform(item / ntile);
+    const int tile = ntile - 1 - (item - bh * ntile);
+    const int b = uniform(bh / p.H), h = bh - b * p.H;
+    const int hk = uniform(h / p.G);
+    // rounds r_first .. R - 1 of eight offsets each
+    const int rounds = fwd_rounds(tile, p.w2);
+    const int r_first = SPLIT ? uniform(fwd_split_round(split, p.q_splits, rounds)) : 0;
+    const int R = SPLIT ? uniform(fwd_split_round(split + 1, p.q_splits, rounds)) : rounds;
+    if (SPLIT && r_first >= R) return;
 
     const int tid = threadIdx.x;
     const int wave = wave_index(), lane = tid & 63;
@@ -100,9 +111,6 @@ __global__ __launch_bounds__(512) void bwd_q_kernel(KParams p, float *ws, int ha
     int mid_lo = (i0 + 31 - p.w1 >= 0) ? (i0 + 31 - p.w1) / 32 + 1 : t_lo;   // first tile that no row masks at the window's lower edge
     mid_lo = mid_lo > t_hi ? t_hi : mid_lo;
     const int n_head = mid_lo - t_lo;                 // leading steps of a round with a lower-edge mask (at most 2)
-    const int nd = p.w2 < i0 + 32 ? p.w2 : i0 + 32;   // offsets that meet at least one valid k
-    const int R = (nd + 7) / 8;
-    const int U = R * NT;
 
     // ---- ring staging: direct-to-LDS loads, wave w moves chunk w of the K1 tile and of the V1 tile (D = 64: four
     // chunks per tile, waves 0-3 stage)
@@ -160,9 +168,9 @@ __global__ __launch_bounds__(512) void bwd_q_kernel(KParams p, float *ws, int ha
         }
         for (int x = tid; x < 39 * PPR; x += 512) {
             const int row = x / PPR, col = (x % PPR) * 16;
-            int kk2 = i0 - 7 + row;
+            int kk2 = i0 - 7 - 8 * r_first + row;
             kk2 = kk2 < 0 ? 0 : (kk2 < N ? kk2 : N - 1);
-            const int slot = (row - 7) & 63;
+            const int slot = (row - 7 - 8 * r_first) & 63;
             *reinterpret_cast<u32x4 *>(lds + C::K2S + slot * PITCH + col) = ld_global16(k2g + (int64_t)kk2 * p.k2.sn + col);
             if constexpr (DQ)
                 *reinterpret_cast<u32x4 *>(lds + C::V2S + slot * PITCH + col) = ld_global16(v2g + (int64_t)kk2 * p.v2.sn + col);
@@ -200,7 +208,7 @@ __global__ __launch_bounds__(512) void bwd_q_kernel(KParams p, float *ws, int ha
     // scatter rows of this tile in the workspace: row x <-> k = i0 - halo + x
     const int srows = 32 + halo;
     const int64_t per_tensor = (int64_t)p.B * p.H * ntile * srows * D;
-    float *wk = ws + (DQ ? 0 : per_tensor) + (((int64_t)b * p.H + h) * ntile + tile) * srows * D;
+    float *wk = ws + split * p.q_ws_stride + (DQ ? 0 : per_tensor) + (((int64_t)b * p.H + h) * ntile + tile) * srows * D;
     // rows k - i0 = lo .. lo + n - 1 of the circular buffer go to the workspace and are cleared for reuse
     auto flush_rows = [&](int lo, int n) {
         for (int x = tid; x < n * (D / 4); x += 512) {
@@ -227,7 +235,7 @@ __global__ __launch_bounds__(512) void bwd_q_kernel(KParams p, float *ws, int ha
     u32x4 Bv[DQ ? KS : 1];
 
     __syncthreads();
-    for (int r = 0; r < R; ++r) {
+    for (int r = r_first; r < R; ++r) {
         const int dlt = 8 * r + wave;
         const int kr = i - dlt;
         const bool col_ok = row_ok && kr >= 0 && dlt < p.w2;
@@ -401,6 +409,12 @@ __global__ __launch_bounds__(512) void bwd_q_kernel(KParams p, float *ws, int ha
         const int ir = i0 + row;
         if (ir < N) {
             const float *src = dqs + row * C::SPITCH + seg * SEG;
+            if constexpr (SPLIT) {
+                float *dst = p.q_parts + ((((int64_t)split * p.B + b) * p.H + h) * N + ir) * D + seg * SEG;
+#pragma unroll
+                for (int x = 0; x < SEG; x += 2) *reinterpret_cast<float2 *>(dst + x) = *reinterpret_cast<const float2 *>(src + x);
+                return;
+            }
             char *orow = p.dq.ptr + b * p.dq.sb + (int64_t)ir * p.dq.sn + h * p.dq.sh + seg * SEG * 2;
             if constexpr (SEG == 8) {
                 float4 a = *reinterpret_cast<const float4 *>(src);
@@ -495,15 +509,36 @@ __global__ __launch_bounds__(Dv2Cfg<D>::THREADS) void dv2_from_saved_kernel(KPar
 // dK2 / dV2 from the partial rows of the workspace: sums the tiles that reach a row and the query heads of a group.
 // Workspace rows of a tile with first query row i0: index x <-> k = i0 - halo + x, so
 // rows 0..halo-1 are the halo below the tile and rows halo..halo+31 its own rows.
+// With split query tiles (p.q_splits > 1) the shares of a tile are added in split order (a share has written the rows its
+// rounds reach, k - i0 = -8 R + 1 .. 31 - 8 r_first) and the blocks of grid row 1 form dq from the shares' fp32 rows.
 template <int D>
 __global__ __launch_bounds__(256) void dk2_dv2_combine_kernel(KParams p, const float *ws, int srows, int with_dv2) {
     constexpr int LP = D / 8;   // threads per row, 8 d each
     const int N = p.N, ntile = (N + 31) / 32;
     const int halo = srows - 32;
-    const int64_t rows = (int64_t)p.B * p.HK * N;
-    const int64_t row = (int64_t)blockIdx.x * (256 / LP) + threadIdx.x / LP;
-    if (row >= rows) return;
     const int piece = threadIdx.x % LP;
+    const int64_t row = (int64_t)blockIdx.x * (256 / LP) + threadIdx.x / LP;
+    if (blockIdx.y == 1) {
+        const int64_t rows = (int64_t)p.B * p.H * N;
+        if (row >= rows) return;
+        const int i = (int)(row % N), h = (int)((row / N) % p.H), b = (int)(row / ((int64_t)N * p.H));
+        const int rounds = fwd_rounds(i / 32, p.w2);
+        const int splits = p.q_splits < rounds ? p.q_splits : rounds;
+        float a[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+        for (int s = 0; s < splits; ++s) {
+            const float *src = p.q_parts + (s * rows + row) * D + piece * 8;
+#pragma unroll
+            for (int x = 0; x < 8; ++x) a[x] += src[x];
+        }
+        u32x4 o;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) o[w] = pack_bf16(a[2 * w] * p.scale, a[2 * w + 1] * p.scale);
+        st_global16(p.dq.ptr + b * p.dq.sb + (int64_t)i * p.dq.sn + h * p.dq.sh + piece * 16, o);
+        return;
+    }
+    const int64_t rows = (int64_t)p.B * p.HK * N;
+    if (row >= rows) return;
     const int k = (int)(row % N);
     const int hk = (int)((row / N) % p.HK);
     const int b = (int)(row / ((int64_t)N * p.HK));
@@ -517,6 +552,20 @@ __global__ __launch_bounds__(256) void dk2_dv2_combine_kernel(KParams p, const f
         const float *base = ws + (((int64_t)b * p.H + h) * ntile) * srows * D;
         for (int m = 0; tile + m < ntile && kl + halo - 32 * m >= 0; ++m) {
             const float *src = base + ((int64_t)(tile + m) * srows + (kl + halo - 32 * m)) * D + piece * 8;
+            if (p.q_splits > 1) {
+                const int rounds = fwd_rounds(tile + m, p.w2), rel = kl - 32 * m;
+                for (int s = 0; s < p.q_splits; ++s) {
+                    const int r0 = fwd_split_round(s, p.q_splits, rounds), r1 = fwd_split_round(s + 1, p.q_splits, rounds);
+                    if (r0 >= r1 || rel > 31 - 8 * r0 || rel < 1 - 8 * r1) continue;
+                    const float *ss = src + s * p.q_ws_stride;
+#pragma unroll
+                    for (int x = 0; x < 8; ++x) {
+                        ak[x] += ss[x];
+                        if (with_dv2) av[x] += ss[per_tensor + x];
+                    }
+                }
+                continue;
+            }
 #pragma unroll
             for (int x = 0; x < 8; ++x) {
                 ak[x] += src[x];

@@ -52,9 +52,17 @@ struct KParams {
     int w1, w2;
     float scale;          // softmax scale
     float scale_log2e;    // scale * log2(e)
-    // dK1/dV1 computed in two parts per key slab (each part walks half of the slab's query tiles): fp32 partial rows
-    // [part][dk1, dv1][B][HK][N][D], summed by dkv1_parts_combine_kernel; nullptr when the slabs are not split
+    // dK1/dV1 computed in parts (each part walks a share of a key slab's query tiles and offsets): fp32 partial rows
+    // [part][dk1, dv1][B][HK][N][D], summed by dkv1_parts_combine_kernel; nullptr when the slabs are not split.
+    // kv_chunk: (query tile, offset pair) steps a part holds at most; kv_max_parts: parts of the longest walk
     float *kv_parts;
+    int kv_chunk, kv_max_parts;
+    // query-stationary kernels with the rounds of a query tile split over q_splits workgroups: forward, fp32
+    // [split][B][H][N][D] output rows and [split][B][H][N] pairs (reference, row sum) behind them; backward, fp32
+    // [split][B][H][N][D] rows of dq
+    float *q_parts;
+    int q_splits;
+    int64_t q_ws_stride;  // backward: floats between the scatter rows of consecutive splits
 };
 
 // compile-time loop: f(integral_constant<int, B>) ... f(integral_constant<int, E - 1>)
@@ -100,6 +108,10 @@ __device__ __forceinline__ float add_bf16x2(uint32_t x, float c) {
 
 // wave index as a scalar: branches on it are uniform and index arithmetic stays on the scalar unit
 __device__ __forceinline__ int wave_index() { return __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); }
+
+// a value that is the same in every lane, on the scalar unit (an integer division leaves its result in a vector register,
+// and what is computed from it follows)
+__device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
 
 __device__ __forceinline__ f32x16 mfma32(u32x4 a, u32x4 b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(a), as_bf16x8(b), c, 0, 0, 0);

@@ -77,7 +77,20 @@ struct FwdCfg {
     static constexpr int PIECES = 32 * PPR;           // ... per tile
 };
 
-template <int D>
+// rounds of eight offsets that query tile `tile` walks, and the first round of split s of `splits` (a tile with fewer
+// rounds than splits uses as many splits as it has rounds)
+__host__ __device__ inline int fwd_rounds(int tile, int w2) {
+    const int top = 32 * tile + 32;
+    return ((w2 < top ? w2 : top) + 7) / 8;
+}
+__host__ __device__ inline int fwd_split_round(int s, int splits, int rounds) {
+    return splits < rounds ? rounds * s / splits : (s < rounds ? s : rounds);
+}
+
+// SPLIT: several workgroups per query tile (p.q_splits of them in the grid), each walks a share of the tile's rounds and
+// leaves its fp32 output rows, their reference and their row sums in p.q_parts, which fwd_combine_kernel merges.  For grids
+// too small to give every CU a workgroup (q_plan in sa2_api.hip has the rule).
+template <int D, bool SPLIT = false>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(FwdCfg<D>::WPE, FwdCfg<D>::WPE))) void fwd_kernel(KParams p) {
     using C = FwdCfg<D>;
     constexpr int KS = C::KS, DT = C::DT, PPR = C::PPR, PITCH = C::PITCH;
@@ -86,11 +99,18 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(FwdCfg<D>::
 
     const int N = p.N;
     const int ntile = (N + 31) / 32;
-    const int item = xcd_contiguous(blockIdx.x, gridDim.x);
-    const int tile = ntile - 1 - item % ntile;
-    const int bh = item / ntile;
-    const int h = bh % p.H, b = bh / p.H;
-    const int hk = h / p.G;
+    const int item_all = xcd_contiguous(blockIdx.x, gridDim.x);
+    const int item = SPLIT ? uniform(item_all / p.q_splits) : item_all;
+    const int split = SPLIT ? item_all - item * p.q_splits : 0;
+    const int bh = uniform(item / ntile);
+    const int tile = ntile - 1 - (item - bh * ntile);
+    const int b = uniform(bh / p.H), h = bh - b * p.H;
+    const int hk = uniform(h / p.G);
+    // rounds r_first .. R - 1 of eight offsets each
+    const int rounds = fwd_rounds(tile, p.w2);
+    const int r_first = SPLIT ? uniform(fwd_split_round(split, p.q_splits, rounds)) : 0;
+    const int R = SPLIT ? uniform(fwd_split_round(split + 1, p.q_splits, rounds)) : rounds;
+    if (SPLIT && r_first >= R) return;
 
     const int tid = threadIdx.x;
     const int wave = wave_index(), lane = tid & 63;
@@ -111,10 +131,6 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(FwdCfg<D>::
     int mid_lo = (i0 + 31 - p.w1 >= 0) ? (i0 + 31 - p.w1) / 32 + 1 : t_lo;   // first tile below the diagonal that no row masks
     mid_lo = mid_lo > t_hi ? t_hi : mid_lo;
     const int n_masked = 1 + (mid_lo - t_lo);         // leading steps of a round that need a mask (at most 3)
-    const int nd = p.w2 < i0 + 32 ? p.w2 : i0 + 32;   // offsets that meet at least one valid k
-    const int R = (nd + 7) / 8;
-    const int U = R * NT;
-    auto tile_of = [&](int n) { return n == 0 ? t_hi : t_lo + n - 1; };
 
     // ---- ring staging: direct-to-LDS loads, wave w moves chunk(s) w of the K1 tile and of the V1 tile.  Lane p of a
     // chunk load fetches row (p / 4) % RPC, segment p / (4 RPC), piece p % 4 of the segment
@@ -178,12 +194,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(FwdCfg<D>::
                 *reinterpret_cast<u32x4 *>(lds + C::QS + row * C::QPITCH + col) = fq;
             }
         }
-        // rows k - i0 = -32 .. 31 fill the 64 slots: the first four rounds find their rows here
+        // rows k - i0 = -32 .. 31 (less 8 per round that other workgroups walk) fill the 64 slots: the first four
+        // rounds find their rows here
         for (int x = tid; x < 64 * PPR; x += 512) {
             const int row = x / PPR, col = (x % PPR) * 16;
-            int kk2 = i0 - 32 + row;
+            int kk2 = i0 - 32 - 8 * r_first + row;
             kk2 = kk2 < 0 ? 0 : (kk2 < N ? kk2 : N - 1);
-            const int slot = (row - 32) & 63;
+            const int slot = (row - 32 - 8 * r_first) & 63;
             *reinterpret_cast<u32x4 *>(lds + C::K2S + slot * PITCH + col) = ld_global16(k2g + (int64_t)kk2 * p.k2.sn + col);
             *reinterpret_cast<u32x4 *>(lds + C::V2S + slot * PITCH + col) = ld_global16(v2g + (int64_t)kk2 * p.v2.sn + col);
         }
@@ -202,7 +219,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(FwdCfg<D>::
     }
     // the 8 rows that round r + 1 adds (k - i0 = -8r - 15 .. -8r - 8), one 16-byte piece per thread; only rounds
     // beyond the fourth add rows that the prologue has not staged
-    auto adds_rows = [&](int r) { return r + 1 < R && r + 1 >= 4; };
+    auto adds_rows = [&](int r) { return r + 1 < R && r + 1 >= r_first + 4; };
     const bool row_stager = tid < 2 * 8 * PPR;
     const int rs_sel = tid / (8 * PPR), rs_row = (tid / PPR) % 8, rs_col = (tid % PPR) * 16;
     u32x4 st_r = {0u, 0u, 0u, 0u};
@@ -244,7 +261,6 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(FwdCfg<D>::
     issue_loads();
     issue_loads();
     issue_loads();
-    int u = 0;
     wait_loads<0>();
     // start of step u: the tile of step u + 1 has landed (at most the transfers of step u + 2 are still in flight),
     // everything is published, the transfer of step u + 3 starts
@@ -261,11 +277,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(FwdCfg<D>::
     auto close_step = [&]() {
         b_cur = b_nxt;
         b_nxt = (b_nxt == (C::NBUF - 1) * C::BUF) ? 0 : b_nxt + C::BUF;
-        ++u;
     };
     __syncthreads();           // the staged rows, the mask tables and the zeroed accumulator are visible
 
-    for (int r = 0; r < R; ++r) {
+    for (int r = r_first; r < R; ++r) {
         const int dlt = 8 * r + wave;
         const int kr = i - dlt;
         const bool col_ok = row_ok && kr >= 0 && dlt < p.w2;
@@ -388,7 +403,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(FwdCfg<D>::
             }
         } else {
             int n = 0;
-            if (r == 0) {
+            if (r == r_first) {
                 // ---- the wave's very first step, the diagonal tile of its first offset: every valid row
                 // attends an entry of it, so this is where the rows get their softmax reference M
                 open_step();
@@ -548,8 +563,17 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(FwdCfg<D>::
         float L = 0.f;
 #pragma unroll
         for (int w = 0; w < 8; ++w) L += xl[w * 32 + row];
-        const float inv = 1.f / L;
         const float *src = acc_sh + row * C::APITCH + seg * SEG;
+        if constexpr (SPLIT) {
+            // (a share that attends nothing of a row leaves zeros with the reference -inf)
+            const int64_t rows = (int64_t)p.B * p.H * N, prow = (int64_t)split * rows + ((int64_t)b * p.H + h) * N + ir;
+            float *dst = p.q_parts + prow * D + seg * SEG;
+#pragma unroll
+            for (int x = 0; x < SEG; x += 2) *reinterpret_cast<float2 *>(dst + x) = *reinterpret_cast<const float2 *>(src + x);
+            if (seg == 0) *reinterpret_cast<float2 *>(p.q_parts + (int64_t)p.q_splits * rows * D + 2 * prow) = make_float2(xm[row], L);
+            return;
+        }
+        const float inv = 1.f / L;
         char *orow = p.o.ptr + b * p.o.sb + (int64_t)ir * p.o.sn + h * p.o.sh + seg * SEG * 2;
         char *rrow = p.o_lo.ptr ? p.o_lo.ptr + b * p.o_lo.sb + (int64_t)ir * p.o_lo.sn + h * p.o_lo.sh + seg * SEG * 2 : nullptr;
         float o[SEG];
@@ -585,6 +609,53 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(FwdCfg<D>::
         }
         if (seg == 0) p.lse[((int64_t)b * p.H + h) * N + ir] = (xm[row] + __builtin_amdgcn_logf(L)) * kLn2;
     }
+}
+
+// Output and lse from the shares of split query tiles: out = sum_s O_s 2^(m_s - m) / sum_s l_s 2^(m_s - m), m = max m_s, in
+// split order; a thread holds 8 d of one row
+template <int D>
+__global__ __launch_bounds__(256) void fwd_combine_kernel(KParams p) {
+    constexpr int LP = D / 8;
+    const int64_t rows = (int64_t)p.B * p.H * p.N;
+    const int64_t row = (int64_t)blockIdx.x * (256 / LP) + threadIdx.x / LP;
+    if (row >= rows) return;
+    const int piece = threadIdx.x % LP;
+    const int i = (int)(row % p.N);
+    const int h = (int)((row / p.N) % p.H);
+    const int b = (int)(row / ((int64_t)p.N * p.H));
+    const int rounds = fwd_rounds(i / 32, p.w2);
+    const int splits = p.q_splits < rounds ? p.q_splits : rounds;
+    const float2 *ml = reinterpret_cast<const float2 *>(p.q_parts + (int64_t)p.q_splits * rows * D) + row;
+    float m = -INFINITY;
+    for (int s = 0; s < splits; ++s) m = fmaxf(m, ml[s * rows].x);
+    float L = 0.f, o[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    const float *src = p.q_parts + row * D + piece * 8;
+#pragma unroll 4
+    for (int s = 0; s < splits; ++s) {
+        const float2 x = ml[s * rows];
+        const float4 a0 = *reinterpret_cast<const float4 *>(src + s * rows * D), a1 = *reinterpret_cast<const float4 *>(src + s * rows * D + 4);
+        const float w = fast_exp2(x.x - m);
+        L += x.y * w;
+        o[0] += a0.x * w;
+        o[1] += a0.y * w;
+        o[2] += a0.z * w;
+        o[3] += a0.w * w;
+        o[4] += a1.x * w;
+        o[5] += a1.y * w;
+        o[6] += a1.z * w;
+        o[7] += a1.w * w;
+    }
+    const float inv = 1.f / L;
+    u32x4 ov, rv;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+        const float x = o[2 * w] * inv, y = o[2 * w + 1] * inv;
+        ov[w] = pack_bf16(x, y);
+        rv[w] = pack_bf16(x - bf16_lo(ov[w]), y - bf16_hi(ov[w]));
+    }
+    st_global16(p.o.ptr + b * p.o.sb + (int64_t)i * p.o.sn + h * p.o.sh + piece * 16, ov);
+    if (p.o_lo.ptr) st_global16(p.o_lo.ptr + b * p.o_lo.sb + (int64_t)i * p.o_lo.sn + h * p.o_lo.sh + piece * 16, rv);
+    if (piece == 0) p.lse[row] = (m + __builtin_amdgcn_logf(L)) * kLn2;
 }
 
 }  // namespace sa2

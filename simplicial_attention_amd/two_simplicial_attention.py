@@ -156,12 +156,14 @@ class SlidingTwoSimplicialAttention(Function):
                 partials_budget.release(t_bytes, index)
                 raise
             partials_budget.track(t_save, t_bytes)
+        fwd_ws_bytes = lib.sa2_fwd_workspace_bytes(prob)
+        fwd_ws = torch.empty(fwd_ws_bytes, dtype=torch.uint8, device=q.device) if fwd_ws_bytes else None
         with torch.cuda.device_of(q):
-            _native.check(lib.sa2_fwd(prob, *(_native.tensor_arg(t) for t in (q, k1, k2, v1, v2, out)),
+            _native.check(lib.sa2_fwd_ws(prob, *(_native.tensor_arg(t) for t in (q, k1, k2, v1, v2, out)),
                                       _native.tensor_arg(residual) if needs_grad else None,
                                       lse.data_ptr(),
                                       _native.saved_arg(t_save, m_save) if t_save is not None else None,
-                                      _stream_handle(q.device)))
+                                      fwd_ws.data_ptr() if fwd_ws_bytes else None, fwd_ws_bytes, _stream_handle(q.device)))
         ctx.save_for_backward(q, k1, k2, v1, v2, out, lse, residual, t_save, m_save)
         ctx.problem = (batch, seq_len, heads, kv_heads, dim, w1, w2, scale)
         ctx.in_dtype = in_dtype
@@ -177,12 +179,11 @@ class SlidingTwoSimplicialAttention(Function):
         dq = torch.empty_like(q)
         dk1, dk2, dv1, dv2 = (torch.empty((batch, seq_len, kv_heads, dim), dtype=q.dtype, device=q.device) for _ in range(4))
         prob = _native.problem(batch, seq_len, heads, kv_heads, dim, w1, w2, True, scale)
-        # (with the forward's saved partials only the dK2 half of the workspace is used)
-        ws_bytes = lib.sa2_bwd_workspace_bytes_with_saved(prob) if t_save is not None else lib.sa2_bwd_workspace_bytes(prob)
+        ws_bytes = lib.sa2_bwd_split_workspace_bytes(prob, t_save is not None)
         workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
         arg = _native.tensor_arg
         with torch.cuda.device_of(q):
-            _native.check(lib.sa2_bwd(prob, arg(q), arg(k1), arg(k2), arg(v1), arg(v2), arg(out),
+            _native.check(lib.sa2_bwd_split(prob, arg(q), arg(k1), arg(k2), arg(v1), arg(v2), arg(out),
                                       arg(residual) if residual is not None else None, arg(dout),
                                       lse.data_ptr(),
                                       _native.saved_arg(t_save, m_save) if t_save is not None else None,
