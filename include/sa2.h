@@ -219,6 +219,22 @@ int sa2_bwd_noalloc(const sa2_problem *prob,
                     const sa2_tensor *dq, const sa2_tensor *dk1, const sa2_tensor *dk2,
                     const sa2_tensor *dv1, const sa2_tensor *dv2, void *hip_stream);
 
+/* ---- tensors of other types and head dimensions ----
+ *
+ * Converts up to SA2_CONVERT_MOST (batch, seq, heads, dim) tensors in one launch: element type of `src` to that of `dst`
+ * (round to nearest even), channels src_dim .. dst_dim - 1 of `dst` zero, channels beyond dst_dim of `src` left out.
+ * Innermost strides are 1; any alignment (16-byte aligned rows move faster).  The reference's kernels take any float
+ * type (triton_two_simplicial_attention.py:110-112) and a head dimension of 64. */
+typedef enum sa2_element { SA2_ELEMENT_BF16 = 0, SA2_ELEMENT_F16 = 1, SA2_ELEMENT_F32 = 2 } sa2_element;
+typedef struct sa2_conversion {
+    sa2_tensor src, dst;
+    int32_t src_type, dst_type;     /* sa2_element */
+    int32_t src_dim, dst_dim;
+    int32_t batch, seq_len, heads;
+} sa2_conversion;
+#define SA2_CONVERT_MOST 6
+int sa2_convert(const sa2_conversion *items, int32_t count, void *hip_stream);
+
 /* ---- module pre-processing around the attention core (first of the "next" rows) ----
  *
  * Fused split + per-head RMSNorm of the qkv projection.  Replaces, for

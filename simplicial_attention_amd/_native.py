@@ -7,12 +7,14 @@ an exception is raised.
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import os
 import subprocess
 import threading
 
 _CSRC = os.path.join(os.path.dirname(os.path.abspath(__file__)), 'csrc')
 LIB_PATH = os.path.join(_CSRC, 'libsa2.so')
+TORCH_EXT_PATH = os.path.join(_CSRC, '_sa2_torch.so')    # host path of the autograd Functions, links libsa2.so
 PROF_LIB_PATH = os.path.join(_CSRC, 'libsa2_prof.so')   # -DSA2_PROFILING build, for bench.py only
 
 SA2_OK = 0
@@ -29,7 +31,7 @@ EXPORTS = ('sa2_version', 'sa2_last_error', 'sa2_supported', 'sa2_saved_t_bytes'
            'sa2_bwd_delta', 'sa2_bwd_workspace_bytes', 'sa2_bwd_workspace_bytes_with_saved',
            'sa2_bwd_split', 'sa2_bwd_split_workspace_bytes', 'sa2_bwd_dq_dkv2', 'sa2_bwd_dkv1', 'sa2_bwd',
            'sa2_bwd_noalloc_scratch_bytes', 'sa2_bwd_noalloc',
-           'sa2_qkv_norm_fwd', 'sa2_qkv_norm_bwd_workspace_bytes', 'sa2_qkv_norm_bwd')
+           'sa2_convert', 'sa2_qkv_norm_fwd', 'sa2_qkv_norm_bwd_workspace_bytes', 'sa2_qkv_norm_bwd')
 
 
 class Sa2Error(RuntimeError):
@@ -57,13 +59,14 @@ class Saved(ctypes.Structure):
 
 _lib = None
 _prof_lib = None
+_torch_ext = None
 _lock = threading.Lock()
 
 
 def build(verbose: bool = False) -> str:
     """Compile libsa2.so for gfx950 (always recompiles)."""
     out = None if verbose else subprocess.DEVNULL
-    subprocess.check_call(['make', '-B', '-C', _CSRC, 'libsa2.so', 'libsa2_prof.so'], stdout=out, stderr=out)
+    subprocess.check_call(['make', '-B', '-C', _CSRC, 'libsa2.so', 'libsa2_prof.so', '_sa2_torch.so'], stdout=out, stderr=out)
     return LIB_PATH
 
 
@@ -132,6 +135,27 @@ def load_profiling() -> ctypes.CDLL:
                 raise _missing(PROF_LIB_PATH)
             _prof_lib = _declare(ctypes.CDLL(PROF_LIB_PATH))
         return _prof_lib
+
+
+def torch_ext():
+    """The module _sa2_torch (sa2_torch.cpp).  Raises if it has not been built."""
+    global _torch_ext
+    if _torch_ext is None:
+        with _lock:
+            if _torch_ext is None:
+                for path in (LIB_PATH, TORCH_EXT_PATH):
+                    if not os.path.exists(path):
+                        raise _missing(path)
+                import torch  # noqa: F401  (its libraries have to be in the process first)
+                spec = importlib.util.spec_from_file_location('_sa2_torch', TORCH_EXT_PATH)
+                module = importlib.util.module_from_spec(spec)
+                spec.loader.exec_module(module)
+                _torch_ext = module
+    return _torch_ext
+
+
+def check_failed(status: int, message: str) -> None:
+    raise Sa2Error(status, message)
 
 
 def check(status: int) -> None:

@@ -14,6 +14,7 @@
 #include "sa2_bwd_kv8.hpp"
 #include "sa2_bwd_q.hpp"
 #include "sa2_common.hpp"
+#include "sa2_convert.hpp"
 #include "sa2_lds.hpp"
 #include "sa2_qkv_norm.hpp"
 #include "sa2_fwd.hpp"
@@ -682,6 +683,50 @@ int sa2_bwd_noalloc(const sa2_problem *prob, const sa2_tensor *q, const sa2_tens
     // call (delta rows, partial rows), so nothing needs clearing between calls
     return sa2_bwd(prob, q, k1, k2, v1, v2, out, out_residual, dout, lse, saved, delta, dq, dk1, dk2, dv1, dv2, ws,
                    sa2_bwd_workspace_bytes(prob), hip_stream);
+}
+
+// ---- type and head dimension conversion
+int sa2_convert(const sa2_conversion *items, int32_t count, void *hip_stream) {
+    static_assert(SA2_CONVERT_MOST == sa2::kConvertMost, "tensors per launch");
+    if (!items) return fail(SA2_ERR_NULL_POINTER, "items is NULL");
+    if (count < 1 || count > SA2_CONVERT_MOST) return fail(SA2_ERR_BAD_SHAPE, "%d conversions: 1 to %d fit one call", count, SA2_CONVERT_MOST);
+    sa2::ConvertParams p{};
+    int64_t most = 0;
+    for (int x = 0; x < count; ++x) {
+        const sa2_conversion &c = items[x];
+        if (!c.src.ptr || !c.dst.ptr) return fail(SA2_ERR_NULL_POINTER, "conversion %d: src or dst is NULL", x);
+        if (c.batch < 1 || c.seq_len < 1 || c.heads < 1 || c.src_dim < 1 || c.dst_dim < 1)
+            return fail(SA2_ERR_BAD_SHAPE, "conversion %d: sizes must be >= 1", x);
+        if (c.src_type < 0 || c.src_type > SA2_ELEMENT_F32 || c.dst_type < 0 || c.dst_type > SA2_ELEMENT_F32)
+            return fail(SA2_ERR_UNSUPPORTED, "conversion %d: unknown element type", x);
+        sa2::ConvertTensor &t = p.t[x];
+        auto vec = [](const sa2_tensor &a, int type) {
+            const int per16 = type == SA2_ELEMENT_F32 ? 4 : 8;
+            return (reinterpret_cast<uintptr_t>(a.ptr) & 15) == 0 && a.stride_b % per16 == 0 && a.stride_n % per16 == 0 && a.stride_h % per16 == 0;
+        };
+        t.src = static_cast<const char *>(c.src.ptr);
+        t.dst = static_cast<char *>(c.dst.ptr);
+        t.ssb = c.src.stride_b;
+        t.ssn = c.src.stride_n;
+        t.ssh = c.src.stride_h;
+        t.dsb = c.dst.stride_b;
+        t.dsn = c.dst.stride_n;
+        t.dsh = c.dst.stride_h;
+        t.src_type = c.src_type;
+        t.dst_type = c.dst_type;
+        t.src_dim = c.src_dim;
+        t.dst_dim = c.dst_dim;
+        t.N = c.seq_len;
+        t.H = c.heads;
+        t.pieces = (int64_t)c.batch * c.seq_len * c.heads * ((c.dst_dim + 7) / 8);
+        t.src_vec = vec(c.src, c.src_type);
+        t.dst_vec = vec(c.dst, c.dst_type);
+        most = t.pieces > most ? t.pieces : most;
+    }
+    const int64_t blocks = (most + 255) / 256;
+    const int grid = (int)(blocks < 16 * kComputeUnits ? blocks : 16 * kComputeUnits);
+    hipLaunchKernelGGL(sa2::convert_kernel, dim3(grid, count), dim3(256), 0, static_cast<hipStream_t>(hip_stream), p);
+    return after_launch("convert");
 }
 
 // ---- fused split + per-head RMSNorm of the qkv projection -------------------------------

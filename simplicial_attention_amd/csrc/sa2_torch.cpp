@@ -1,0 +1,380 @@
+// Host path of the package's autograd Functions: argument checks, allocation, the launches of libsa2 and the autograd
+// nodes, in one native call per direction.  (From Python through ctypes the same work took 25 us for a forward and 150 us
+// for a forward and backward, which is what small calls then cost whatever the kernels do.)
+//
+// Bound to Python as the module _sa2_torch; two_simplicial_attention.py and qkv_norm.py are its callers.
+#include <torch/extension.h>
+
+#include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <c10/core/DeviceGuard.h>
+
+#include <array>
+#include <atomic>
+
+#include "sa2.h"
+
+namespace py = pybind11;
+using at::Tensor;
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+
+namespace {
+
+constexpr int kMostDevices = 64;
+// bytes of saved partials that have died, per device (the budget in Python subtracts them from what it admitted)
+std::array<std::atomic<int64_t>, kMostDevices> g_released{};
+
+void check(int status) {
+    if (status == SA2_OK) return;
+    // the exception class of the package (Sa2Error) is raised by its own check function
+    py::gil_scoped_acquire gil;
+    py::module_::import("simplicial_attention_amd._native").attr("check_failed")(status, std::string(sa2_last_error()));
+}
+
+[[noreturn]] void raise(PyObject *type, const std::string &text) {
+    py::gil_scoped_acquire gil;
+    PyErr_SetString(type, text.c_str());
+    throw py::error_already_set();
+}
+
+void *stream_of(const Tensor &t) { return c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(t.device().index()).stream(); }
+
+sa2_tensor arg(const Tensor &t) { return {t.data_ptr(), t.stride(0), t.stride(1), t.stride(2)}; }
+
+// the kernels need a unit innermost stride, 16-byte aligned rows and base
+Tensor aligned(const Tensor &t) {
+    const bool ok = t.stride(3) == 1 && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 && t.stride(0) % 8 == 0 && t.stride(1) % 8 == 0 &&
+                    t.stride(2) % 8 == 0;
+    return ok ? t : t.clone(at::MemoryFormat::Contiguous);
+}
+
+int element_of(const Tensor &t) {
+    switch (t.scalar_type()) {
+        case at::kBFloat16: return SA2_ELEMENT_BF16;
+        case at::kHalf: return SA2_ELEMENT_F16;
+        case at::kFloat: return SA2_ELEMENT_F32;
+        default: return -1;
+    }
+}
+
+// Several conversions in one launch.
+struct Conversions {
+    sa2_conversion items[SA2_CONVERT_MOST];
+    int count = 0;
+    void add(const Tensor &src, const Tensor &dst) {
+        sa2_conversion &c = items[count++];
+        c.src = arg(src);
+        c.dst = arg(dst);
+        c.src_type = element_of(src);
+        c.dst_type = element_of(dst);
+        c.src_dim = (int)src.size(3);
+        c.dst_dim = (int)dst.size(3);
+        c.batch = (int)src.size(0);
+        c.seq_len = (int)src.size(1);
+        c.heads = (int)src.size(2);
+    }
+    void run(void *stream) {
+        if (count) check(sa2_convert(items, count, stream));
+    }
+};
+
+Tensor rows_of(const Tensor &t) { return t.stride(3) == 1 ? t : t.contiguous(); }
+
+// a (b, n, h, d) tensor as bf16 rows of `dim` channels, converted if it is not that already (the conversion is queued)
+Tensor as_rows(const Tensor &t, int64_t dim, Conversions &todo, std::vector<Tensor> &alive) {
+    if (t.scalar_type() == at::kBFloat16 && t.size(3) == dim) return aligned(t);
+    Tensor src = rows_of(t), dst = at::empty({t.size(0), t.size(1), t.size(2), dim}, t.options().dtype(at::kBFloat16));
+    todo.add(src, dst);
+    alive.push_back(src);
+    return dst;
+}
+
+struct Geometry {
+    int64_t batch, seq, heads, kv_heads, dim_qk, dim_v, dim;      // dim: the kernels' head dimension
+    int64_t w1, w2;
+    double scale;
+    sa2_problem problem() const {
+        return {(int32_t)batch, (int32_t)seq, (int32_t)heads, (int32_t)kv_heads, (int32_t)dim, (int32_t)w1, (int32_t)w2, 1, (float)scale, SA2_BF16};
+    }
+};
+
+struct Forward {
+    Tensor q, k1, k2, v1, v2;          // the kernels' operands
+    Tensor out, lse, residual, t_save, m_save;
+    Tensor result;                     // out in the caller's type and head dimension
+};
+
+// a buffer that reports its bytes as released when its last tensor dies
+Tensor counted_buffer(int64_t bytes, const Tensor &like, int64_t counted) {
+    Tensor base = at::empty({bytes}, like.options().dtype(at::kByte));
+    void *ptr = base.data_ptr();
+    const int device = like.device().index();
+    return at::for_blob(ptr, {bytes})
+        .deleter([base, device, counted](void *) mutable {
+            base.reset();
+            g_released[device].fetch_add(counted);
+        })
+        .options(like.options().dtype(at::kByte))
+        .target_device(like.device())
+        .make_tensor();
+}
+
+Forward run_forward(const Tensor &q, const Tensor &k1, const Tensor &k2, const Tensor &v1, const Tensor &v2, const Geometry &g, bool needs_grad,
+                    bool save) {
+    Forward f;
+    const c10::DeviceGuard guard(q.device());
+    void *stream = stream_of(q);
+    Conversions todo;
+    std::vector<Tensor> alive;
+    f.q = as_rows(q, g.dim, todo, alive);
+    f.k1 = as_rows(k1, g.dim, todo, alive);
+    f.k2 = as_rows(k2, g.dim, todo, alive);
+    f.v1 = as_rows(v1, g.dim, todo, alive);
+    f.v2 = as_rows(v2, g.dim, todo, alive);
+    todo.run(stream);
+    const auto bf16 = q.options().dtype(at::kBFloat16);
+    f.out = at::empty({g.batch, g.seq, g.heads, g.dim}, bf16);
+    f.lse = at::empty({g.batch, g.heads, g.seq}, q.options().dtype(at::kFloat));
+    // bf16 residual of the fp32 accumulator, kept only when a backward may follow
+    if (needs_grad) f.residual = at::empty({g.batch, g.seq, g.heads, g.dim}, bf16);
+    const sa2_problem prob = g.problem();
+    sa2_saved saved{};
+    if (save) {
+        const int64_t t_bytes = sa2_saved_t_bytes(&prob), m_bytes = sa2_saved_m_bytes(&prob);
+        try {
+            f.t_save = counted_buffer(t_bytes, q, t_bytes + m_bytes);
+        } catch (...) {
+            g_released[q.device().index()].fetch_add(t_bytes + m_bytes);      // (no buffer: give the admitted bytes back)
+            throw;
+        }
+        f.m_save = at::empty({g.batch, g.heads, g.w2, g.seq}, f.lse.options());
+        saved = {f.t_save.data_ptr(), static_cast<float *>(f.m_save.data_ptr())};
+    }
+    const int64_t ws_bytes = sa2_fwd_workspace_bytes(&prob);
+    Tensor ws;
+    if (ws_bytes > 0) ws = at::empty({ws_bytes}, q.options().dtype(at::kByte));
+    const sa2_tensor aq = arg(f.q), ak1 = arg(f.k1), ak2 = arg(f.k2), av1 = arg(f.v1), av2 = arg(f.v2), ao = arg(f.out);
+    sa2_tensor ar{};
+    if (needs_grad) ar = arg(f.residual);
+    check(sa2_fwd_ws(&prob, &aq, &ak1, &ak2, &av1, &av2, &ao, needs_grad ? &ar : nullptr, static_cast<float *>(f.lse.data_ptr()),
+                     save ? &saved : nullptr, ws_bytes > 0 ? ws.data_ptr() : nullptr, ws_bytes, stream));
+    if (q.scalar_type() == at::kBFloat16 && g.dim_v == g.dim) {
+        f.result = f.out;
+    } else {
+        f.result = at::empty({g.batch, g.seq, g.heads, g.dim_v}, q.options());
+        Conversions back;
+        back.add(f.out, f.result);
+        back.run(stream);
+    }
+    return f;
+}
+
+struct Attend : public torch::autograd::Function<Attend> {
+    static Tensor forward(AutogradContext *ctx, const Tensor &q, const Tensor &k1, const Tensor &k2, const Tensor &v1, const Tensor &v2,
+                          const Geometry &g, bool save) {
+        Forward f = run_forward(q, k1, k2, v1, v2, g, true, save);
+        ctx->save_for_backward({f.q, f.k1, f.k2, f.v1, f.v2, f.out, f.lse, f.residual, f.t_save, f.m_save});
+        c10::List<int64_t> n;
+        for (const int64_t v : {g.batch, g.seq, g.heads, g.kv_heads, g.dim_qk, g.dim_v, g.dim, g.w1, g.w2}) n.push_back(v);
+        for (const Tensor *t : {&q, &k1, &k2, &v1, &v2}) n.push_back((int64_t)t->scalar_type());
+        ctx->saved_data["geometry"] = n;
+        ctx->saved_data["scale"] = g.scale;
+        return f.result;
+    }
+
+    static variable_list backward(AutogradContext *ctx, variable_list douts) {
+        const variable_list s = ctx->get_saved_variables();
+        const Tensor &q = s[0], &k1 = s[1], &k2 = s[2], &v1 = s[3], &v2 = s[4], &out = s[5], &lse = s[6], &residual = s[7], &t_save = s[8], &m_save = s[9];
+        const c10::List<int64_t> n = ctx->saved_data["geometry"].toIntList();
+        Geometry g;
+        g.batch = n[0]; g.seq = n[1]; g.heads = n[2]; g.kv_heads = n[3]; g.dim_qk = n[4]; g.dim_v = n[5]; g.dim = n[6]; g.w1 = n[7]; g.w2 = n[8];
+        g.scale = ctx->saved_data["scale"].toDouble();
+        const c10::DeviceGuard guard(q.device());
+        void *stream = stream_of(q);
+        Conversions todo;
+        std::vector<Tensor> alive;
+        const Tensor dout = as_rows(douts[0], g.dim, todo, alive);
+        todo.run(stream);
+        const auto bf16 = q.options();
+        const std::array<int64_t, 4> q_shape{g.batch, g.seq, g.heads, g.dim}, kv_shape{g.batch, g.seq, g.kv_heads, g.dim};
+        variable_list grads(5);
+        for (int x = 0; x < 5; ++x) grads[x] = at::empty(x == 0 ? q_shape : kv_shape, bf16);
+        const sa2_problem prob = g.problem();
+        sa2_saved saved{};
+        const bool have_saved = t_save.defined();
+        if (have_saved) saved = {t_save.data_ptr(), static_cast<float *>(m_save.data_ptr())};
+        // delta rows and the kernels' workspace in one buffer
+        const int64_t delta_bytes = (g.batch * g.heads * g.seq * 4 + 255) / 256 * 256, ws_bytes = sa2_bwd_split_workspace_bytes(&prob, have_saved);
+        const Tensor ws = at::empty({delta_bytes + ws_bytes}, q.options().dtype(at::kByte));
+        char *base = static_cast<char *>(ws.data_ptr());
+        const sa2_tensor aq = arg(q), ak1 = arg(k1), ak2 = arg(k2), av1 = arg(v1), av2 = arg(v2), ao = arg(out), ar = arg(residual), ad = arg(dout);
+        sa2_tensor ag[5];
+        for (int x = 0; x < 5; ++x) ag[x] = arg(grads[x]);
+        check(sa2_bwd_split(&prob, &aq, &ak1, &ak2, &av1, &av2, &ao, &ar, &ad, static_cast<float *>(lse.data_ptr()), have_saved ? &saved : nullptr,
+                            reinterpret_cast<float *>(base), &ag[0], &ag[1], &ag[2], &ag[3], &ag[4], base + delta_bytes, ws_bytes, stream));
+        // back to the types and head dimensions of the inputs
+        Conversions back;
+        variable_list result(7);
+        for (int x = 0; x < 5; ++x) {
+            const auto type = (at::ScalarType)(int64_t)n[9 + x];
+            const int64_t dim = x < 3 ? g.dim_qk : g.dim_v;
+            if (type == at::kBFloat16 && dim == g.dim) {
+                result[x] = grads[x];
+            } else {
+                result[x] = at::empty({g.batch, g.seq, x == 0 ? g.heads : g.kv_heads, dim}, q.options().dtype(type));
+                back.add(grads[x], result[x]);
+            }
+        }
+        back.run(stream);
+        return result;
+    }
+};
+
+int64_t kernel_dim(int64_t dim) {
+    for (const int64_t d : {32, 64, 128, 256})
+        if (dim <= d) return d;
+    return 0;
+}
+
+// `save`: called with the bytes of the partials, says whether they may be kept
+Tensor attend(const Tensor &q, const Tensor &k1, const Tensor &k2, const Tensor &v1, const Tensor &v2, int64_t w1, int64_t w2, double scale,
+              const py::object &admit) {
+    Geometry g;
+    g.batch = q.size(0);
+    g.seq = q.size(1);
+    g.heads = q.size(2);
+    g.kv_heads = k1.size(2);
+    g.dim_qk = q.size(3);
+    g.dim_v = v1.size(3);
+    g.dim = kernel_dim(std::max(g.dim_qk, g.dim_v));
+    g.w1 = w1;
+    g.w2 = w2;
+    g.scale = scale;
+    const bool needs_grad = at::GradMode::is_enabled() && (q.requires_grad() || k1.requires_grad() || k2.requires_grad() || v1.requires_grad() || v2.requires_grad());
+    if (!needs_grad) return run_forward(q, k1, k2, v1, v2, g, false, false).result;
+    // per-offset value partials, kept for the backward when they fit the budget: dV2 then needs no recomputation of the
+    // attention weights (a size of 0: the kernels of this head dimension keep none)
+    const sa2_problem prob = g.problem();
+    const int64_t bytes = sa2_saved_t_bytes(&prob) + sa2_saved_m_bytes(&prob);
+    const bool save = bytes > 0 && admit(bytes, (int)q.device().index()).cast<bool>();
+    return Attend::apply(q, k1, k2, v1, v2, g, save);
+}
+
+// shapes, types and windows of the Function and the wrapper; `pads`: other head dimensions and types than the kernels' are welcome
+Tensor checked_attend(const Tensor &q, const Tensor &k1, const Tensor &k2, const Tensor &v1, const Tensor &v2, int64_t w1, int64_t w2,
+                      std::optional<double> scale, bool pads, const py::object &admit) {
+    const Tensor *all[5] = {&q, &k1, &k2, &v1, &v2};
+    for (const Tensor *t : all)
+        if (!t->is_cuda()) raise(PyExc_AssertionError, "sliding-window 2-simplicial attention runs on the GPU only");
+    for (const Tensor *t : all)
+        if (element_of(*t) < 0 || (!pads && t->scalar_type() != q.scalar_type()))
+            raise(PyExc_TypeError, "q, k1, k2, v1, v2 must share one dtype out of bfloat16, float16, float32");
+    if (q.dim() != 4) raise(PyExc_ValueError, "expected (batch, seq, heads, dim_head) tensors");
+    for (const Tensor *t : all)
+        if (t->dim() != 4 || t->size(0) != q.size(0) || t->size(1) != q.size(1) || (t != &q && t->size(2) != k1.size(2)) ||
+            t->size(3) != (t == &v1 || t == &v2 ? (pads ? v1 : q) : q).size(3) || t->device() != q.device())
+            raise(PyExc_ValueError, "key/value shape " + std::string(py::str(py::cast(t->sizes().vec()))) + " does not match the queries' " +
+                                        std::string(py::str(py::cast(q.sizes().vec()))));
+    if (k1.size(2) < 1 || q.size(2) % k1.size(2) != 0)
+        raise(PyExc_ValueError, "query heads " + std::to_string(q.size(2)) + " not divisible by key/value heads " + std::to_string(k1.size(2)));
+    if (w1 < 1 || w2 < 1) raise(PyExc_ValueError, "window sizes must be at least 1");
+    const int64_t dim = std::max(q.size(3), v1.size(3));
+    if (pads ? dim > 256 || dim < 1 : !sa2_supported((int32_t)dim, 1, 1, SA2_BF16))
+        raise(PyExc_NotImplementedError, "dim_head=" + std::to_string(dim) + " is not covered by the kernels (dim_head 32, 64, 128 or 256)");
+    return attend(q, k1, k2, v1, v2, std::min<int64_t>(w1, INT32_MAX), std::min<int64_t>(w2, INT32_MAX),
+                  scale ? *scale : 1.0 / std::sqrt((double)q.size(3)), admit);
+}
+
+// ---- fused split + per-head RMSNorm of the qkv projection
+struct QKVNorm : public torch::autograd::Function<QKVNorm> {
+    using Weight = std::optional<Tensor>;
+    static variable_list forward(AutogradContext *ctx, const Tensor &qkv, const Weight &wq, const Weight &wk1, const Weight &wk2, const Weight &wv1,
+                                 const Weight &wv2, int64_t heads, int64_t kv_heads, int64_t dim, double eps) {
+        return run(ctx, qkv, {&wq, &wk1, &wk2, &wv1, &wv2}, heads, kv_heads, dim, eps);
+    }
+
+    // (ctx == nullptr: no backward follows)
+    static variable_list run(AutogradContext *ctx, const Tensor &qkv_in, const std::array<const Weight *, 5> &w, int64_t heads, int64_t kv_heads,
+                             int64_t dim, double eps) {
+        const int64_t batch = qkv_in.size(0), seq = qkv_in.size(1);
+        const Tensor qkv = qkv_in.stride(2) == 1 && qkv_in.stride(0) == seq * qkv_in.stride(1) ? qkv_in : qkv_in.contiguous();
+        const c10::DeviceGuard guard(qkv.device());
+        variable_list weights(5), outs(5);
+        for (int x = 0; x < 5; ++x)
+            if (w[x]->has_value()) weights[x] = (*w[x])->detach().to(at::kBFloat16).contiguous();
+        for (int x = 0; x < 5; ++x) outs[x] = at::empty({batch, seq, x == 0 ? heads : kv_heads, dim}, qkv.options());
+        const Tensor rstd = at::empty({batch * seq, heads + 4 * kv_heads}, qkv.options().dtype(at::kFloat));
+        const sa2_problem prob = problem(batch, seq, heads, kv_heads, dim);
+        sa2_tensor a[5];
+        const void *p[5];
+        for (int x = 0; x < 5; ++x) {
+            a[x] = arg(outs[x]);
+            p[x] = weights[x].defined() ? weights[x].data_ptr() : nullptr;
+        }
+        check(sa2_qkv_norm_fwd(&prob, qkv.data_ptr(), qkv.stride(1), p[0], p[1], p[2], p[3], p[4], (float)eps, &a[0], &a[1], &a[2], &a[3], &a[4],
+                               static_cast<float *>(rstd.data_ptr()), stream_of(qkv)));
+        if (ctx) {
+            ctx->save_for_backward({qkv, rstd, weights[0], weights[1], weights[2], weights[3], weights[4]});
+            c10::List<int64_t> n;
+            for (const int64_t v : {batch, seq, heads, kv_heads, dim}) n.push_back(v);
+            for (int x = 0; x < 5; ++x) n.push_back(w[x]->has_value() ? (int64_t)(*w[x])->scalar_type() : -1);
+            ctx->saved_data["geometry"] = n;
+        }
+        return outs;
+    }
+
+    static sa2_problem problem(int64_t batch, int64_t seq, int64_t heads, int64_t kv_heads, int64_t dim) {
+        return {(int32_t)batch, (int32_t)seq, (int32_t)heads, (int32_t)kv_heads, (int32_t)dim, 1, 1, 1, 1.f, SA2_BF16};
+    }
+
+    static variable_list backward(AutogradContext *ctx, variable_list douts) {
+        const variable_list s = ctx->get_saved_variables();
+        const Tensor &qkv = s[0], &rstd = s[1];
+        const c10::List<int64_t> n = ctx->saved_data["geometry"].toIntList();
+        const int64_t batch = n[0], seq = n[1], heads = n[2], kv_heads = n[3], dim = n[4];
+        const c10::DeviceGuard guard(qkv.device());
+        const sa2_problem prob = problem(batch, seq, heads, kv_heads, dim);
+        sa2_tensor a[5];
+        const void *p[5];
+        for (int x = 0; x < 5; ++x) {
+            douts[x] = douts[x].defined() ? aligned(douts[x]) : at::zeros({batch, seq, x == 0 ? heads : kv_heads, dim}, qkv.options());
+            a[x] = arg(douts[x]);
+            p[x] = s[2 + x].defined() ? s[2 + x].data_ptr() : nullptr;
+        }
+        const Tensor dqkv = at::empty({batch, seq, qkv.size(2)}, qkv.options());
+        const Tensor dw = at::empty({5, dim}, qkv.options().dtype(at::kFloat));
+        const int64_t ws_bytes = sa2_qkv_norm_bwd_workspace_bytes(&prob);
+        const Tensor ws = at::empty({ws_bytes}, qkv.options().dtype(at::kByte));
+        check(sa2_qkv_norm_bwd(&prob, qkv.data_ptr(), qkv.stride(1), p[0], p[1], p[2], p[3], p[4], &a[0], &a[1], &a[2], &a[3], &a[4],
+                               static_cast<float *>(rstd.data_ptr()), dqkv.data_ptr(), static_cast<float *>(dw.data_ptr()), ws.data_ptr(), ws_bytes,
+                               stream_of(qkv)));
+        variable_list result(10);
+        result[0] = dqkv;
+        // (one cast for weights of one type)
+        Tensor cast = dw;
+        for (int x = 0; x < 5; ++x) {
+            if (n[5 + x] < 0) continue;
+            const auto type = (at::ScalarType)(int64_t)n[5 + x];
+            if (cast.scalar_type() != type) cast = dw.to(type);
+            result[1 + x] = cast.select(0, x);
+        }
+        return result;
+    }
+};
+
+variable_list qkv_norm(const Tensor &qkv, const QKVNorm::Weight &wq, const QKVNorm::Weight &wk1, const QKVNorm::Weight &wk2,
+                       const QKVNorm::Weight &wv1, const QKVNorm::Weight &wv2, int64_t heads, int64_t kv_heads, int64_t dim, double eps) {
+    bool grad = qkv.requires_grad();
+    const std::array<const QKVNorm::Weight *, 5> w{&wq, &wk1, &wk2, &wv1, &wv2};
+    for (const auto *x : w) grad = grad || (x->has_value() && (*x)->requires_grad());
+    if (!(grad && at::GradMode::is_enabled())) return QKVNorm::run(nullptr, qkv, w, heads, kv_heads, dim, eps);
+    return QKVNorm::apply(qkv, wq, wk1, wk2, wv1, wv2, heads, kv_heads, dim, eps);
+}
+
+}  // namespace
+
+PYBIND11_MODULE(_sa2_torch, m) {
+    m.def("attend", &checked_attend);
+    m.def("qkv_norm", &qkv_norm);
+    m.def("released_bytes", [](int device) { return device >= 0 && device < kMostDevices ? g_released[device].load() : int64_t(0); });
+}
