@@ -810,7 +810,7 @@ int sa2_qkv_norm_bwd(const sa2_problem *prob, const void *qkv, int64_t row_strid
     SA2_FOR_ANY_DIM_HEAD(prob->dim_head, hipLaunchKernelGGL(sa2::qkv_norm_bwd_kernel<DH>, dim3(blocks), dim3(256), 0, s, np, groups));
     SA2_TRY(after_launch("qkv norm backward"));
     const int n = 5 * prob->dim_head;
-    hipLaunchKernelGGL(sa2::qkv_norm_dw_kernel, dim3((n + 15) / 16), dim3(256), 0, s, np.dw_part, dw, blocks, n);
+    hipLaunchKernelGGL(sa2::qkv_norm_dw_kernel, dim3((n + 15) / 16), dim3(1024), 0, s, np.dw_part, dw, blocks, n);
     return after_launch("qkv norm weight gradients");
 }
 

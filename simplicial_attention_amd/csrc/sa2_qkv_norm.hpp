@@ -142,22 +142,25 @@ __global__ __launch_bounds__(256) void qkv_norm_bwd_kernel(NormParams p, int ngr
     }
 }
 
-// dw[tensor][d] = sum over blocks of the partials, in a fixed order.  A block of 256 threads owns 16 consecutive
-// outputs x = (tensor, d); thread (x, phase) adds the partials of the blocks phase, phase + 16, ... (the 16 threads of
-// a phase read 64 consecutive bytes of one partial), then the 16 phases of an output are added in phase order.
-__global__ __launch_bounds__(256) void qkv_norm_dw_kernel(const float *part, float *dw, int nblocks, int n /* 5 * D */) {
-    __shared__ float red[16][17];
+// dw[tensor][d] = sum over blocks of the partials, in a fixed order.  A block of 1024 threads owns 16 consecutive
+// outputs x = (tensor, d); thread (x, phase) adds the partials of the blocks phase, phase + 64, ... (the 16 threads of
+// a phase read 64 consecutive bytes of one partial), then the 64 phases of an output are added in phase order.
+// Latency-bound: with 16 phases a thread's 128 dependent loads took 36 us, with 64 and eight loads in flight 6 us.
+__global__ __launch_bounds__(1024) void qkv_norm_dw_kernel(const float *part, float *dw, int nblocks, int n /* 5 * D */) {
+    __shared__ float red[64][17];
     const int xl = threadIdx.x & 15, phase = threadIdx.x >> 4;
     const int x = blockIdx.x * 16 + xl;
     float s = 0.f;
-    if (x < n)
-        for (int b = phase; b < nblocks; b += 16) s += part[(int64_t)b * n + x];
+    if (x < n) {
+#pragma unroll 8
+        for (int b = phase; b < nblocks; b += 64) s += part[(int64_t)b * n + x];
+    }
     red[phase][xl] = s;
     __syncthreads();
     if (phase == 0 && x < n) {
         float t = 0.f;
 #pragma unroll
-        for (int q = 0; q < 16; ++q) t += red[q][xl];
+        for (int q = 0; q < 64; ++q) t += red[q][xl];
         dw[x] = t;
     }
 }
