@@ -192,13 +192,13 @@ int64_t sa2_saved_m_bytes(const sa2_problem *prob) {
 static constexpr int kComputeUnits = 256;
 
 // Estimated finish time of `groups` workgroups of at most `longest` units each (their sum: `total`) that the CUs take one
-// at a time: one round of the longest while they fit the chip, else an even share and a ragged end, but hardly less than
+// at a time: one round of the longest while they fit the chip, else an even share and a ragged end, but no less than
 // the whole rounds that workgroups of equal length would take (list schedules of the shapes of the tests and the benchmark
 // end within 5 % of this).
 static double finish_time(double groups, double longest, double total) {
     if (groups <= kComputeUnits) return longest;
     const double full = std::ceil(groups / kComputeUnits) * longest, even = total / kComputeUnits + 0.2 * longest;
-    return full * 0.95 > even ? full * 0.95 : even;
+    return full > even ? full : even;
 }
 
 // Query-stationary kernels: the rounds (eight offsets each) of a query tile over several workgroups.  A unit is one step
@@ -212,43 +212,57 @@ static int64_t q_parts_bytes(const sa2_problem *prob, int splits) {
     return (int64_t)splits * prob->batch * prob->heads * prob->seq_len * prob->dim_head * 4;
 }
 
-static int q_splits(const sa2_problem *prob, int merge_cost) {
+// `shared`: two workgroups of the kernel fit a CU and together finish 1.4 times the work of one (the forward at D = 32
+// and 64), so up to two workgroups per CU run at once and each takes 1.45 times as long.
+static int q_splits(const sa2_problem *prob, int merge_cost, bool shared) {
     if (prob->dim_head == kWideDimHead) return 1;
     const int ntile = (prob->seq_len + 31) / 32;
-    const int64_t heads = (int64_t)prob->batch * prob->heads;
-    const int64_t items = heads * ntile;
-    // (rows of 128 lanes and up fill the chip many times over: nothing to gain)
-    if (items > 8 * kComputeUnits) return 1;
+    const double heads = (double)prob->batch * prob->heads;
+    if (heads * ntile > 4 * kComputeUnits) return 1;       // (fills the chip many times over: nothing to gain)
     const int rounds = sa2::fwd_rounds(ntile - 1, prob->w2);
+    // tiles of equal rounds and steps, as (rounds, steps per round, how many)
+    struct Class {
+        int rounds, steps, count;
+    };
+    Class cls[68];
+    int ncls = 0;
+    for (int t = 0; t < ntile; ++t) {
+        const int lo = 32 * t - prob->w1 + 1 > 0 ? (32 * t - prob->w1 + 1) / 32 : 0;
+        const int r = sa2::fwd_rounds(t, prob->w2), n = t - lo + 1;
+        if (ncls && cls[ncls - 1].rounds == r && cls[ncls - 1].steps == n) ++cls[ncls - 1].count;
+        else if (ncls < 68) cls[ncls++] = {r, n, 1};
+        else ++cls[ncls - 1].count;                        // (windows of over 2000 rows: the last class stands for the rest)
+    }
     int best = 1;
     double best_cost = 0;
     for (int splits = 1; splits <= rounds; ++splits) {
         if (splits > 1 && q_parts_bytes(prob, splits) > kQueryPartBytes) break;
         double total = 0, longest = 0, groups = 0;
-        for (int t = 0; t < ntile; ++t) {
-            const int lo = 32 * t - prob->w1 + 1 > 0 ? (32 * t - prob->w1 + 1) / 32 : 0;
-            const int r = sa2::fwd_rounds(t, prob->w2), n = splits < r ? splits : r;
-            const double step = t - lo + 1 + kRoundEnd;
-            const double one = (r + n - 1) / n * step + kQueryCost;
+        for (int x = 0; x < ncls; ++x) {
+            const int r = cls[x].rounds, n = splits < r ? splits : r;
+            const double step = cls[x].steps + kRoundEnd, one = (r + n - 1) / n * step + kQueryCost;
             longest = one > longest ? one : longest;
-            total += r * step + n * kQueryCost;
-            groups += n;
+            total += cls[x].count * (r * step + n * kQueryCost);
+            groups += (double)cls[x].count * n;
         }
+        groups *= heads;
+        total *= heads;
         const double merge = splits > 1 ? merge_cost + 2.0 * (double)q_parts_bytes(prob, splits) / 3.5e6 : 0;
-        const double cost = finish_time(groups * heads, longest, total * heads) + merge;
-        if (splits == 1 || cost < 0.95 * best_cost) {
+        const double time = shared && groups > kComputeUnits ? finish_time(0.5 * groups, 1.45 * longest, 0.73 * total) : finish_time(groups, longest, total);
+        if (splits == 1 || time + merge < 0.95 * best_cost) {
             best = splits;
-            best_cost = cost;
+            best_cost = time + merge;
         }
     }
     return best;
 }
 
-static constexpr int kFwdMergeCost = 8, kBwdMergeCost = 2;        // (the forward's merge is a launch of its own)
+static int fwd_splits(const sa2_problem *prob) { return q_splits(prob, 8, prob->dim_head != 128); }   // (the merge is a launch of its own)
+static int bwd_splits(const sa2_problem *prob) { return q_splits(prob, 2, false); }
 
 int64_t sa2_fwd_workspace_bytes(const sa2_problem *prob) {
     if (check_problem(prob) != SA2_OK) return -1;
-    const int splits = q_splits(prob, kFwdMergeCost);
+    const int splits = fwd_splits(prob);
     return splits > 1 ? q_parts_bytes(prob, splits) + 8ll * splits * prob->batch * prob->heads * prob->seq_len : 0;
 }
 
@@ -291,7 +305,7 @@ int sa2_fwd_ws(const sa2_problem *prob, const sa2_tensor *q, const sa2_tensor *k
         SA2_FOR_DIM_HEAD(prob->dim_head, hipLaunchKernelGGL(sa2::fwd_kernel<DH>, dim3(grid), dim3(512), 0, s, k));
         return after_launch("forward");
     }
-    k.q_splits = q_splits(prob, kFwdMergeCost);
+    k.q_splits = fwd_splits(prob);
     k.q_parts = static_cast<float *>(workspace);
     SA2_FOR_DIM_HEAD(prob->dim_head, hipLaunchKernelGGL((sa2::fwd_kernel<DH, true>), dim3(k.q_splits * grid), dim3(512), 0, s, k));
     SA2_TRY(after_launch("forward in splits"));
@@ -380,7 +394,7 @@ static int64_t max64(int64_t a, int64_t b) { return a > b ? a : b; }
 // unequal length at 8 sequences of 2048 rows).  The rule estimates the finish time of every part count in units of one
 // pair (a query tile and two offsets, 1.3 us at D = 64, 1.9 us at D = 128); a part costs kPartCost pairs on top of its share
 // (its K1/V1 rows, the first rows and operand tiles, 2 * 128 * D fp32 values written and read again).
-static constexpr int kPartCost = 8;
+static constexpr int kPartCost = 12;
 static constexpr int kMaxParts = 64;
 
 struct Kv8Plan {
@@ -399,11 +413,20 @@ static Kv8Plan kv8_plan(const sa2_problem *prob) {
     const int nslab = (prob->seq_len + 127) / 128, G = prob->heads / prob->kv_heads;
     const int64_t heads = (int64_t)prob->batch * prob->kv_heads;
     const int64_t budget = max64(kPartBytes, partial_rows_bytes(prob));
+    // slabs of equal length, as (pairs, how many): those at a sequence's ends differ from the others
+    struct Class {
+        int64_t pairs;
+        int count;
+    };
+    Class cls[24];
+    int ncls = 0;
     int64_t longest = 0, total = 0;
     for (int t = 0; t < nslab; ++t) {
         const int64_t n = (int64_t)sa2::kv8_walk_pairs(t, prob->seq_len, prob->w1, prob->w2) * G;
         longest = n > longest ? n : longest;
         total += n;
+        if (ncls && (cls[ncls - 1].pairs == n || ncls == 24)) ++cls[ncls - 1].count;
+        else cls[ncls++] = {n, 1};
     }
     total *= heads;
     Kv8Plan best = {0, 1};
@@ -411,10 +434,13 @@ static Kv8Plan kv8_plan(const sa2_problem *prob) {
     for (int parts = 1; parts <= kMaxParts && parts <= longest && (parts == 1 || parts * kv_part_bytes(prob) <= budget); ++parts) {
         const int64_t chunk = (longest + parts - 1) / parts;
         const double extra = parts > 1 ? kPartCost : 0;
-        const double groups = parts == 1 ? (double)heads * nslab : (double)total / chunk;      // of about equal length
-        const double cost = finish_time(groups, chunk + extra, (double)total + extra * groups);
-        // (a second launch has to pay for itself)
-        if (parts == 1 || cost < 0.98 * best_cost) {
+        double groups = 0;
+        for (int x = 0; x < ncls; ++x) groups += (double)cls[x].count * sa2::kv8_parts_of(cls[x].pairs, (int)chunk, parts);
+        groups *= heads;
+        // (the combine kernel: a launch, and the partial rows read at 5.8 TB/s; a pair is worth 1.3 us of it)
+        const double merge = parts > 1 ? 2 + (double)(parts * kv_part_bytes(prob)) / 7.5e6 : 0;
+        const double cost = finish_time(groups, chunk + extra, (double)total + extra * groups) + merge;
+        if (parts == 1 || cost < 0.995 * best_cost) {
             best = {(int)chunk, parts};
             best_cost = cost;
         }
@@ -458,7 +484,7 @@ int64_t sa2_bwd_split_workspace_bytes(const sa2_problem *prob, int with_saved) {
     if (check_problem(prob) != SA2_OK) return -1;
     const Kv8Plan plan = kv8_plan(prob);
     const int64_t parts = plan.parts > 1 ? plan.parts * kv_part_bytes(prob) : 0;
-    return max64(q_workspace_bytes(prob, q_splits(prob, kBwdMergeCost), with_saved != 0), parts);
+    return max64(q_workspace_bytes(prob, bwd_splits(prob), with_saved != 0), parts);
 }
 
 // The launches behind sa2_bwd_dq_dkv2: the MFMA kernel(s) on stream `s`; the kernel that streams the forward's saved
@@ -485,7 +511,7 @@ static int prepare_dq_dkv2(const sa2_problem *prob, const sa2_tensor *q, const s
     // the dK2 partial rows are the first half of the workspace, the dV2 partial rows the second: with saved
     // forward partials dV2 needs none
     const bool saved_given = saved != nullptr;
-    const int splits = may_split ? q_splits(prob, kBwdMergeCost) : 1;
+    const int splits = may_split ? bwd_splits(prob) : 1;
     const int64_t need = q_workspace_bytes(prob, splits, saved_given);
     if (workspace_bytes < need)
         return fail(SA2_ERR_BAD_SHAPE, "workspace of %lld bytes is smaller than the %lld bytes this call needs (sa2_bwd_%sworkspace_bytes%s())",
@@ -533,7 +559,14 @@ static int launch_q_mfma(const sa2_problem *prob, const QLaunch &L, int pass, hi
 
 static int launch_dv2_from_saved(const sa2_problem *prob, const QLaunch &L, hipStream_t s) {
     const int dgrid = prob->batch * prob->kv_heads * ((prob->seq_len + 31) / 32);
-    SA2_FOR_DIM_HEAD(prob->dim_head, hipLaunchKernelGGL(sa2::dv2_from_saved_kernel<DH>, dim3(dgrid), dim3(sa2::Dv2Cfg<DH>::THREADS), 0, s, L.k));
+    // up to two workgroups per CU the chain of loads of one workgroup is what the kernel takes: split it inside the workgroup
+    const bool grouped = prob->dim_head < 128 && dgrid <= 2 * kComputeUnits;
+    if (grouped && prob->dim_head == 64)
+        hipLaunchKernelGGL((sa2::dv2_from_saved_kernel<64, true>), dim3(dgrid), dim3((sa2::Dv2Cfg<64, true>::THREADS)), 0, s, L.k);
+    else if (grouped)
+        hipLaunchKernelGGL((sa2::dv2_from_saved_kernel<32, true>), dim3(dgrid), dim3((sa2::Dv2Cfg<32, true>::THREADS)), 0, s, L.k);
+    else
+        SA2_FOR_DIM_HEAD(prob->dim_head, hipLaunchKernelGGL((sa2::dv2_from_saved_kernel<DH, false>), dim3(dgrid), dim3((sa2::Dv2Cfg<DH, false>::THREADS)), 0, s, L.k));
     return after_launch("dv2 from saved partials");
 }
 
@@ -582,27 +615,25 @@ static int launch_dkv1(const sa2_problem *prob, const sa2_tensor *q, const sa2_t
     }
     const int grid = prob->batch * prob->kv_heads * ((prob->seq_len + 127) / 128);
     // dim_head 128: the two waves of a slab split the contractions; dim_head 64 and 32: each wave forms both outputs
-    if (plan.parts > 1) {
-        if (prob->dim_head == 128)
-            hipLaunchKernelGGL((sa2::bwd_kv8_kernel<128, sa2::kKvSplit, true>), dim3(plan.parts * grid), dim3(512), 0, s, k);
-        else if (prob->dim_head == 64)
-            hipLaunchKernelGGL((sa2::bwd_kv8_kernel<64, sa2::kKvBoth, true>), dim3(plan.parts * grid), dim3(512), 0, s, k);
-        else
-            hipLaunchKernelGGL((sa2::bwd_kv8_kernel<32, sa2::kKvBoth, true>), dim3(plan.parts * grid), dim3(512), 0, s, k);
-        SA2_TRY(after_launch("dk1/dv1 in parts"));
-        const int64_t rows = (int64_t)prob->batch * prob->kv_heads * prob->seq_len;
-        const int rows_per_block = 256 / (prob->dim_head / 8);
-        const int cgrid = (int)((rows + rows_per_block - 1) / rows_per_block);
-        SA2_FOR_DIM_HEAD(prob->dim_head, hipLaunchKernelGGL(sa2::dkv1_parts_combine_kernel<DH>, dim3(cgrid, 2), dim3(256), 0, s, k));
-        return after_launch("dk1/dv1 parts combine");
+    const bool in_parts = plan.parts > 1;
+    const dim3 kgrid(in_parts ? plan.parts * grid : grid), block(512);
+    if (prob->dim_head == 128) {
+        if (in_parts) hipLaunchKernelGGL((sa2::bwd_kv8_kernel<128, sa2::kKvSplit, true>), kgrid, block, 0, s, k);
+        else hipLaunchKernelGGL((sa2::bwd_kv8_kernel<128, sa2::kKvSplit>), kgrid, block, 0, s, k);
+    } else if (prob->dim_head == 64) {
+        if (in_parts) hipLaunchKernelGGL((sa2::bwd_kv8_kernel<64, sa2::kKvBoth, true>), kgrid, block, 0, s, k);
+        else hipLaunchKernelGGL((sa2::bwd_kv8_kernel<64, sa2::kKvBoth>), kgrid, block, 0, s, k);
+    } else {
+        if (in_parts) hipLaunchKernelGGL((sa2::bwd_kv8_kernel<32, sa2::kKvBoth, true>), kgrid, block, 0, s, k);
+        else hipLaunchKernelGGL((sa2::bwd_kv8_kernel<32, sa2::kKvBoth>), kgrid, block, 0, s, k);
     }
-    if (prob->dim_head == 128)
-        hipLaunchKernelGGL((sa2::bwd_kv8_kernel<128, sa2::kKvSplit>), dim3(grid), dim3(512), 0, s, k);
-    else if (prob->dim_head == 64)
-        hipLaunchKernelGGL((sa2::bwd_kv8_kernel<64, sa2::kKvBoth>), dim3(grid), dim3(512), 0, s, k);
-    else
-        hipLaunchKernelGGL((sa2::bwd_kv8_kernel<32, sa2::kKvBoth>), dim3(grid), dim3(512), 0, s, k);
-    return after_launch("dk1/dv1");
+    SA2_TRY(after_launch("dk1/dv1"));
+    if (!in_parts) return SA2_OK;
+    const int64_t rows = (int64_t)prob->batch * prob->kv_heads * prob->seq_len;
+    const int rows_per_block = 256 / (prob->dim_head / 8);
+    const int cgrid = (int)((rows + rows_per_block - 1) / rows_per_block);
+    SA2_FOR_DIM_HEAD(prob->dim_head, hipLaunchKernelGGL(sa2::dkv1_parts_combine_kernel<DH>, dim3(cgrid, 2), dim3(256), 0, s, k));
+    return after_launch("dk1/dv1 parts combine");
 }
 
 int sa2_bwd_dkv1(const sa2_problem *prob, const sa2_tensor *q, const sa2_tensor *k1, const sa2_tensor *k2,
@@ -631,7 +662,13 @@ static int bwd_all(bool split, const sa2_problem *prob, const sa2_tensor *q, con
     QLaunch L;
     SA2_TRY(prepare_dq_dkv2(prob, q, k1, k2, v1, v2, dout, lse, delta_ws, saved, dq, dk2, dv2, workspace, workspace_bytes, split, &L));
     hipStream_t s = static_cast<hipStream_t>(hip_stream);
-    SA2_TRY(sa2_bwd_delta(prob, out, out_residual, dout, delta_ws, hip_stream));
+    if (L.k.q_splits <= 1) {
+        SA2_TRY(sa2_bwd_delta(prob, out, out_residual, dout, delta_ws, hip_stream));
+    } else {
+        // a split dQ/dK2 kernel forms delta itself and leaves it in delta_ws
+        L.k.o = dev(out);
+        if (out_residual) L.k.o_lo = dev(out_residual);
+    }
     SA2_TRY(launch_q_mfma(prob, L, 0, s));
     if (L.use_saved) SA2_TRY(launch_dv2_from_saved(prob, L, s));
     SA2_TRY(launch_q_combine(prob, L, s));

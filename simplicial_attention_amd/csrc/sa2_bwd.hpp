@@ -21,7 +21,7 @@
 namespace sa2 {
 
 // ------------------------------------------------------------------------------------
-// delta[b,h,i] = sum_d (out + out_residual) * dout
+// delta[b,h,i] = sum_d (out + out_residual) * dout  (a split dQ/dK2 kernel forms it itself)
 // ------------------------------------------------------------------------------------
 template <int D>
 __global__ __launch_bounds__(256) void delta_kernel(KParams p) {
@@ -35,18 +35,11 @@ __global__ __launch_bounds__(256) void delta_kernel(KParams p) {
         const int i = (int)(row % p.N);
         const int h = (int)((row / p.N) % p.H);
         const int b = (int)(row / ((int64_t)p.N * p.H));
-        u32x4 o = ld_global16(p.o.ptr + b * p.o.sb + (int64_t)i * p.o.sn + h * p.o.sh + piece * 16);
-        u32x4 g = ld_global16(p.dout.ptr + b * p.dout.sb + (int64_t)i * p.dout.sn + h * p.dout.sh + piece * 16);
-#pragma unroll
-        for (int w = 0; w < 4; ++w) s += bf16_lo(o[w]) * bf16_lo(g[w]) + bf16_hi(o[w]) * bf16_hi(g[w]);
-        if (p.o_lo.ptr) {
-            u32x4 r = ld_global16(p.o_lo.ptr + b * p.o_lo.sb + (int64_t)i * p.o_lo.sn + h * p.o_lo.sh + piece * 16);
-#pragma unroll
-            for (int w = 0; w < 4; ++w) s += bf16_lo(r[w]) * bf16_lo(g[w]) + bf16_hi(r[w]) * bf16_hi(g[w]);
-        }
+        const u32x4 o = ld_global16(p.o.ptr + b * p.o.sb + (int64_t)i * p.o.sn + h * p.o.sh + piece * 16);
+        const u32x4 g = ld_global16(p.dout.ptr + b * p.dout.sb + (int64_t)i * p.dout.sn + h * p.dout.sh + piece * 16);
+        s = delta_piece(o, g, p.o_lo.ptr ? p.o_lo.ptr + b * p.o_lo.sb + (int64_t)i * p.o_lo.sn + h * p.o_lo.sh + piece * 16 : nullptr);
     }
-#pragma unroll
-    for (int off = LP / 2; off >= 1; off >>= 1) s += __shfl_xor(s, off, 64);
+    s = delta_row_sum<LP>(s);
     if (ok && piece == 0) p.delta[row] = s;
 }
 

@@ -101,8 +101,11 @@ __global__ __launch_bounds__(512) void bwd_q_kernel(KParams p, float *ws, int ha
     const char *k2g = p.k2.ptr + b * p.k2.sb + hk * p.k2.sh;
     const char *v2g = p.v2.ptr + b * p.v2.sb + hk * p.v2.sh;
     const float lse2 = p.lse[((int64_t)b * p.H + h) * N + ic] * kLog2e;
+    // delta of the tile's rows: read, or, in a split grid that is given the out rows, formed here and left for the dK1/dV1
+    // kernel (small grids only: there a launch less counts, while the kernel of its own is 1/2 % of a large backward)
+    __shared__ float delta_s[SPLIT ? 32 : 1];
     float dl = 0.f;
-    if constexpr (DQ) dl = p.delta[((int64_t)b * p.H + h) * N + ic];
+    if constexpr (DQ && !SPLIT) dl = p.delta[((int64_t)b * p.H + h) * N + ic];
 
     // tiles of the first window, walked in order t_lo .. t_hi; masked: the tiles below mid_lo and the diagonal one
     const int t_lo = (i0 - p.w1 + 1 > 0 ? i0 - p.w1 + 1 : 0) / 32;
@@ -164,7 +167,21 @@ __global__ __launch_bounds__(512) void bwd_q_kernel(KParams p, float *ws, int ha
             float4 *qdst = reinterpret_cast<float4 *>(lds + C::QS + row * C::QPITCH + col * 2);
             qdst[0] = make_float4(bf16_lo(fq[0]) * c2, bf16_hi(fq[0]) * c2, bf16_lo(fq[1]) * c2, bf16_hi(fq[1]) * c2);
             qdst[1] = make_float4(bf16_lo(fq[2]) * c2, bf16_hi(fq[2]) * c2, bf16_lo(fq[3]) * c2, bf16_hi(fq[3]) * c2);
-            *reinterpret_cast<u32x4 *>(lds + C::DOS + row * PITCH + col) = ld_global16(dog + (int64_t)ii * p.dout.sn + col);
+            const u32x4 fd = ld_global16(dog + (int64_t)ii * p.dout.sn + col);
+            *reinterpret_cast<u32x4 *>(lds + C::DOS + row * PITCH + col) = fd;
+            if constexpr (DQ && SPLIT) {
+                if (p.o.ptr) {
+                    const u32x4 fo = ld_global16(p.o.ptr + b * p.o.sb + (int64_t)ii * p.o.sn + h * p.o.sh + col);
+                    const float part = delta_piece(fo, fd, p.o_lo.ptr ? p.o_lo.ptr + b * p.o_lo.sb + (int64_t)ii * p.o_lo.sn + h * p.o_lo.sh + col : nullptr);
+                    const float dsum = delta_row_sum<PPR>(part);
+                    if (col == 0) {
+                        delta_s[row] = dsum;
+                        if (split == 0 && i0 + row < N) p.delta[((int64_t)b * p.H + h) * N + i0 + row] = dsum;
+                    }
+                } else if (col == 0) {
+                    delta_s[row] = p.delta[((int64_t)b * p.H + h) * N + ii];
+                }
+            }
         }
         for (int x = tid; x < 39 * PPR; x += 512) {
             const int row = x / PPR, col = (x % PPR) * 16;
@@ -229,12 +246,13 @@ __global__ __launch_bounds__(512) void bwd_q_kernel(KParams p, float *ws, int ha
         issue_loads();
     };
 
-    const f32x16 neg_delta = splat16(-dl);      // DQ: -delta_i in every element (one query row per lane column)
     f32x16 acc[DT];            // G^T (DQ) or T^T (DV) of the running offset
     u32x4 A[KS];
     u32x4 Bv[DQ ? KS : 1];
 
     __syncthreads();
+    if constexpr (DQ && SPLIT) dl = delta_s[c];
+    const f32x16 neg_delta = splat16(-dl);      // DQ: -delta_i in every element (one query row per lane column)
     for (int r = r_first; r < R; ++r) {
         const int dlt = 8 * r + wave;
         const int kr = i - dlt;
@@ -440,26 +458,32 @@ __global__ __launch_bounds__(512) void bwd_q_kernel(KParams p, float *ws, int ha
 // (h = hk*G + g).  Streams T once from HBM.  A workgroup owns 32 rows k, a thread 8 d of one row; consecutive
 // threads own consecutive rows, whose pieces are consecutive in the blocked layout of T (saved_t_offset).  The do
 // rows k0 .. k0 + 62 that 32 offsets reach and the 32 x 32 weights are staged in LDS per block of 32 offsets.
-template <int D>
+// GROUPS: at D = 32 and 64 the threads of a workgroup form OG groups that take every OG-th offset and meet through LDS.  The
+// loop over the offsets is a chain of loads, which few workgroups do not hide (launch_dv2_from_saved has the rule); a large grid does
+// and loses by the larger workgroups (152 us instead of 130 at 8 x 8 x 2048 rows of 64).
+template <int D, bool GROUPS>
 struct Dv2Cfg {
     static constexpr int LP = D / 8;                 // 16-byte pieces per row
-    static constexpr int THREADS = 32 * LP;
+    static constexpr int OG = GROUPS ? 16 / LP : 1;  // offset groups
+    static constexpr int THREADS = 32 * LP * OG;
     static constexpr int PITCH = tile_pitch<D>();
 };
 
-template <int D>
-__global__ __launch_bounds__(Dv2Cfg<D>::THREADS) void dv2_from_saved_kernel(KParams p) {
-    using C = Dv2Cfg<D>;
-    constexpr int LP = C::LP, NTH = C::THREADS, PITCH = C::PITCH;
+template <int D, bool GROUPS>
+__global__ __launch_bounds__((Dv2Cfg<D, GROUPS>::THREADS)) void dv2_from_saved_kernel(KParams p) {
+    using C = Dv2Cfg<D, GROUPS>;
+    constexpr int LP = C::LP, NTH = C::THREADS, PITCH = C::PITCH, OG = C::OG;
     __shared__ __attribute__((aligned(16))) char dos[63 * PITCH];
     __shared__ float wsh[32 * 32];
+    __shared__ float4 red[OG > 1 ? (OG - 1) * 32 * LP * 2 : 1];
     const int N = p.N;
     const int ntile = (N + 31) / 32;
     const int kt = blockIdx.x % ntile;
     const int bh = blockIdx.x / ntile;
     const int hk = bh % p.HK, b = bh / p.HK;
     const int tid = threadIdx.x;
-    const int c = tid & 31, piece = tid >> 5;         // d = 8 piece .. 8 piece + 7
+    const int og = GROUPS ? tid / (32 * LP) : 0, t_in = GROUPS ? tid % (32 * LP) : tid;
+    const int c = t_in & 31, piece = t_in >> 5;       // d = 8 piece .. 8 piece + 7
     const int k0 = 32 * kt, k = k0 + c;
     const int t_piece = saved_t_offset(0, (piece >> 1) & 1, piece >> 2, piece & 1);
     float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
@@ -486,7 +510,7 @@ __global__ __launch_bounds__(Dv2Cfg<D>::THREADS) void dv2_from_saved_kernel(KPar
             __syncthreads();
             const int nl = nd - d0 < 32 ? nd - d0 : 32;
 #pragma unroll 8
-            for (int dl = 0; dl < nl; ++dl) {
+            for (int dl = og; dl < nl; dl += OG) {
                 // (rows past the end have weight 0; their T is read from the last row, which every offset has written)
                 const int i = k + d0 + dl < N ? k + d0 + dl : N - 1;
                 const int64_t sbh = bh_row * p.w2 + d0 + dl;
@@ -499,6 +523,27 @@ __global__ __launch_bounds__(Dv2Cfg<D>::THREADS) void dv2_from_saved_kernel(KPar
                     acc[2 * x + 1] += bf16_hi(o[x]) * bf16_hi(t[x]) * w;
                 }
             }
+        }
+    }
+    if constexpr (OG > 1) {
+        if (og > 0) {
+            float4 *dst = red + ((og - 1) * 32 * LP + t_in) * 2;
+            dst[0] = make_float4(acc[0], acc[1], acc[2], acc[3]);
+            dst[1] = make_float4(acc[4], acc[5], acc[6], acc[7]);
+        }
+        __syncthreads();
+        if (og > 0) return;
+#pragma unroll
+        for (int x = 0; x < OG - 1; ++x) {
+            const float4 a = red[(x * 32 * LP + t_in) * 2], e = red[(x * 32 * LP + t_in) * 2 + 1];
+            acc[0] += a.x;
+            acc[1] += a.y;
+            acc[2] += a.z;
+            acc[3] += a.w;
+            acc[4] += e.x;
+            acc[5] += e.y;
+            acc[6] += e.z;
+            acc[7] += e.w;
         }
     }
     if (k >= N) return;
@@ -553,10 +598,13 @@ __global__ __launch_bounds__(256) void dk2_dv2_combine_kernel(KParams p, const f
         for (int m = 0; tile + m < ntile && kl + halo - 32 * m >= 0; ++m) {
             const float *src = base + ((int64_t)(tile + m) * srows + (kl + halo - 32 * m)) * D + piece * 8;
             if (p.q_splits > 1) {
+                // the shares whose rounds r0 .. r1 - 1 reach the row: 1 - 8 r1 <= rel <= 31 - 8 r0
                 const int rounds = fwd_rounds(tile + m, p.w2), rel = kl - 32 * m;
-                for (int s = 0; s < p.q_splits; ++s) {
+                const int r_lo = rel >= 0 ? 0 : (-rel) / 8, r_hi = (31 - rel) / 8;        // rounds that reach it
+                for (int s = fwd_split_of(r_lo, p.q_splits, rounds); s < p.q_splits; ++s) {
                     const int r0 = fwd_split_round(s, p.q_splits, rounds), r1 = fwd_split_round(s + 1, p.q_splits, rounds);
-                    if (r0 >= r1 || rel > 31 - 8 * r0 || rel < 1 - 8 * r1) continue;
+                    if (r0 >= r1 || r0 > r_hi) break;
+                    if (rel < 1 - 8 * r1) continue;
                     const float *ss = src + s * p.q_ws_stride;
 #pragma unroll
                     for (int x = 0; x < 8; ++x) {

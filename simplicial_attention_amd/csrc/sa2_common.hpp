@@ -106,12 +106,38 @@ __device__ __forceinline__ float add_bf16x2(uint32_t x, float c) {
     return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, x), __builtin_bit_cast(bf16x2_t, 0x3f803f80u), c, false);
 }
 
+// a 16-byte piece's share of delta = sum_d (o + residual) * dO  (`residual` NULL: none)
+__device__ __forceinline__ float delta_piece(u32x4 o, u32x4 g, const char *residual) {
+    float s = 0.f;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) s += bf16_lo(o[w]) * bf16_lo(g[w]) + bf16_hi(o[w]) * bf16_hi(g[w]);
+    if (residual) {
+        const u32x4 r = ld_global16(residual);
+#pragma unroll
+        for (int w = 0; w < 4; ++w) s += bf16_lo(r[w]) * bf16_lo(g[w]) + bf16_hi(r[w]) * bf16_hi(g[w]);
+    }
+    return s;
+}
+// the sum over the LP consecutive lanes that hold a row
+template <int LP>
+__device__ __forceinline__ float delta_row_sum(float s) {
+#pragma unroll
+    for (int off = LP / 2; off >= 1; off >>= 1) s += __shfl_xor(s, off, 64);
+    return s;
+}
+
 // wave index as a scalar: branches on it are uniform and index arithmetic stays on the scalar unit
 __device__ __forceinline__ int wave_index() { return __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); }
 
 // a value that is the same in every lane, on the scalar unit (an integer division leaves its result in a vector register,
 // and what is computed from it follows)
 __device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
+
+__device__ __forceinline__ const char *uniform(const char *p) {
+    const uint64_t x = reinterpret_cast<uint64_t>(p);
+    const uint32_t lo = (uint32_t)uniform((int)(uint32_t)x), hi = (uint32_t)uniform((int)(uint32_t)(x >> 32));
+    return reinterpret_cast<const char *>(((uint64_t)hi << 32) | lo);
+}
 
 __device__ __forceinline__ f32x16 mfma32(u32x4 a, u32x4 b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(a), as_bf16x8(b), c, 0, 0, 0);

@@ -87,6 +87,11 @@ __host__ __device__ inline int fwd_split_round(int s, int splits, int rounds) {
     return splits < rounds ? rounds * s / splits : (s < rounds ? s : rounds);
 }
 
+// a split at or before the one that walks round r
+__host__ __device__ inline int fwd_split_of(int r, int splits, int rounds) {
+    return splits < rounds ? r * splits / rounds : r;
+}
+
 // SPLIT: several workgroups per query tile (p.q_splits of them in the grid), each walks a share of the tile's rounds and
 // leaves its fp32 output rows, their reference and their row sums in p.q_parts, which fwd_combine_kernel merges.  For grids
 // too small to give every CU a workgroup (q_plan in sa2_api.hip has the rule).
