@@ -109,7 +109,7 @@ def cpu_baseline(N, D, w1, w2, slices, runs=3, naive_runs=5):
 
 
 # the sources that the kernels of head dimensions 32, 64 and 128 are built from (the kernels whose HBM traffic is stored)
-MEASURED_KERNEL_SOURCES = ('sa2_common.hpp', 'sa2_lds.hpp', 'sa2_fwd.hpp', 'sa2_bwd.hpp', 'sa2_bwd_q.hpp', 'sa2_bwd_kv8.hpp')
+MEASURED_KERNEL_SOURCES = ('sa2_common.hpp', 'sa2_lds.hpp', 'sa2_acc.hpp', 'sa2_fwd.hpp', 'sa2_fwd2.hpp', 'sa2_bwd.hpp', 'sa2_bwd_q.hpp', 'sa2_bwd_kv8.hpp')
 
 
 def source_digest():
@@ -132,7 +132,7 @@ def kernel_symbol(entry, D, w2):
     if D == 256:
         return {'fwd': 'sa2::fwd_wide_kernel<256>', 'bwd_dq_dk2_pass': 'sa2::bwd_wide_q_kernel<256>', 'bwd_dkv1': 'sa2::bwd_wide_kv_kernel<256>'}.get(entry)
     if entry == 'fwd':
-        return 'sa2::fwd_kernel<%d>' % D
+        return 'sa2::fwd2_kernel<128>' if D == 128 else 'sa2::fwd_kernel<%d>' % D
     if entry == 'bwd_dq_dk2_pass':
         return 'sa2::bwd_q_kernel<%d, true>' % D
     if entry == 'bwd_dkv1':
@@ -170,7 +170,7 @@ def traffic_from(directory):
         for f in glob.glob(os.path.join(directory, sub, '**', '*counter_collection.csv'), recursive=True):
             for row in csv.DictReader(open(f)):
                 name = row.get('Kernel_Name', '')
-                if kernel_part == 'fwd' and 'fwd_kernel' not in name:
+                if kernel_part == 'fwd' and 'fwd_kernel' not in name and 'fwd2_kernel' not in name:
                     continue
                 if row.get('Counter_Name') == counter and kernel_part in name:
                     vals.append(float(row['Counter_Value']))

@@ -66,7 +66,7 @@ _lock = threading.Lock()
 def build(verbose: bool = False) -> str:
     """Compile libsa2.so for gfx950 (always recompiles)."""
     out = None if verbose else subprocess.DEVNULL
-    subprocess.check_call(['make', '-B', '-C', _CSRC, 'libsa2.so', 'libsa2_prof.so', '_sa2_torch.so'], stdout=out, stderr=out)
+    subprocess.check_call(['make', '-B', '-j4', '-C', _CSRC, 'libsa2.so', 'libsa2_prof.so', '_sa2_torch.so'], stdout=out, stderr=out)
     return LIB_PATH
 
 

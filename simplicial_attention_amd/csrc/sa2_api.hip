@@ -18,6 +18,7 @@
 #include "sa2_lds.hpp"
 #include "sa2_qkv_norm.hpp"
 #include "sa2_fwd.hpp"
+#include "sa2_launch.hpp"
 #include "sa2_wide.hpp"
 #ifdef SA2_PROFILING
 #include "sa2_prof_mix.hpp"
@@ -260,6 +261,19 @@ static int q_splits(const sa2_problem *prob, int merge_cost, bool shared) {
 static int fwd_splits(const sa2_problem *prob) { return q_splits(prob, 8, prob->dim_head != 128); }   // (the merge is a launch of its own)
 static int bwd_splits(const sa2_problem *prob) { return q_splits(prob, 2, false); }
 
+// dim_head 128: one wave per SIMD with two offsets each; 64 and 32: two workgroups of eight waves per CU
+static void launch_fwd(int dim_head, bool split, int grid, hipStream_t s, const sa2::KParams &k) {
+    if (dim_head == 128) {
+        sa2::launch_fwd2(split, grid, s, k);
+    } else if (dim_head == 64) {
+        if (split) hipLaunchKernelGGL((sa2::fwd_kernel<64, true>), dim3(grid), dim3(512), 0, s, k);
+        else hipLaunchKernelGGL((sa2::fwd_kernel<64>), dim3(grid), dim3(512), 0, s, k);
+    } else {
+        if (split) hipLaunchKernelGGL((sa2::fwd_kernel<32, true>), dim3(grid), dim3(512), 0, s, k);
+        else hipLaunchKernelGGL((sa2::fwd_kernel<32>), dim3(grid), dim3(512), 0, s, k);
+    }
+}
+
 int64_t sa2_fwd_workspace_bytes(const sa2_problem *prob) {
     if (check_problem(prob) != SA2_OK) return -1;
     const int splits = fwd_splits(prob);
@@ -302,12 +316,12 @@ int sa2_fwd_ws(const sa2_problem *prob, const sa2_tensor *q, const sa2_tensor *k
     }
     const int64_t need = workspace ? sa2_fwd_workspace_bytes(prob) : 0;
     if (need == 0 || workspace_bytes < need) {
-        SA2_FOR_DIM_HEAD(prob->dim_head, hipLaunchKernelGGL(sa2::fwd_kernel<DH>, dim3(grid), dim3(512), 0, s, k));
+        launch_fwd(prob->dim_head, false, grid, s, k);
         return after_launch("forward");
     }
     k.q_splits = fwd_splits(prob);
     k.q_parts = static_cast<float *>(workspace);
-    SA2_FOR_DIM_HEAD(prob->dim_head, hipLaunchKernelGGL((sa2::fwd_kernel<DH, true>), dim3(k.q_splits * grid), dim3(512), 0, s, k));
+    launch_fwd(prob->dim_head, true, k.q_splits * grid, s, k);
     SA2_TRY(after_launch("forward in splits"));
     const int64_t rows = (int64_t)prob->batch * prob->heads * prob->seq_len;
     const int rows_per_block = 256 / (prob->dim_head / 8);

@@ -1,4 +1,4 @@
-// Forward kernel (eight waves, two per SIMD).
+// Forward kernel for head dimensions 32 and 64 (eight waves per workgroup, two workgroups per CU; fwd2_kernel is the one for 128).
 //
 // One workgroup owns 32 query rows of one (batch, head).  In round r wave w handles the
 // offset dlt = i - k = 8r + w (any second window: ceil(w2 / 8) rounds); all eight waves walk
@@ -56,13 +56,12 @@ struct FwdCfg {
     // q rows of the tile [32][QPITCH bytes]: fp32 times scale log2(e); at D = 64 bf16 (the instance then fits 80 KiB of
     // LDS and 128 registers: two workgroups per CU)
     static constexpr bool QF = D != 64;
-    // waves per SIMD the instance is compiled for: D = 128 needs 236 registers (one workgroup per CU); D = 64 is held
-    // to 128 registers (a few spills outside the step's MFMA blocks) so that two workgroups share a CU, which is worth
-    // 20 % at D = 64; D = 32 fits by itself
-    static constexpr int WPE = D == 128 ? 2 : 4;
-    // fragments in flight per operand and chain: a rolling window of four of the eight at D = 128; two of the four at
-    // D = 64, where four waves per SIMD cover the latency and the registers are the scarcer resource
-    static constexpr int FW = D == 64 ? 2 : (KS < 4 ? KS : 4);
+    // waves per SIMD: D = 64 is held to 128 registers (a few spills outside the step's MFMA blocks) so that two workgroups
+    // share a CU, which is worth 20 % at D = 64; D = 32 fits by itself
+    static constexpr int WPE = 4;
+    // fragments in flight per operand and chain: two of the four at D = 64, where four waves per SIMD cover the latency
+    // and the registers are the scarcer resource; both at D = 32
+    static constexpr int FW = 2;
     static constexpr int QS = RING + ACC + 2 * EXCH;
     static constexpr int QPITCH = QF ? D * 4 + 16 : tile_pitch<D>();
     static constexpr int KSLOTS = 64;                 // circular k2 / v2 rows
@@ -71,7 +70,7 @@ struct FwdCfg {
     static constexpr int MASKS = V2S + KSLOTS * PITCH; // additive masks (0 / -inf) of the diagonal tile and of up to two lower-edge tiles
     static constexpr int MASK = 16 * 64 * 4;          // one table: [4 quarters][64 lanes][4 floats]
     static constexpr int LDS = MASKS + 3 * MASK;
-    static_assert(D == 128 || 2 * LDS <= 160 * 1024, "two workgroups per CU need half the LDS each");
+    static_assert(D <= 64 && 2 * LDS <= 160 * 1024, "two workgroups per CU need half the LDS each");
     static_assert(RING - CP < 65536, "the LDS address of a direct load travels in 16 bits of M0");
     static constexpr int PPR = D / 8;                 // 16-byte pieces per row
     static constexpr int PIECES = 32 * PPR;           // ... per tile
@@ -94,7 +93,7 @@ __host__ __device__ inline int fwd_split_of(int r, int splits, int rounds) {
 
 // SPLIT: several workgroups per query tile (p.q_splits of them in the grid), each walks a share of the tile's rounds and
 // leaves its fp32 output rows, their reference and their row sums in p.q_parts, which fwd_combine_kernel merges.  For grids
-// too small to give every CU a workgroup (q_plan in sa2_api.hip has the rule).
+// too small to give every CU a workgroup (q_splits in sa2_api.hip has the rule).
 template <int D, bool SPLIT = false>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(FwdCfg<D>::WPE, FwdCfg<D>::WPE))) void fwd_kernel(KParams p) {
     using C = FwdCfg<D>;
@@ -588,16 +587,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(FwdCfg<D>::
             o[x] = v.x * inv;
             o[x + 1] = v.y * inv;
         }
-        if constexpr (SEG == 8) {
-            u32x4 ov, rv;
-#pragma unroll
-            for (int w = 0; w < 4; ++w) {
-                ov[w] = pack_bf16(o[2 * w], o[2 * w + 1]);
-                rv[w] = pack_bf16(o[2 * w] - bf16_lo(ov[w]), o[2 * w + 1] - bf16_hi(ov[w]));
-            }
-            st_global16(orow, ov);
-            if (rrow) st_global16(rrow, rv);
-        } else if constexpr (SEG == 4) {
+        if constexpr (SEG == 4) {
             u32x2 ov, rv;
 #pragma unroll
             for (int w = 0; w < 2; ++w) {
@@ -607,7 +597,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(FwdCfg<D>::
             *reinterpret_cast<u32x2 *>(orow) = ov;
             if (rrow) *reinterpret_cast<u32x2 *>(rrow) = rv;
         } else {
-            static_assert(SEG == 2, "head dimension 32, 64 or 128");
+            static_assert(SEG == 2, "head dimension 32 or 64");
             const uint32_t ov = pack_bf16(o[0], o[1]);
             *reinterpret_cast<uint32_t *>(orow) = ov;
             if (rrow) *reinterpret_cast<uint32_t *>(rrow) = pack_bf16(o[0] - bf16_lo(ov), o[1] - bf16_hi(ov));
