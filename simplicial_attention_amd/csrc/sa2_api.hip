@@ -19,7 +19,6 @@
 #include "sa2_qkv_norm.hpp"
 #include "sa2_fwd.hpp"
 #include "sa2_launch.hpp"
-#include "sa2_wide.hpp"
 #ifdef SA2_PROFILING
 #include "sa2_prof_mix.hpp"
 #endif
@@ -311,7 +310,7 @@ int sa2_fwd_ws(const sa2_problem *prob, const sa2_tensor *q, const sa2_tensor *k
     const int grid = prob->batch * prob->heads * ((prob->seq_len + 31) / 32);
     if (prob->dim_head == kWideDimHead) {
         const int wgrid = prob->batch * prob->heads * ((prob->seq_len + 127) / 128);
-        hipLaunchKernelGGL(sa2::fwd_wide_kernel<kWideDimHead>, dim3(wgrid), dim3(256), 0, s, k);
+        sa2::launch_fwd_wide(wgrid, s, k);
         return after_launch("forward");
     }
     const int64_t need = workspace ? sa2_fwd_workspace_bytes(prob) : 0;
@@ -554,8 +553,8 @@ static int prepare_dq_dkv2(const sa2_problem *prob, const sa2_tensor *q, const s
 
 static int launch_q_mfma(const sa2_problem *prob, const QLaunch &L, int pass, hipStream_t s) {
     if (prob->dim_head == kWideDimHead) {
-        // one kernel forms dQ and both sets of partial rows
-        hipLaunchKernelGGL(sa2::bwd_wide_q_kernel<kWideDimHead>, dim3(L.grid), dim3(256), 0, s, L.k, L.ws, L.halo);
+        sa2::launch_bwd_wide_q(true, L.grid, s, L.k, L.ws, L.halo);
+        if (pass != 1) sa2::launch_bwd_wide_q(false, L.grid, s, L.k, L.ws, L.halo);
         return after_launch("dq/dk2/dv2");
     }
     if (L.k.q_splits > 1) {
@@ -624,7 +623,7 @@ static int launch_dkv1(const sa2_problem *prob, const sa2_tensor *q, const sa2_t
     hipStream_t s = static_cast<hipStream_t>(hip_stream);
     if (prob->dim_head == kWideDimHead) {
         const int wgrid = prob->batch * prob->kv_heads * ((prob->seq_len + 31) / 32);
-        hipLaunchKernelGGL(sa2::bwd_wide_kv_kernel<kWideDimHead>, dim3(wgrid), dim3(256), 0, s, k);
+        sa2::launch_bwd_wide_kv(wgrid, s, k);
         return after_launch("dk1/dv1");
     }
     const int grid = prob->batch * prob->kv_heads * ((prob->seq_len + 127) / 128);

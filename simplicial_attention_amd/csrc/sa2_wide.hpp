@@ -308,163 +308,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 }
 
 // ------------------------------------------------------------------------------------------------------------------
-// Workspace block of a tile: [32 + halo][D] fp32 rows per tensor, row x <-> k = i0 - halo + x (the layout that
-// dk2_dv2_combine_kernel reads: the dk2 rows carry q * scale * log2(e), the kernel multiplies by ln 2).
-template <int D>
-__global__ __launch_bounds__(256) void bwd_wide_q_kernel(KParams p, float *ws, int halo) {
-    using C = WideCfg<D>;
-    constexpr int DB = C::DB, KQ = C::KQ;
-    // operand tiles A, B; two buffers of K1 / V1 tiles; the exchange areas of the partial tiles; the packed weights
-    __shared__ __attribute__((aligned(16))) char lds[6 * C::TILE + 2 * C::XCH + 2 * 2048];
-    char *tA = lds, *tB = lds + C::TILE;
-    char *xs = lds + 6 * C::TILE, *xp = xs + C::XCH, *pexP = xp + C::XCH, *pexS = pexP + 2048;
-    int buf = 0;
-
-    const int N = p.N;
-    const int ntile = (N + 31) / 32;
-    const int item = xcd_contiguous(blockIdx.x, gridDim.x);
-    const int tile = ntile - 1 - item % ntile;
-    const int bh = item / ntile;
-    const int h = bh % p.H, b = bh / p.H;
-    const int hk = h / p.G;
-    const int tid = threadIdx.x;
-    const int wave = wave_index(), lane = tid & 63;
-    const int c = lane & 31, hf = lane >> 5;
-    const int i0 = tile * 32, i = i0 + c;
-    const bool row_ok = i < N;
-
-    const char *qg = p.q.ptr + b * p.q.sb + h * p.q.sh;
-    const char *dog = p.dout.ptr + b * p.dout.sb + h * p.dout.sh;
-    const char *k1g = p.k1.ptr + b * p.k1.sb + hk * p.k1.sh;
-    const char *v1g = p.v1.ptr + b * p.v1.sb + hk * p.v1.sh;
-    const char *k2g = p.k2.ptr + b * p.k2.sb + hk * p.k2.sh;
-    const char *v2g = p.v2.ptr + b * p.v2.sb + hk * p.v2.sh;
-    const SwzLane<D> sw(lane);
-
-    u32x4 qp[C::NP], dop[C::NP];
-    wide_pieces<D>(qp, qg, p.q.sn, i0, N, tid);
-    wide_pieces<D>(dop, dog, p.dout.sn, i0, N, tid);
-    const int64_t srow = ((int64_t)b * p.H + h) * N + (row_ok ? i : N - 1);
-    const float lse2 = p.lse[srow] * kLog2e, dl = p.delta[srow];
-
-    const int srows = 32 + halo;
-    const int64_t per_tensor = (int64_t)p.B * p.H * ntile * srows * D;
-    float *wk = ws + (((int64_t)b * p.H + h) * ntile + tile) * srows * D, *wv = wk + per_tensor;
-    for (int x = tid; x < srows * D / 4; x += 256) {
-        reinterpret_cast<float4 *>(wk)[x] = make_float4(0.f, 0.f, 0.f, 0.f);
-        reinterpret_cast<float4 *>(wv)[x] = make_float4(0.f, 0.f, 0.f, 0.f);
-    }
-
-    const int t_lo = (i0 - p.w1 + 1 > 0 ? i0 - p.w1 + 1 : 0) / 32, t_hi = i0 / 32;
-    const int nd = p.w2 < i0 + 32 ? p.w2 : i0 + 32;
-    const int col0 = wave * C::DQ + 16 * hf;              // first column of this lane's accumulator registers
-
-    f32x16 dQ[DB], G[DB], T[DB];
-#pragma unroll
-    for (int db = 0; db < DB; ++db) dQ[db] = zero16();
-
-    // fetched one step ahead: the k2 / v2 rows of the next offset, the K1 / V1 rows of the next tile
-    u32x4 nyk[C::NP], nyv[C::NP], nk[C::NP], nv[C::NP];
-    wide_pieces<D>(nyk, k2g, p.k2.sn, i0, N, tid);
-    wide_pieces<D>(nyv, v2g, p.v2.sn, i0, N, tid);
-    wide_pieces<D>(nk, k1g, p.k1.sn, 32 * t_lo, N, tid);
-    wide_pieces<D>(nv, v1g, p.v1.sn, 32 * t_lo, N, tid);
-
-    for (int dlt = 0; dlt < nd; ++dlt) {
-        __syncthreads();      // operand tiles free; the rows this offset adds to were written at least one barrier ago
-        wide_build<D>(tA, qp, nyk, p.scale_log2e, tid);
-        wide_build<D>(tB, dop, nyv, 1.f, tid);
-        wide_pieces<D>(nyk, k2g, p.k2.sn, i0 - dlt - 1, N, tid);
-        wide_pieces<D>(nyv, v2g, p.v2.sn, i0 - dlt - 1, N, tid);
-#pragma unroll
-        for (int db = 0; db < DB; ++db) G[db] = T[db] = zero16();
-        const bool col_ok = row_ok && i - dlt >= 0;
-        for (int t = t_lo; t <= t_hi; ++t) {
-            // (two tile buffers: a store meets no reader, every wave has passed three barriers since the buffer's last use)
-            char *tK = lds + 2 * C::TILE + buf * 2 * C::TILE, *tV = tK + C::TILE;
-            buf ^= 1;
-            wide_store<D>(tK, nk, tid);
-            wide_store<D>(tV, nv, tid);
-            {
-                const int tn = t < t_hi ? t + 1 : t_lo;
-                wide_pieces<D>(nk, k1g, p.k1.sn, 32 * tn, N, tid);
-                wide_pieces<D>(nv, v1g, p.v1.sn, 32 * tn, N, tid);
-            }
-            __syncthreads();
-            {
-                f32x16 X = zero16(), Y = zero16();
-#pragma unroll
-                for (int kq = 0; kq < KQ; ++kq) {
-                    X = mfma32(sw.row_frag(tK, wave * KQ + kq), sw.row_frag(tA, wave * KQ + kq), X);
-                    Y = mfma32(sw.row_frag(tV, wave * KQ + kq), sw.row_frag(tB, wave * KQ + kq), Y);
-                }
-                wide_put(xs, wave, lane, X);
-                wide_put(xp, wave, lane, Y);
-            }
-            __syncthreads();
-            {
-                // this wave's quarter of the tile: key rows j = 32 t + 8 wave + 4 hf + e
-                const float4 x4 = wide_sum_quarter(xs, wave, lane), y4 = wide_sum_quarter(xp, wave, lane);
-                const int rel = col_ok ? i - 32 * t - 4 * hf - 8 * wave : -(1 << 30);
-                const float xe[4] = {x4.x, x4.y, x4.z, x4.w}, ye[4] = {y4.x, y4.y, y4.z, y4.w};
-                float pr[4], ds[4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const bool ok = (unsigned)(rel - e) < (unsigned)p.w1;
-                    pr[e] = ok ? fast_exp2(xe[e] - lse2) : 0.f;
-                    ds[e] = pr[e] * (ye[e] - dl);
-                }
-                wide_put_packed(pexP, wave, lane, pr[0], pr[1], pr[2], pr[3]);
-                wide_put_packed(pexS, wave, lane, ds[0], ds[1], ds[2], ds[3]);
-            }
-            __syncthreads();
-            u32x4 pbP[2], pbS[2];
-            wide_get_packed(pbP, pexP, lane);
-            wide_get_packed(pbS, pexS, lane);
-#pragma unroll
-            for (int db = 0; db < DB; ++db)
-#pragma unroll
-                for (int k2s = 0; k2s < 2; ++k2s) {
-                    G[db] = mfma32(sw.tr_frag(tK, k2s, wave * DB + db), pbS[k2s], G[db]);
-                    T[db] = mfma32(sw.tr_frag(tV, k2s, wave * DB + db), pbP[k2s], T[db]);
-                }
-        }
-        // dq_i += k2_{i-dlt} * G;  row k = i - dlt of the tile's partial rows += (q_i scale log2e) * G and do_i * T
-        int kr = i - dlt;
-        kr = kr < 0 ? 0 : (kr < N ? kr : N - 1);
-        fma_row<DB>(dQ, G, k2g + (int64_t)kr * p.k2.sn + col0 * 2);
-        if (col_ok) {
-            float *rk = wk + (int64_t)(c - dlt + halo) * D + col0, *rv = wv + (int64_t)(c - dlt + halo) * D + col0;
-            const char *qrow = qg + (int64_t)i * p.q.sn + col0 * 2, *dorow = dog + (int64_t)i * p.dout.sn + col0 * 2;
-#pragma unroll
-            for (int db = 0; db < DB; ++db)
-#pragma unroll
-                for (int half = 0; half < 2; ++half) {
-                    const u32x4 xq = ld_global16(qrow + db * 64 + half * 16), xd = ld_global16(dorow + db * 64 + half * 16);
-#pragma unroll
-                    for (int e = 0; e < 2; ++e) {
-                        float4 *dk = reinterpret_cast<float4 *>(rk + 32 * db + 8 * half + 4 * e);
-                        float4 *dv = reinterpret_cast<float4 *>(rv + 32 * db + 8 * half + 4 * e);
-                        float4 a = *dk, bq = *dv;
-                        const int r0 = 8 * half + 4 * e;
-                        a.x += bf16_lo(xq[2 * e]) * p.scale_log2e * G[db][r0];
-                        a.y += bf16_hi(xq[2 * e]) * p.scale_log2e * G[db][r0 + 1];
-                        a.z += bf16_lo(xq[2 * e + 1]) * p.scale_log2e * G[db][r0 + 2];
-                        a.w += bf16_hi(xq[2 * e + 1]) * p.scale_log2e * G[db][r0 + 3];
-                        bq.x += bf16_lo(xd[2 * e]) * T[db][r0];
-                        bq.y += bf16_hi(xd[2 * e]) * T[db][r0 + 1];
-                        bq.z += bf16_lo(xd[2 * e + 1]) * T[db][r0 + 2];
-                        bq.w += bf16_hi(xd[2 * e + 1]) * T[db][r0 + 3];
-                        *dk = a;
-                        *dv = bq;
-                    }
-                }
-        }
-    }
-    if (row_ok) store_row<DB>(p.dq.ptr + b * p.dq.sb + (int64_t)i * p.dq.sn + h * p.dq.sh + col0 * 2, dQ, p.scale);
-}
-
-// ------------------------------------------------------------------------------------------------------------------
 template <int D>
 __global__ __launch_bounds__(256) void bwd_wide_kv_kernel(KParams p) {
     using C = WideCfg<D>;
