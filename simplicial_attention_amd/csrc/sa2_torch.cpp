@@ -173,27 +173,36 @@ struct Attend : public torch::autograd::Function<Attend> {
     static Tensor forward(AutogradContext *ctx, const Tensor &q, const Tensor &k1, const Tensor &k2, const Tensor &v1, const Tensor &v2,
                           const Geometry &g, bool save) {
         Forward f = run_forward(q, k1, k2, v1, v2, g, true, save);
-        ctx->save_for_backward({f.q, f.k1, f.k2, f.v1, f.v2, f.out, f.lse, f.residual, f.t_save, f.m_save});
-        c10::List<int64_t> n;
-        for (const int64_t v : {g.batch, g.seq, g.heads, g.kv_heads, g.dim_qk, g.dim_v, g.dim, g.w1, g.w2}) n.push_back(v);
-        for (const Tensor *t : {&q, &k1, &k2, &v1, &v2}) n.push_back((int64_t)t->scalar_type());
-        ctx->saved_data["geometry"] = n;
+        ctx->save_for_backward(saved_of(f));
+        ctx->saved_data["geometry"] = c10::List<int64_t>(sizes_of(g, {&q, &k1, &k2, &v1, &v2}));
         ctx->saved_data["scale"] = g.scale;
         return f.result;
     }
 
     static variable_list backward(AutogradContext *ctx, variable_list douts) {
-        const variable_list s = ctx->get_saved_variables();
+        variable_list grads = run_backward(ctx->get_saved_variables(), ctx->saved_data["geometry"].toIntVector(), ctx->saved_data["scale"].toDouble(), douts[0]);
+        grads.resize(7);
+        return grads;
+    }
+
+    // what the backward needs of a forward: tensors, and as numbers the geometry and the types of the inputs
+    static variable_list saved_of(const Forward &f) { return {f.q, f.k1, f.k2, f.v1, f.v2, f.out, f.lse, f.residual, f.t_save, f.m_save}; }
+    static std::vector<int64_t> sizes_of(const Geometry &g, const std::array<const Tensor *, 5> &inputs) {
+        std::vector<int64_t> n{g.batch, g.seq, g.heads, g.kv_heads, g.dim_qk, g.dim_v, g.dim, g.w1, g.w2};
+        for (const Tensor *t : inputs) n.push_back((int64_t)t->scalar_type());
+        return n;
+    }
+
+    static variable_list run_backward(const variable_list &s, const std::vector<int64_t> &n, double scale, const Tensor &given) {
         const Tensor &q = s[0], &k1 = s[1], &k2 = s[2], &v1 = s[3], &v2 = s[4], &out = s[5], &lse = s[6], &residual = s[7], &t_save = s[8], &m_save = s[9];
-        const c10::List<int64_t> n = ctx->saved_data["geometry"].toIntList();
         Geometry g;
         g.batch = n[0]; g.seq = n[1]; g.heads = n[2]; g.kv_heads = n[3]; g.dim_qk = n[4]; g.dim_v = n[5]; g.dim = n[6]; g.w1 = n[7]; g.w2 = n[8];
-        g.scale = ctx->saved_data["scale"].toDouble();
+        g.scale = scale;
         const c10::DeviceGuard guard(q.device());
         void *stream = stream_of(q);
         Conversions todo;
         std::vector<Tensor> alive;
-        const Tensor dout = as_rows(douts[0], g.dim, todo, alive);
+        const Tensor dout = as_rows(given, g.dim, todo, alive);
         todo.run(stream);
         const auto bf16 = q.options();
         const std::array<int64_t, 4> q_shape{g.batch, g.seq, g.heads, g.dim}, kv_shape{g.batch, g.seq, g.kv_heads, g.dim};
@@ -214,9 +223,9 @@ struct Attend : public torch::autograd::Function<Attend> {
                             reinterpret_cast<float *>(base), &ag[0], &ag[1], &ag[2], &ag[3], &ag[4], base + delta_bytes, ws_bytes, stream));
         // back to the types and head dimensions of the inputs
         Conversions back;
-        variable_list result(7);
+        variable_list result(5);
         for (int x = 0; x < 5; ++x) {
-            const auto type = (at::ScalarType)(int64_t)n[9 + x];
+            const auto type = (at::ScalarType)n[9 + x];
             const int64_t dim = x < 3 ? g.dim_qk : g.dim_v;
             if (type == at::kBFloat16 && dim == g.dim) {
                 result[x] = grads[x];
@@ -236,9 +245,7 @@ int64_t kernel_dim(int64_t dim) {
     return 0;
 }
 
-// `save`: called with the bytes of the partials, says whether they may be kept
-Tensor attend(const Tensor &q, const Tensor &k1, const Tensor &k2, const Tensor &v1, const Tensor &v2, int64_t w1, int64_t w2, double scale,
-              const py::object &admit) {
+Geometry geometry_of(const Tensor &q, const Tensor &k1, const Tensor &v1, int64_t w1, int64_t w2, double scale) {
     Geometry g;
     g.batch = q.size(0);
     g.seq = q.size(1);
@@ -250,19 +257,34 @@ Tensor attend(const Tensor &q, const Tensor &k1, const Tensor &k2, const Tensor 
     g.w1 = w1;
     g.w2 = w2;
     g.scale = scale;
-    const bool needs_grad = at::GradMode::is_enabled() && (q.requires_grad() || k1.requires_grad() || k2.requires_grad() || v1.requires_grad() || v2.requires_grad());
-    if (!needs_grad) return run_forward(q, k1, k2, v1, v2, g, false, false).result;
-    // per-offset value partials, kept for the backward when they fit the budget: dV2 then needs no recomputation of the
-    // attention weights (a size of 0: the kernels of this head dimension keep none)
+    return g;
+}
+
+// Per-offset value partials, kept for the backward when they fit the budget: dV2 then needs no recomputation of the
+// attention weights (a size of 0: the kernels of this head dimension keep none).  `admit`: called with their bytes, says
+// whether they may be kept
+bool keep_partials(const Geometry &g, const Tensor &q, const py::object &admit) {
     const sa2_problem prob = g.problem();
     const int64_t bytes = sa2_saved_t_bytes(&prob) + sa2_saved_m_bytes(&prob);
-    const bool save = bytes > 0 && admit(bytes, (int)q.device().index()).cast<bool>();
-    return Attend::apply(q, k1, k2, v1, v2, g, save);
+    return bytes > 0 && admit(bytes, (int)q.device().index()).cast<bool>();
+}
+
+// a call that autograd has to see: a backward may follow, or an input carries a forward-mode tangent (which the node refuses,
+// also without a graph: the derivative would be lost without a word)
+bool in_autograd(std::initializer_list<const Tensor *> inputs) {
+    for (const Tensor *t : inputs)
+        if ((at::GradMode::is_enabled() && t->requires_grad()) || t->_fw_grad(0).defined()) return true;
+    return false;
+}
+
+Tensor attend(const Tensor &q, const Tensor &k1, const Tensor &k2, const Tensor &v1, const Tensor &v2, const Geometry &g, const py::object &admit) {
+    if (!in_autograd({&q, &k1, &k2, &v1, &v2})) return run_forward(q, k1, k2, v1, v2, g, false, false).result;
+    return Attend::apply(q, k1, k2, v1, v2, g, keep_partials(g, q, admit));
 }
 
 // shapes, types and windows of the Function and the wrapper; `pads`: other head dimensions and types than the kernels' are welcome
-Tensor checked_attend(const Tensor &q, const Tensor &k1, const Tensor &k2, const Tensor &v1, const Tensor &v2, int64_t w1, int64_t w2,
-                      std::optional<double> scale, bool pads, const py::object &admit) {
+Geometry checked(const Tensor &q, const Tensor &k1, const Tensor &k2, const Tensor &v1, const Tensor &v2, int64_t w1, int64_t w2,
+                 std::optional<double> scale, bool pads) {
     const Tensor *all[5] = {&q, &k1, &k2, &v1, &v2};
     for (const Tensor *t : all)
         if (!t->is_cuda()) raise(PyExc_AssertionError, "sliding-window 2-simplicial attention runs on the GPU only");
@@ -281,8 +303,38 @@ Tensor checked_attend(const Tensor &q, const Tensor &k1, const Tensor &k2, const
     const int64_t dim = std::max(q.size(3), v1.size(3));
     if (pads ? dim > 256 || dim < 1 : !sa2_supported((int32_t)dim, 1, 1, SA2_BF16))
         raise(PyExc_NotImplementedError, "dim_head=" + std::to_string(dim) + " is not covered by the kernels (dim_head 32, 64, 128 or 256)");
-    return attend(q, k1, k2, v1, v2, std::min<int64_t>(w1, INT32_MAX), std::min<int64_t>(w2, INT32_MAX),
-                  scale ? *scale : 1.0 / std::sqrt((double)q.size(3)), admit);
+    return geometry_of(q, k1, v1, std::min<int64_t>(w1, INT32_MAX), std::min<int64_t>(w2, INT32_MAX),
+                       scale ? *scale : 1.0 / std::sqrt((double)q.size(3)));
+}
+
+Tensor checked_attend(const Tensor &q, const Tensor &k1, const Tensor &k2, const Tensor &v1, const Tensor &v2, int64_t w1, int64_t w2,
+                      std::optional<double> scale, bool pads, const py::object &admit) {
+    return attend(q, k1, k2, v1, v2, checked(q, k1, k2, v1, v2, w1, w2, scale, pads), admit);
+}
+
+// The two directions on their own, for the Python form of the node (a tracer records calls of Python Functions only).
+using MaybeTensors = std::vector<std::optional<Tensor>>;
+MaybeTensors maybe(const variable_list &all) {
+    MaybeTensors out;
+    for (const Tensor &t : all) out.push_back(t.defined() ? std::optional<Tensor>(t) : std::nullopt);
+    return out;
+}
+variable_list defined(const MaybeTensors &all) {
+    variable_list out;
+    for (const auto &t : all) out.push_back(t.value_or(Tensor()));
+    return out;
+}
+
+std::tuple<Tensor, MaybeTensors, std::vector<int64_t>, double> attend_forward(const Tensor &q, const Tensor &k1, const Tensor &k2, const Tensor &v1,
+                                                                              const Tensor &v2, int64_t w1, int64_t w2, std::optional<double> scale,
+                                                                              bool needs_grad, const py::object &admit) {
+    const Geometry g = checked(q, k1, k2, v1, v2, w1, w2, scale, false);
+    const Forward f = run_forward(q, k1, k2, v1, v2, g, needs_grad, needs_grad && keep_partials(g, q, admit));
+    return {f.result, maybe(Attend::saved_of(f)), Attend::sizes_of(g, {&q, &k1, &k2, &v1, &v2}), g.scale};
+}
+
+variable_list attend_backward(const MaybeTensors &saved, const std::vector<int64_t> &sizes, double scale, const Tensor &dout) {
+    return Attend::run_backward(defined(saved), sizes, scale, dout);
 }
 
 // ---- fused split + per-head RMSNorm of the qkv projection
@@ -290,11 +342,26 @@ struct QKVNorm : public torch::autograd::Function<QKVNorm> {
     using Weight = std::optional<Tensor>;
     static variable_list forward(AutogradContext *ctx, const Tensor &qkv, const Weight &wq, const Weight &wk1, const Weight &wk2, const Weight &wv1,
                                  const Weight &wv2, int64_t heads, int64_t kv_heads, int64_t dim, double eps) {
-        return run(ctx, qkv, {&wq, &wk1, &wk2, &wv1, &wv2}, heads, kv_heads, dim, eps);
+        Saved saved;
+        variable_list outs = run(&saved, qkv, {&wq, &wk1, &wk2, &wv1, &wv2}, heads, kv_heads, dim, eps);
+        ctx->save_for_backward(saved.tensors);
+        ctx->saved_data["geometry"] = c10::List<int64_t>(saved.sizes);
+        return outs;
     }
 
-    // (ctx == nullptr: no backward follows)
-    static variable_list run(AutogradContext *ctx, const Tensor &qkv_in, const std::array<const Weight *, 5> &w, int64_t heads, int64_t kv_heads,
+    static variable_list backward(AutogradContext *ctx, variable_list douts) {
+        variable_list grads = run_backward(ctx->get_saved_variables(), ctx->saved_data["geometry"].toIntVector(), douts);
+        grads.resize(10);
+        return grads;
+    }
+
+    struct Saved {
+        variable_list tensors;
+        std::vector<int64_t> sizes;
+    };
+
+    // (saved == nullptr: no backward follows)
+    static variable_list run(Saved *saved, const Tensor &qkv_in, const std::array<const Weight *, 5> &w, int64_t heads, int64_t kv_heads,
                              int64_t dim, double eps) {
         const int64_t batch = qkv_in.size(0), seq = qkv_in.size(1);
         const Tensor qkv = qkv_in.stride(2) == 1 && qkv_in.stride(0) == seq * qkv_in.stride(1) ? qkv_in : qkv_in.contiguous();
@@ -313,12 +380,10 @@ struct QKVNorm : public torch::autograd::Function<QKVNorm> {
         }
         check(sa2_qkv_norm_fwd(&prob, qkv.data_ptr(), qkv.stride(1), p[0], p[1], p[2], p[3], p[4], (float)eps, &a[0], &a[1], &a[2], &a[3], &a[4],
                                static_cast<float *>(rstd.data_ptr()), stream_of(qkv)));
-        if (ctx) {
-            ctx->save_for_backward({qkv, rstd, weights[0], weights[1], weights[2], weights[3], weights[4]});
-            c10::List<int64_t> n;
-            for (const int64_t v : {batch, seq, heads, kv_heads, dim}) n.push_back(v);
-            for (int x = 0; x < 5; ++x) n.push_back(w[x]->has_value() ? (int64_t)(*w[x])->scalar_type() : -1);
-            ctx->saved_data["geometry"] = n;
+        if (saved) {
+            saved->tensors = {qkv, rstd, weights[0], weights[1], weights[2], weights[3], weights[4]};
+            saved->sizes = {batch, seq, heads, kv_heads, dim};
+            for (int x = 0; x < 5; ++x) saved->sizes.push_back(w[x]->has_value() ? (int64_t)(*w[x])->scalar_type() : -1);
         }
         return outs;
     }
@@ -327,10 +392,8 @@ struct QKVNorm : public torch::autograd::Function<QKVNorm> {
         return {(int32_t)batch, (int32_t)seq, (int32_t)heads, (int32_t)kv_heads, (int32_t)dim, 1, 1, 1, 1.f, SA2_BF16};
     }
 
-    static variable_list backward(AutogradContext *ctx, variable_list douts) {
-        const variable_list s = ctx->get_saved_variables();
+    static variable_list run_backward(const variable_list &s, const std::vector<int64_t> &n, variable_list douts) {
         const Tensor &qkv = s[0], &rstd = s[1];
-        const c10::List<int64_t> n = ctx->saved_data["geometry"].toIntList();
         const int64_t batch = n[0], seq = n[1], heads = n[2], kv_heads = n[3], dim = n[4];
         const c10::DeviceGuard guard(qkv.device());
         const sa2_problem prob = problem(batch, seq, heads, kv_heads, dim);
@@ -348,13 +411,13 @@ struct QKVNorm : public torch::autograd::Function<QKVNorm> {
         check(sa2_qkv_norm_bwd(&prob, qkv.data_ptr(), qkv.stride(1), p[0], p[1], p[2], p[3], p[4], &a[0], &a[1], &a[2], &a[3], &a[4],
                                static_cast<float *>(rstd.data_ptr()), dqkv.data_ptr(), static_cast<float *>(dw.data_ptr()), ws.data_ptr(), ws_bytes,
                                stream_of(qkv)));
-        variable_list result(10);
+        variable_list result(6);
         result[0] = dqkv;
         // (one cast for weights of one type)
         Tensor cast = dw;
         for (int x = 0; x < 5; ++x) {
             if (n[5 + x] < 0) continue;
-            const auto type = (at::ScalarType)(int64_t)n[5 + x];
+            const auto type = (at::ScalarType)n[5 + x];
             if (cast.scalar_type() != type) cast = dw.to(type);
             result[1 + x] = cast.select(0, x);
         }
@@ -364,17 +427,35 @@ struct QKVNorm : public torch::autograd::Function<QKVNorm> {
 
 variable_list qkv_norm(const Tensor &qkv, const QKVNorm::Weight &wq, const QKVNorm::Weight &wk1, const QKVNorm::Weight &wk2,
                        const QKVNorm::Weight &wv1, const QKVNorm::Weight &wv2, int64_t heads, int64_t kv_heads, int64_t dim, double eps) {
-    bool grad = qkv.requires_grad();
+    bool seen = in_autograd({&qkv});
     const std::array<const QKVNorm::Weight *, 5> w{&wq, &wk1, &wk2, &wv1, &wv2};
-    for (const auto *x : w) grad = grad || (x->has_value() && (*x)->requires_grad());
-    if (!(grad && at::GradMode::is_enabled())) return QKVNorm::run(nullptr, qkv, w, heads, kv_heads, dim, eps);
+    for (const auto *x : w) seen = seen || (x->has_value() && in_autograd({&**x}));
+    if (!seen) return QKVNorm::run(nullptr, qkv, w, heads, kv_heads, dim, eps);
     return QKVNorm::apply(qkv, wq, wk1, wk2, wv1, wv2, heads, kv_heads, dim, eps);
+}
+
+// (for the Python form of the node, as attend_forward and attend_backward)
+std::tuple<variable_list, MaybeTensors, std::vector<int64_t>> qkv_norm_forward(const Tensor &qkv, const QKVNorm::Weight &wq, const QKVNorm::Weight &wk1,
+                                                                               const QKVNorm::Weight &wk2, const QKVNorm::Weight &wv1,
+                                                                               const QKVNorm::Weight &wv2, int64_t heads, int64_t kv_heads, int64_t dim,
+                                                                               double eps) {
+    QKVNorm::Saved saved;
+    variable_list outs = QKVNorm::run(&saved, qkv, {&wq, &wk1, &wk2, &wv1, &wv2}, heads, kv_heads, dim, eps);
+    return {outs, maybe(saved.tensors), saved.sizes};
+}
+
+MaybeTensors qkv_norm_backward(const MaybeTensors &saved, const std::vector<int64_t> &sizes, const variable_list &douts) {
+    return maybe(QKVNorm::run_backward(defined(saved), sizes, douts));
 }
 
 }  // namespace
 
 PYBIND11_MODULE(_sa2_torch, m) {
     m.def("attend", &checked_attend);
+    m.def("attend_forward", &attend_forward);
+    m.def("attend_backward", &attend_backward);
     m.def("qkv_norm", &qkv_norm);
+    m.def("qkv_norm_forward", &qkv_norm_forward);
+    m.def("qkv_norm_backward", &qkv_norm_backward);
     m.def("released_bytes", [](int device) { return device >= 0 && device < kMostDevices ? g_released[device].load() : int64_t(0); });
 }

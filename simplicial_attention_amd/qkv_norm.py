@@ -26,7 +26,19 @@ class FusedQKVNorm(Function):
     def apply(cls, qkv, wq, wk1, wk2, wv1, wv2, heads, kv_heads, dim_head, eps):
         assert qkv.is_cuda and qkv.dtype == torch.bfloat16 and qkv.dim() == 3
         assert qkv.shape[-1] == (heads + 4 * kv_heads) * dim_head, 'projection width does not match the head layout'
+        if torch.jit.is_tracing():      # (a tracer sees Python Functions only)
+            return super().apply(qkv, wq, wk1, wk2, wv1, wv2, heads, kv_heads, dim_head, eps)
         return tuple(_native.torch_ext().qkv_norm(qkv, wq, wk1, wk2, wv1, wv2, heads, kv_heads, dim_head, float(eps)))
+
+    @staticmethod
+    def forward(ctx, qkv, wq, wk1, wk2, wv1, wv2, heads, kv_heads, dim_head, eps):
+        outs, saved, ctx.sizes = _native.torch_ext().qkv_norm_forward(qkv, wq, wk1, wk2, wv1, wv2, heads, kv_heads, dim_head, float(eps))
+        ctx.save_for_backward(*saved)
+        return tuple(outs)
+
+    @staticmethod
+    def backward(ctx, *grads):
+        return (*_native.torch_ext().qkv_norm_backward(ctx.saved_tensors, ctx.sizes, grads), None, None, None, None)
 
 
 def fused_qkv_norm(qkv, norms, heads, kv_heads, dim_head):

@@ -14,6 +14,7 @@ import threading
 from functools import partial
 
 import torch
+import torch.nn.functional as F
 from torch import Tensor
 from torch.autograd import Function
 
@@ -96,7 +97,23 @@ class SlidingTwoSimplicialAttention(Function):
         # (csrc/sa2_torch.cpp): from here they cost more than the kernels of a small call.
         if not causal:
             raise NotImplementedError('only causal=True is defined for the sliding windows')
+        # A tracer (torch.jit.trace) sees Python Functions only: it gets this one.
+        if torch.jit.is_tracing():
+            return super().apply(q, k1, k2, v1, v2, w1, w2, causal, scale)
         return _native.torch_ext().attend(q, k1, k2, v1, v2, int(w1), int(w2), scale, False, partials_budget.admit)
+
+    @staticmethod
+    def forward(ctx, q, k1, k2, v1, v2, w1, w2, causal, scale=None):
+        if not causal:
+            raise NotImplementedError('only causal=True is defined for the sliding windows')
+        out, saved, ctx.sizes, ctx.scale = _native.torch_ext().attend_forward(
+            q, k1, k2, v1, v2, int(w1), int(w2), scale, any(ctx.needs_input_grad[:5]), partials_budget.admit)
+        ctx.save_for_backward(*saved)
+        return out
+
+    @staticmethod
+    def backward(ctx, dout):
+        return (*_native.torch_ext().attend_backward(ctx.saved_tensors, ctx.sizes, ctx.scale, dout), None, None, None, None)
 
 
 _sliding_two_simplicial_attn = SlidingTwoSimplicialAttention.apply
@@ -144,6 +161,10 @@ def sliding_two_simplicial_attn(
         return _sliding_two_simplicial_attn(q, k1, k2, v1, v2, w1, w2, causal)
     if not causal:
         raise NotImplementedError('only causal=True is defined for the sliding windows')
+    if torch.jit.is_tracing():
+        kernel_dim = next(d for d in (32, 64, 128, 256) if dim <= d)
+        rows = [F.pad(t.to(torch.bfloat16), (0, kernel_dim - t.shape[-1])) for t in (q, k1, k2, v1, v2)]
+        return _sliding_two_simplicial_attn(*rows, w1, w2, causal, dim_qk ** -0.5)[..., :dim_v].to(dtype)
     k1, k2, v1, v2 = (t if t.dtype in _DTYPES else t.to(torch.bfloat16) for t in (k1, k2, v1, v2))
     return _native.torch_ext().attend(q, k1, k2, v1, v2, int(w1), int(w2), None, True, partials_budget.admit)
 
