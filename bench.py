@@ -130,7 +130,7 @@ ENTRY_KERNEL = {'fwd': 'fwd', 'bwd_dq_dk2_pass': 'bwd_q_kernel', 'bwd_dkv1': 'bw
 
 def kernel_symbol(entry, D, w2):
     if D == 256:
-        return {'fwd': 'sa2::fwd_wide_kernel<256>', 'bwd_dq_dk2_pass': 'sa2::bwd_wide_q_kernel<256, true>', 'bwd_dkv1': 'sa2::bwd_wide_kv_kernel<256>'}.get(entry)
+        return {'fwd': 'sa2::fwd_wide_kernel<256>', 'bwd_dq_dk2_pass': 'sa2::bwd_wide_q_kernel<256, true>', 'bwd_dkv1': 'sa2::bwd_kvr_kernel<256, false>'}.get(entry)
     if entry == 'fwd':
         return 'sa2::fwd2_kernel<128>' if D == 128 else 'sa2::fwd_kernel<%d>' % D
     if entry == 'bwd_dq_dk2_pass':

@@ -422,7 +422,6 @@ static int64_t kv_part_bytes(const sa2_problem *prob) {
 static constexpr int64_t kPartBytes = 192ll << 20;
 
 static Kv8Plan kv8_plan(const sa2_problem *prob) {
-    if (prob->dim_head == kWideDimHead) return {0, 1};
     const int nslab = (prob->seq_len + 127) / 128, G = prob->heads / prob->kv_heads;
     const int64_t heads = (int64_t)prob->batch * prob->kv_heads;
     const int64_t budget = max64(kPartBytes, partial_rows_bytes(prob));
@@ -621,16 +620,14 @@ static int launch_dkv1(const sa2_problem *prob, const sa2_tensor *q, const sa2_t
     k.kv_chunk = plan.chunk;
     k.kv_max_parts = plan.parts;
     hipStream_t s = static_cast<hipStream_t>(hip_stream);
-    if (prob->dim_head == kWideDimHead) {
-        const int wgrid = prob->batch * prob->kv_heads * ((prob->seq_len + 31) / 32);
-        sa2::launch_bwd_wide_kv(wgrid, s, k);
-        return after_launch("dk1/dv1");
-    }
     const int grid = prob->batch * prob->kv_heads * ((prob->seq_len + 127) / 128);
-    // dim_head 128: the two waves of a slab split the contractions; dim_head 64 and 32: each wave forms both outputs
+    // dim_head 256: one wave per SIMD with everything in registers; 128: the two waves of a slab split the contractions (everything
+    // in registers takes 6.0 ms there, 4.9 this way); 64 and 32: each wave forms both outputs
     const bool in_parts = plan.parts > 1;
     const dim3 kgrid(in_parts ? plan.parts * grid : grid), block(512);
-    if (prob->dim_head == 128) {
+    if (prob->dim_head == kWideDimHead) {
+        sa2::launch_bwd_kvr(in_parts, kgrid.x, s, k);
+    } else if (prob->dim_head == 128) {
         if (in_parts) hipLaunchKernelGGL((sa2::bwd_kv8_kernel<128, sa2::kKvSplit, true>), kgrid, block, 0, s, k);
         else hipLaunchKernelGGL((sa2::bwd_kv8_kernel<128, sa2::kKvSplit>), kgrid, block, 0, s, k);
     } else if (prob->dim_head == 64) {
@@ -645,7 +642,7 @@ static int launch_dkv1(const sa2_problem *prob, const sa2_tensor *q, const sa2_t
     const int64_t rows = (int64_t)prob->batch * prob->kv_heads * prob->seq_len;
     const int rows_per_block = 256 / (prob->dim_head / 8);
     const int cgrid = (int)((rows + rows_per_block - 1) / rows_per_block);
-    SA2_FOR_DIM_HEAD(prob->dim_head, hipLaunchKernelGGL(sa2::dkv1_parts_combine_kernel<DH>, dim3(cgrid, 2), dim3(256), 0, s, k));
+    SA2_FOR_ANY_DIM_HEAD(prob->dim_head, hipLaunchKernelGGL(sa2::dkv1_parts_combine_kernel<DH>, dim3(cgrid, 2), dim3(256), 0, s, k));
     return after_launch("dk1/dv1 parts combine");
 }
 

@@ -14,8 +14,4 @@ void launch_bwd_wide_q(bool dq, int grid, hipStream_t stream, const KParams &p, 
     else hipLaunchKernelGGL((bwd_wide_q_kernel<256, false>), dim3(grid), dim3(256), 0, stream, p, ws, halo);
 }
 
-void launch_bwd_wide_kv(int grid, hipStream_t stream, const KParams &p) {
-    hipLaunchKernelGGL(bwd_wide_kv_kernel<256>, dim3(grid), dim3(256), 0, stream, p);
-}
-
 }  // namespace sa2
