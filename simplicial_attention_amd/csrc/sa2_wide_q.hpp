@@ -276,10 +276,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
                     if constexpr (s < KS) X = mfma32(f[s % W], A[s], X);
                     else dP = mfma32(f[s % W], B[DQ ? s - KS : 0], dP);
                     if constexpr (s + W < NFR) f[s % W] = fragment(std::integral_constant<int, s + W>{});
-                    if constexpr (DQ && s >= KS + 2 && s < KS + 10) {
-                        constexpr int e = 2 * (s - KS - 2);
+                    if constexpr (DQ && s > KS) {
+                        constexpr int e = s - KS - 1;           // (one behind each, the last two together)
                         X[e] = fast_exp2(X[e]);
-                        X[e + 1] = fast_exp2(X[e + 1]);
+                        if constexpr (s == NROW - 1) X[e + 1] = fast_exp2(X[e + 1]);
                     }
                     __builtin_amdgcn_sched_barrier(0);
                 });
