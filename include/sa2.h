@@ -265,6 +265,12 @@ int sa2_qkv_norm_bwd(const sa2_problem *prob, const void *qkv, int64_t row_strid
                      const sa2_tensor *dv1, const sa2_tensor *dv2, const float *rstd,
                      void *dqkv, float *dw, void *workspace, int64_t workspace_bytes, void *hip_stream);
 
+/* Weight gradient of a linear layer: dw[out_features][in_features] = sum over rows of dy[row][.] x[row][.]^T, bf16 in and out,
+ * fp32 sums in a fixed order.  The features are multiples of 128; strides in elements.  -1 for other sizes. */
+int64_t sa2_wgrad_workspace_bytes(int64_t rows, int32_t out_features, int32_t in_features);
+int sa2_wgrad(const void *dy, int64_t dy_stride, const void *x, int64_t x_stride, int64_t rows, int32_t out_features, int32_t in_features,
+              void *dw, void *workspace, int64_t workspace_bytes, void *hip_stream);
+
 #ifdef __cplusplus
 }
 #endif

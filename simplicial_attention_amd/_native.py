@@ -31,7 +31,8 @@ EXPORTS = ('sa2_version', 'sa2_last_error', 'sa2_supported', 'sa2_saved_t_bytes'
            'sa2_bwd_delta', 'sa2_bwd_workspace_bytes', 'sa2_bwd_workspace_bytes_with_saved',
            'sa2_bwd_split', 'sa2_bwd_split_workspace_bytes', 'sa2_bwd_dq_dkv2', 'sa2_bwd_dkv1', 'sa2_bwd',
            'sa2_bwd_noalloc_scratch_bytes', 'sa2_bwd_noalloc',
-           'sa2_convert', 'sa2_qkv_norm_fwd', 'sa2_qkv_norm_bwd_workspace_bytes', 'sa2_qkv_norm_bwd')
+           'sa2_convert', 'sa2_qkv_norm_fwd', 'sa2_qkv_norm_bwd_workspace_bytes', 'sa2_qkv_norm_bwd',
+           'sa2_wgrad_workspace_bytes', 'sa2_wgrad')
 
 
 class Sa2Error(RuntimeError):
@@ -106,6 +107,10 @@ def _declare(lib: ctypes.CDLL) -> ctypes.CDLL:
     lib.sa2_qkv_norm_fwd.argtypes = [P, V, I64, V, V, V, V, V, ctypes.c_float, T, T, T, T, T, F, V]
     lib.sa2_qkv_norm_bwd.restype = ctypes.c_int
     lib.sa2_qkv_norm_bwd.argtypes = [P, V, I64, V, V, V, V, V, T, T, T, T, T, F, V, F, V, I64, V]
+    lib.sa2_wgrad_workspace_bytes.restype = I64
+    lib.sa2_wgrad_workspace_bytes.argtypes = [I64, ctypes.c_int32, ctypes.c_int32]
+    lib.sa2_wgrad.restype = ctypes.c_int
+    lib.sa2_wgrad.argtypes = [V, I64, V, I64, I64, ctypes.c_int32, ctypes.c_int32, V, V, I64, V]
     return lib
 
 

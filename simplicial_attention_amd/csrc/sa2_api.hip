@@ -17,6 +17,7 @@
 #include "sa2_convert.hpp"
 #include "sa2_lds.hpp"
 #include "sa2_qkv_norm.hpp"
+#include "sa2_wgrad.hpp"
 #include "sa2_fwd.hpp"
 #include "sa2_launch.hpp"
 #ifdef SA2_PROFILING
@@ -861,6 +862,61 @@ int sa2_qkv_norm_bwd(const sa2_problem *prob, const void *qkv, int64_t row_strid
     const int n = 5 * prob->dim_head;
     hipLaunchKernelGGL(sa2::qkv_norm_dw_kernel, dim3((n + 15) / 16), dim3(1024), 0, s, np.dw_part, dw, blocks, n);
     return after_launch("qkv norm weight gradients");
+}
+
+// ---- weight gradient of a linear layer
+// Shares of the rows: two workgroups per CU, at least sixteen 32-row tiles each.  16384 rows, 1536 x 512 (us): one workgroup per
+// CU 48, two 45, three 56 (the partial blocks are written and read once); 16384 rows, 256 x 512: sixteen tiles 21, eight 27.
+static int wgrad_shares(int64_t rows, int out_features, int in_features, int *share_tiles) {
+    const int64_t tiles = (rows + 31) / 32, blocks = (int64_t)(out_features / 128) * (in_features / 128);
+    int64_t shares = 2 * kComputeUnits / blocks;
+    shares = shares < tiles / 16 ? shares : tiles / 16;
+    shares = shares < 1 ? 1 : shares;
+    const int64_t per = (tiles + shares - 1) / shares;
+    *share_tiles = (int)per;
+    return (int)((tiles + per - 1) / per);
+}
+
+static bool wgrad_fits(int64_t rows, int out_features, int in_features) {
+    return rows >= 1 && rows < (1ll << 30) && out_features >= 128 && out_features % 128 == 0 && in_features >= 128 && in_features % 128 == 0;
+}
+
+int64_t sa2_wgrad_workspace_bytes(int64_t rows, int32_t out_features, int32_t in_features) {
+    if (!wgrad_fits(rows, out_features, in_features)) return -1;
+    int per;
+    return (int64_t)wgrad_shares(rows, out_features, in_features, &per) * out_features * in_features * 4;
+}
+
+int sa2_wgrad(const void *dy, int64_t dy_stride, const void *x, int64_t x_stride, int64_t rows, int32_t out_features, int32_t in_features, void *dw,
+              void *workspace, int64_t workspace_bytes, void *hip_stream) {
+    if (!dy || !x || !dw || !workspace) return fail(SA2_ERR_NULL_POINTER, "dy, x, dw or workspace is NULL");
+    if (!wgrad_fits(rows, out_features, in_features))
+        return fail(SA2_ERR_BAD_SHAPE, "rows=%lld must be positive, out_features=%d and in_features=%d multiples of 128", (long long)rows, out_features, in_features);
+    if (dy_stride < out_features || x_stride < in_features || dy_stride > (1 << 24) || x_stride > (1 << 24))
+        return fail(SA2_ERR_BAD_SHAPE, "row strides %lld and %lld do not hold rows of %d and %d", (long long)dy_stride, (long long)x_stride, out_features, in_features);
+    if (((reinterpret_cast<uintptr_t>(dy) | reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(dw) | reinterpret_cast<uintptr_t>(workspace)) & 15) != 0 ||
+        dy_stride % 8 != 0 || x_stride % 8 != 0)
+        return fail(SA2_ERR_ALIGNMENT, "dy, x, dw, workspace and the rows must be 16-byte aligned");
+    if (workspace_bytes < sa2_wgrad_workspace_bytes(rows, out_features, in_features)) return fail(SA2_ERR_BAD_SHAPE, "the workspace is too small (sa2_wgrad_workspace_bytes())");
+    sa2::WgradParams p{};
+    p.dy = static_cast<const char *>(dy);
+    p.x = static_cast<const char *>(x);
+    p.dy_row = dy_stride * 2;
+    p.x_row = x_stride * 2;
+    p.parts = static_cast<float *>(workspace);
+    p.dw = static_cast<char *>(dw);
+    p.K = (int)rows;
+    p.M = out_features;
+    p.N = in_features;
+    p.shares = wgrad_shares(rows, out_features, in_features, &p.share_tiles);
+    const int64_t blocks = (int64_t)(out_features / 128) * (in_features / 128) * p.shares;
+    if (blocks > 0x7fffffffll) return fail(SA2_ERR_BAD_SHAPE, "problem too large for a 1-D grid");
+    hipStream_t s = static_cast<hipStream_t>(hip_stream);
+    hipLaunchKernelGGL(sa2::wgrad_kernel, dim3((unsigned)blocks), dim3(256), 0, s, p);
+    SA2_TRY(after_launch("weight gradient"));
+    const int64_t cgrid = ((int64_t)out_features * in_features / 8 + 255) / 256;
+    hipLaunchKernelGGL(sa2::wgrad_combine_kernel, dim3((unsigned)cgrid), dim3(256), 0, s, p);
+    return after_launch("weight gradient combine");
 }
 
 #ifdef SA2_PROFILING

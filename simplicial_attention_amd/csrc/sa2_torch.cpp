@@ -448,6 +448,48 @@ MaybeTensors qkv_norm_backward(const MaybeTensors &saved, const std::vector<int6
     return maybe(QKVNorm::run_backward(defined(saved), sizes, douts));
 }
 
+// ---- linear layer whose weight gradient is this library's kernel (the products with the weight stay torch's)
+struct Linear : public torch::autograd::Function<Linear> {
+    static Tensor forward(AutogradContext *ctx, const Tensor &x, const Tensor &w, const std::optional<Tensor> &bias) {
+        ctx->save_for_backward({x, w});
+        ctx->saved_data["bias"] = bias.has_value();
+        return at::linear(x, w, bias);
+    }
+
+    static variable_list backward(AutogradContext *ctx, variable_list douts) {
+        const variable_list s = ctx->get_saved_variables();
+        const Tensor &x = s[0], &w = s[1], &dy = douts[0];
+        const Tensor dy2 = dy.reshape({-1, w.size(0)}), x2 = x.reshape({-1, w.size(1)});
+        variable_list grads(3);
+        if (ctx->needs_input_grad(0)) grads[0] = dy2.mm(w).view_as(x);
+        if (ctx->needs_input_grad(1)) grads[1] = at::GradMode::is_enabled() ? dy2.t().mm(x2) : weight_gradient(dy2, x2);   // (a graph of the backward needs torch's)
+        if (ctx->saved_data["bias"].toBool() && ctx->needs_input_grad(2)) grads[2] = dy2.sum(0);
+        return grads;
+    }
+
+    static Tensor weight_gradient(const Tensor &dy, const Tensor &x) {
+        const c10::DeviceGuard guard(x.device());
+        auto rows = [](const Tensor &t) {
+            const bool ok = t.stride(1) == 1 && t.stride(0) >= t.size(1) && t.stride(0) % 8 == 0 && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+            return ok ? t : t.clone(at::MemoryFormat::Contiguous);
+        };
+        const Tensor a = rows(dy), b = rows(x), dw = at::empty({dy.size(1), x.size(1)}, x.options());
+        const int64_t ws_bytes = sa2_wgrad_workspace_bytes(x.size(0), (int32_t)dy.size(1), (int32_t)x.size(1));
+        const Tensor ws = at::empty({ws_bytes}, x.options().dtype(at::kByte));
+        check(sa2_wgrad(a.data_ptr(), a.stride(0), b.data_ptr(), b.stride(0), x.size(0), (int32_t)dy.size(1), (int32_t)x.size(1), dw.data_ptr(), ws.data_ptr(),
+                        ws_bytes, stream_of(x)));
+        return dw;
+    }
+};
+
+Tensor linear(const Tensor &x, const Tensor &w, const std::optional<Tensor> &bias) {
+    // (functorch's wrappers, forward-mode tangents and subclasses with a dispatch of their own keep torch's node)
+    const c10::DispatchKeySet foreign({c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper, c10::DispatchKey::Python, c10::DispatchKey::Functionalize});
+    bool plain = !at::GradMode::is_enabled() || !w.requires_grad();
+    for (const Tensor *t : {&x, &w, bias ? &*bias : &w}) plain = plain || t->key_set().has_any(foreign) || t->_fw_grad(0).defined();
+    return plain ? at::linear(x, w, bias) : Linear::apply(x, w, bias);
+}
+
 }  // namespace
 
 PYBIND11_MODULE(_sa2_torch, m) {
@@ -457,5 +499,6 @@ PYBIND11_MODULE(_sa2_torch, m) {
     m.def("qkv_norm", &qkv_norm);
     m.def("qkv_norm_forward", &qkv_norm_forward);
     m.def("qkv_norm_backward", &qkv_norm_backward);
+    m.def("linear", &linear);
     m.def("released_bytes", [](int device) { return device >= 0 && device < kMostDevices ? g_released[device].load() : int64_t(0); });
 }

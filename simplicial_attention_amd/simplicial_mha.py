@@ -13,6 +13,7 @@ from typing import Callable
 import torch
 from torch import nn
 
+from .linear import apply_linear
 from .naive import naive_two_simplicial_attend, nth_order_attend
 
 
@@ -84,13 +85,13 @@ class HigherOrderAttention(nn.Module):
 
     def forward(self, tokens):
         tokens = self.prenorm(tokens)
-        qkv = self.to_qkv(tokens)
+        qkv = apply_linear(self.to_qkv, tokens)
         if qkv.dim() == 3 and self._can_fuse(qkv):
             from .qkv_norm import fused_qkv_norm
             norms = (self.q_norm, *self.k_norms, *self.v_norms)
             q, k1, k2, v1, v2 = fused_qkv_norm(qkv, norms, self.heads, self.key_value_heads, self.split_dims[0] // self.heads)
             out = self.attend(q, (k1, k2), (v1, v2))
-            return self.postnorm(self.combine_heads(out.flatten(-2)))
+            return self.postnorm(apply_linear(self.combine_heads, out.flatten(-2)))
         q, k, v = qkv.split(self.split_dims, dim=-1)
         queries = self._split(q, self.heads)
         keys = self._split(k, self.key_value_heads).chunk(self.kv_sets, dim=-1)
@@ -102,7 +103,7 @@ class HigherOrderAttention(nn.Module):
         out = self.attend(queries, keys, values)
         if self.head_first_dim:
             out = out.transpose(1, 2)
-        out = self.combine_heads(out.flatten(-2))
+        out = apply_linear(self.combine_heads, out.flatten(-2))
         return self.postnorm(out)
 
 

@@ -14,6 +14,7 @@ import torch
 import torch.nn.functional as F
 from torch import nn
 
+from .linear import apply_linear
 from .two_simplicial_attention import SlidingWindowTwoSimplicialMHA
 
 
@@ -34,18 +35,31 @@ class Attention(nn.Module):
     def forward(self, x):
         b, n, _ = x.shape
         x = self.prenorm(x)
-        q = self.to_q(x).view(b, n, self.heads, self.dim_head).transpose(1, 2)
+        q = apply_linear(self.to_q, x).view(b, n, self.heads, self.dim_head).transpose(1, 2)
         # channel order of the fused projection: (key | value, head, d)
-        kv = self.to_kv(x).view(b, n, 2, self.key_value_heads, self.dim_head)
+        kv = apply_linear(self.to_kv, x).view(b, n, 2, self.key_value_heads, self.dim_head)
         k, v = kv[:, :, 0].transpose(1, 2), kv[:, :, 1].transpose(1, 2)
         out = F.scaled_dot_product_attention(q, k, v, is_causal=True, enable_gqa=self.heads != self.key_value_heads)
-        return self.to_out(out.transpose(1, 2).reshape(b, n, self.heads * self.dim_head))
+        return apply_linear(self.to_out, out.transpose(1, 2).reshape(b, n, self.heads * self.dim_head))
+
+
+class _Layers(nn.Sequential):
+    """``nn.Sequential`` whose plain linear layers go through ``apply_linear``."""
+
+    def forward(self, x):
+        if torch.jit.is_scripting():
+            for layer in self:
+                x = layer(x)
+        else:
+            for layer in self:
+                x = apply_linear(layer, x)
+        return x
 
 
 def FeedForward(dim, expansion=4.):
     """RMSNorm -> Linear -> GELU -> Linear (two_simplicial_transformer.py:69-76)."""
     inner = int(dim * expansion)
-    return nn.Sequential(nn.RMSNorm(dim), nn.Linear(dim, inner), nn.GELU(), nn.Linear(inner, dim))
+    return _Layers(nn.RMSNorm(dim), nn.Linear(dim, inner), nn.GELU(), nn.Linear(inner, dim))
 
 
 class TwoSimplicialTransformer(nn.Module):
@@ -94,7 +108,7 @@ class TwoSimplicialLM(nn.Module):
             x, target = x[:, :-1], x[:, 1:]
         positions = torch.arange(x.shape[-1], device=x.device)
         hidden = self.transformer(self.token_emb(x) + self.pos_emb(positions))
-        logits = self.to_logits(hidden)
+        logits = apply_linear(self.to_logits, hidden)
         if target is None:
             return logits
         return F.cross_entropy(logits.flatten(0, 1).float(), target.flatten())
