@@ -31,7 +31,7 @@ def test_against_oracle(b, n, hq, hk, w1, w2, d):
     U.check_all(out, grads, ref_out, ref_grads)
 
 
-@pytest.mark.parametrize('d', [128, 256])
+@pytest.mark.parametrize('d', [32, 64, 128, 256])
 def test_several_workgroups_per_slab_against_one(d):
     """The same sums in shares: fp32 partial sums in another order, rounded to bf16 once."""
     from simplicial_attention_amd import _native

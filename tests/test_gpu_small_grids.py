@@ -1,0 +1,68 @@
+"""Work shared by several workgroups against the same work in one, and the conversions around the kernels."""
+import pytest
+import torch
+
+from tests import parity_util as U
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [
+    # b, n, hq, hk, w1, w2
+    (1, 40, 1, 1, 16, 33),         # two query tiles of several rounds
+    (1, 333, 2, 1, 512, 32),
+    (1, 700, 2, 2, 300, 20),
+]
+
+
+@pytest.mark.parametrize('d', [32, 64, 128])
+@pytest.mark.parametrize('b,n,h,hk,w1,w2', SHAPES)
+def test_forward_in_shares(b, n, h, hk, w1, w2, d):
+    """fp32 partial rows merged once: out and lse agree to one bf16 rounding and to fp32 sums."""
+    from simplicial_attention_amd import _native
+    lib = _native.load()
+    print(f'\ncase b={b} n={n} h={h} hk={hk} d={d} w1={w1} w2={w2}', flush=True)
+    ins = [t.cuda() for t in U.make_inputs(b, n, h, hk, d, seed=n + d)][:5]
+    prob = _native.problem(b, n, h, hk, d, w1, w2, True, d ** -0.5)
+    size = lib.sa2_fwd_workspace_bytes(prob)
+    assert size > 0, 'the grid is not small enough to be shared out'
+    arg, stream = _native.tensor_arg, torch.cuda.current_stream().cuda_stream
+    results = []
+    for ws in (None, torch.full((size,), 255, dtype=torch.uint8, device='cuda')):
+        out, lse = torch.full_like(ins[0], float('nan')), torch.full((b, h, n), float('nan'), device='cuda')
+        _native.check(lib.sa2_fwd_ws(prob, *(arg(t) for t in ins), arg(out), None, lse.data_ptr(), None, None if ws is None else ws.data_ptr(),
+                                     0 if ws is None else size, stream))
+        torch.cuda.synchronize()
+        results.append((out.float(), lse))
+    (o0, l0), (o1, l1) = results
+    assert float((l0 - l1).abs().max()) <= 1e-4 * max(1.0, float(l0.abs().max()))
+    # (the saved maximum of a share differs, so weights round to bf16 at other places: 2^-9 each, averaged over the row)
+    assert float((o0 - o1).norm() / o0.norm()) <= 2.0 ** -8
+
+
+@pytest.mark.parametrize('src_type,dst_type', [(torch.float32, torch.bfloat16), (torch.float16, torch.bfloat16), (torch.bfloat16, torch.float32),
+                                               (torch.bfloat16, torch.float16), (torch.bfloat16, torch.bfloat16)])
+@pytest.mark.parametrize('src_dim,dst_dim,vector', [(96, 128, True), (128, 96, True), (33, 64, False), (64, 33, False), (5, 32, False), (64, 64, True)])
+def test_conversions_against_torch(src_type, dst_type, src_dim, dst_dim, vector):
+    """Truncated or zero-padded rows; `vector`: whether rows are aligned for 16-byte accesses.  One rounding, as torch's."""
+    import ctypes
+    from simplicial_attention_amd import _native
+    lib = _native.load()
+    lib.sa2_convert.restype = ctypes.c_int
+    code = {torch.bfloat16: 0, torch.float16: 1, torch.float32: 2}
+
+    class Conversion(ctypes.Structure):
+        _fields_ = [('src', _native.TensorArg), ('dst', _native.TensorArg)] + [(f, ctypes.c_int32) for f in
+                   ('src_type', 'dst_type', 'src_dim', 'dst_dim', 'batch', 'seq_len', 'heads')]
+
+    b, n, h = 2, 37, 3
+    pad = 8 if vector else 3
+    src = (torch.randn(b, n, h, src_dim + pad, device='cuda') * 3).to(src_type)[..., :src_dim]
+    src[0, 0, 0, :3] = torch.tensor([float('inf'), float('nan'), -0.0], device='cuda').to(src_type)
+    dst = torch.full((b, n, h, dst_dim + pad), 7.0, device='cuda').to(dst_type)
+    item = Conversion(_native.tensor_arg(src), _native.tensor_arg(dst[..., :dst_dim]), code[src_type], code[dst_type], src_dim, dst_dim, b, n, h)
+    _native.check(lib.sa2_convert(ctypes.byref(item), 1, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    want = torch.zeros(b, n, h, dst_dim, device='cuda', dtype=dst_type)
+    common = min(src_dim, dst_dim)
+    want[..., :common] = src[..., :common].to(dst_type)
+    assert torch.equal(torch.nan_to_num(dst[..., :dst_dim], nan=123.0), torch.nan_to_num(want, nan=123.0))
+    assert torch.equal(dst[..., :dst_dim].isnan(), want.isnan()) and bool((dst[..., dst_dim:] == 7.0).all())
