@@ -24,10 +24,12 @@ def _faster(rows, out_features, in_features):
 
 def apply_linear(layer, x):
     """``layer(x)``; plain bf16 ``nn.Linear`` layers under training take the node with the kernel of their own."""
-    if torch.compiler.is_compiling() or torch.jit.is_tracing() or type(layer) is not nn.Linear or not x.is_cuda or not torch.is_grad_enabled():
+    # (torch.fx hands over proxies: the type comes first)
+    if (type(x) is not Tensor or type(layer) is not nn.Linear or torch.compiler.is_compiling() or torch.jit.is_tracing()
+            or not x.is_cuda or not torch.is_grad_enabled()):
         return layer(x)
     weight, bias = layer.weight, layer.bias
-    if (type(x) is not Tensor or type(weight) is not nn.Parameter or type(bias) not in (nn.Parameter, type(None))
+    if (type(weight) is not nn.Parameter or type(bias) not in (nn.Parameter, type(None))
             or x.dtype is not torch.bfloat16 or weight.dtype is not torch.bfloat16 or (bias is not None and bias.dtype is not torch.bfloat16)
             or x.device != weight.device or x.dim() < 2 or x.shape[-1] != weight.shape[1]
             or not _faster(x.numel() // x.shape[-1] if x.shape[-1] else 0, *weight.shape)

@@ -8,7 +8,7 @@ import torch
 
 from oracle import reference_attend as R
 from simplicial_attention_amd.two_simplicial_attention import SlidingWindowTwoSimplicialMHA
-from simplicial_attention_amd.two_simplicial_transformer import Attention, TwoSimplicialLM, TwoSimplicialTransformer
+from simplicial_attention_amd.two_simplicial_transformer import Attention, FeedForward, TwoSimplicialLM, TwoSimplicialTransformer
 
 
 def test_layer_placement_and_parameter_names():
@@ -72,3 +72,14 @@ def test_small_language_model_loss_and_gradients_on_gpu():
         worst = max(worst, rel)
         assert rel <= 4e-2, (name, rel)      # bf16 parameters, activations and 4 layers of bf16 matmuls against an fp32 model
     print('largest relative gradient error', worst)
+
+
+@pytest.mark.parametrize('module,shape', [
+    (FeedForward(64), (2, 9, 64)),
+    (Attention(64, dim_head=32, heads=4, key_value_heads=2), (2, 9, 64)),
+    (TwoSimplicialTransformer(64, depth=2, heads=2, key_value_heads=2, dim_head=32, two_simplicial_attn_every=4), (2, 9, 64)),
+], ids=['feed_forward', 'attention', 'transformer_without_simplicial_layers'])
+def test_symbolic_traces(module, shape):
+    """``torch.fx.symbolic_trace`` runs the Python of these modules on proxies."""
+    x = torch.randn(shape)
+    assert torch.equal(torch.fx.symbolic_trace(module)(x), module(x))
