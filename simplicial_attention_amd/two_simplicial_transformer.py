@@ -35,12 +35,19 @@ class Attention(nn.Module):
     def forward(self, x):
         b, n, _ = x.shape
         x = self.prenorm(x)
-        q = apply_linear(self.to_q, x).view(b, n, self.heads, self.dim_head).transpose(1, 2)
+        if torch.jit.is_scripting():      # (a scripted module takes its own submodules only)
+            q, kv = self.to_q(x), self.to_kv(x)
+        else:
+            q, kv = apply_linear(self.to_q, x), apply_linear(self.to_kv, x)
+        q = q.view(b, n, self.heads, self.dim_head).transpose(1, 2)
         # channel order of the fused projection: (key | value, head, d)
-        kv = apply_linear(self.to_kv, x).view(b, n, 2, self.key_value_heads, self.dim_head)
+        kv = kv.view(b, n, 2, self.key_value_heads, self.dim_head)
         k, v = kv[:, :, 0].transpose(1, 2), kv[:, :, 1].transpose(1, 2)
         out = F.scaled_dot_product_attention(q, k, v, is_causal=True, enable_gqa=self.heads != self.key_value_heads)
-        return apply_linear(self.to_out, out.transpose(1, 2).reshape(b, n, self.heads * self.dim_head))
+        out = out.transpose(1, 2).reshape(b, n, self.heads * self.dim_head)
+        if torch.jit.is_scripting():
+            return self.to_out(out)
+        return apply_linear(self.to_out, out)
 
 
 class _Layers(nn.Sequential):

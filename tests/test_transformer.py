@@ -83,3 +83,9 @@ def test_symbolic_traces(module, shape):
     """``torch.fx.symbolic_trace`` runs the Python of these modules on proxies."""
     x = torch.randn(shape)
     assert torch.equal(torch.fx.symbolic_trace(module)(x), module(x))
+
+
+@pytest.mark.parametrize('module', [FeedForward(64), Attention(64, dim_head=32, heads=4, key_value_heads=2)], ids=['feed_forward', 'attention'])
+def test_scripts(module):
+    x = torch.randn(2, 9, 64)
+    assert torch.equal(torch.jit.script(module)(x), module(x))
