@@ -2,15 +2,22 @@
 from __future__ import annotations
 
 import torch
+import torch.nn.functional as F
 from torch import Tensor, nn
 from torch.nn.modules import module as _module
 
 from . import _native
 
 
+# what a call of a linear layer goes through, as torch has it
+_FORWARD, _CALL, _CALL_IMPL, _LINEAR = nn.Linear.forward, nn.Linear.__call__, nn.Linear._call_impl, F.linear
+
+
 def _watched(layer):
     """Someone else sees the calls of this layer, or has changed what it is."""
-    return bool(layer._forward_hooks or layer._forward_pre_hooks or layer._backward_hooks or layer._backward_pre_hooks
+    if nn.Linear.forward is not _FORWARD or nn.Linear.__call__ is not _CALL or nn.Linear._call_impl is not _CALL_IMPL or F.linear is not _LINEAR:
+        return True
+    return bool(layer._compiled_call_impl is not None or layer._forward_hooks or layer._forward_pre_hooks or layer._backward_hooks or layer._backward_pre_hooks
                 or _module._global_forward_hooks or _module._global_forward_pre_hooks or _module._global_backward_hooks
                 or _module._global_backward_pre_hooks or 'forward' in layer.__dict__)
 

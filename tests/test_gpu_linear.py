@@ -84,3 +84,28 @@ def test_hooks_see_the_layer():
     apply_linear(layer, x)
     handle.remove()
     assert seen == [(4, 2048, 256)]
+
+
+@pytest.mark.parametrize('owner,name', [(nn.Linear, 'forward'), (nn.Module, '__call__'), (nn.Module, '_call_impl'), (nn.functional, 'linear')])
+def test_replaced_functions_see_the_layer(owner, name, monkeypatch):
+    """Replacements for all linear layers: the class's forward, a module's call, the function behind them."""
+    from simplicial_attention_amd.linear import apply_linear
+    layer, x = _layer()
+    seen, original = [], getattr(owner, name)
+
+    def replacement(*args, **kwargs):
+        seen.append(name)
+        return original(*args, **kwargs)
+
+    monkeypatch.setattr(owner, name, replacement)
+    apply_linear(layer, x)
+    assert seen
+
+
+def test_a_compiled_layer_is_called():
+    from simplicial_attention_amd.linear import apply_linear
+    layer, x = _layer()
+    seen = []
+    layer._compiled_call_impl = lambda *args: seen.append(args) or layer._call_impl(*args)      # (what nn.Module.compile sets)
+    apply_linear(layer, x)
+    assert seen
