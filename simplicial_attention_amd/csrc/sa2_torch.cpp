@@ -448,6 +448,14 @@ MaybeTensors qkv_norm_backward(const MaybeTensors &saved, const std::vector<int6
     return maybe(QKVNorm::run_backward(defined(saved), sizes, douts));
 }
 
+// batched tensors (vmap's and is_grads_batched's), functorch's wrappers, subclasses with a dispatch of their own and
+// forward-mode tangents: a kernel launched on their data pointers would miss what they carry
+bool foreign(const Tensor &t) {
+    static const c10::DispatchKeySet keys({c10::DispatchKey::Batched, c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper,
+                                           c10::DispatchKey::Python, c10::DispatchKey::Functionalize});
+    return t.key_set().has_any(keys) || t._fw_grad(0).defined();
+}
+
 // ---- linear layer whose weight gradient is this library's kernel (the products with the weight stay torch's)
 struct Linear : public torch::autograd::Function<Linear> {
     static Tensor forward(AutogradContext *ctx, const Tensor &x, const Tensor &w, const std::optional<Tensor> &bias) {
@@ -462,7 +470,8 @@ struct Linear : public torch::autograd::Function<Linear> {
         const Tensor dy2 = dy.reshape({-1, w.size(0)}), x2 = x.reshape({-1, w.size(1)});
         variable_list grads(3);
         if (ctx->needs_input_grad(0)) grads[0] = dy2.mm(w).view_as(x);
-        if (ctx->needs_input_grad(1)) grads[1] = at::GradMode::is_enabled() ? dy2.t().mm(x2) : weight_gradient(dy2, x2);   // (a graph of the backward needs torch's)
+        // (a graph of the backward and batched gradients need torch's product)
+        if (ctx->needs_input_grad(1)) grads[1] = at::GradMode::is_enabled() || foreign(dy) || foreign(x) ? dy2.t().mm(x2) : weight_gradient(dy2, x2);
         if (ctx->saved_data["bias"].toBool() && ctx->needs_input_grad(2)) grads[2] = dy2.sum(0);
         return grads;
     }
@@ -483,10 +492,8 @@ struct Linear : public torch::autograd::Function<Linear> {
 };
 
 Tensor linear(const Tensor &x, const Tensor &w, const std::optional<Tensor> &bias) {
-    // (functorch's wrappers, forward-mode tangents and subclasses with a dispatch of their own keep torch's node)
-    const c10::DispatchKeySet foreign({c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper, c10::DispatchKey::Python, c10::DispatchKey::Functionalize});
     bool plain = !at::GradMode::is_enabled() || !w.requires_grad();
-    for (const Tensor *t : {&x, &w, bias ? &*bias : &w}) plain = plain || t->key_set().has_any(foreign) || t->_fw_grad(0).defined();
+    for (const Tensor *t : {&x, &w, bias ? &*bias : &w}) plain = plain || foreign(*t);
     return plain ? at::linear(x, w, bias) : Linear::apply(x, w, bias);
 }
 

@@ -109,3 +109,31 @@ def test_a_compiled_layer_is_called():
     layer._compiled_call_impl = lambda *args: seen.append(args) or layer._call_impl(*args)      # (what nn.Module.compile sets)
     apply_linear(layer, x)
     assert seen
+
+
+@pytest.mark.parametrize('bias', [True, False])
+def test_batched_output_gradients(bias):
+    """``is_grads_batched``: the node meets a batched tensor in its backward only."""
+    from simplicial_attention_amd.linear import apply_linear
+    layer, x = _layer(bias)
+    douts = torch.randn(3, 4, 2048, 256, device='cuda').bfloat16()
+    params = [x, *layer.parameters()]
+    out = apply_linear(layer, x)
+    got = torch.autograd.grad(out, params, douts, retain_graph=True, is_grads_batched=True)
+    for n in range(3):
+        for a, b in zip(got, torch.autograd.grad(out, params, douts[n], retain_graph=True)):
+            assert float((a[n].float() - b.float()).norm() / b.float().norm()) <= 2.0 ** -8      # (two bf16 roundings of the same sums)
+
+
+def test_tangents_of_output_gradients_stay():
+    """Forward over reverse: the layer's own inputs are plain, the gradient that comes back carries a tangent."""
+    import torch.autograd.forward_ad as fwAD
+    from simplicial_attention_amd.linear import apply_linear
+    layer, x = _layer()
+    out = apply_linear(layer, x)
+    dout, tangent = torch.randn_like(out), torch.randn_like(out)
+    with fwAD.dual_level():
+        got = torch.autograd.grad(out, layer.weight, fwAD.make_dual(dout, tangent), retain_graph=True)[0]
+        got = fwAD.unpack_dual(got).tangent
+    want = torch.autograd.grad(out, layer.weight, tangent)[0]
+    assert got is not None and float((got.float() - want.float()).norm() / want.float().norm()) <= 2.0 ** -8
