@@ -459,7 +459,8 @@ bool foreign(const Tensor &t) {
 // ---- linear layer whose weight gradient is this library's kernel (the products with the weight stay torch's)
 struct Linear : public torch::autograd::Function<Linear> {
     static Tensor forward(AutogradContext *ctx, const Tensor &x, const Tensor &w, const std::optional<Tensor> &bias) {
-        ctx->save_for_backward({x, w});
+        // (the weight is for the gradient of x alone: without one it may be changed in place before the backward)
+        ctx->save_for_backward({x, x.requires_grad() ? w : Tensor()});
         ctx->saved_data["bias"] = bias.has_value();
         return at::linear(x, w, bias);
     }
@@ -467,7 +468,7 @@ struct Linear : public torch::autograd::Function<Linear> {
     static variable_list backward(AutogradContext *ctx, variable_list douts) {
         const variable_list s = ctx->get_saved_variables();
         const Tensor &x = s[0], &w = s[1], &dy = douts[0];
-        const Tensor dy2 = dy.reshape({-1, w.size(0)}), x2 = x.reshape({-1, w.size(1)});
+        const Tensor dy2 = dy.reshape({-1, dy.size(-1)}), x2 = x.reshape({-1, x.size(-1)});
         variable_list grads(3);
         if (ctx->needs_input_grad(0)) grads[0] = dy2.mm(w).view_as(x);
         // (a graph of the backward and batched gradients need torch's product)

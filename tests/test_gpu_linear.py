@@ -137,3 +137,17 @@ def test_tangents_of_output_gradients_stay():
         got = fwAD.unpack_dual(got).tangent
     want = torch.autograd.grad(out, layer.weight, tangent)[0]
     assert got is not None and float((got.float() - want.float()).norm() / want.float().norm()) <= 2.0 ** -8
+
+
+def test_a_weight_that_no_gradient_needs_may_change():
+    """As with torch's node: an input without a gradient leaves the weight free between forward and backward; one with a gradient does not."""
+    from simplicial_attention_amd.linear import apply_linear
+    layer, x = _layer()
+    dout = torch.randn(4, 2048, 256, device='cuda').bfloat16()
+    want = torch.autograd.grad(apply_linear(layer, x.detach()), layer.weight, dout)[0]
+    out, with_x = apply_linear(layer, x.detach()), apply_linear(layer, x)
+    with torch.no_grad():
+        layer.weight.mul_(2)
+    assert torch.equal(torch.autograd.grad(out, layer.weight, dout)[0], want)
+    with pytest.raises(RuntimeError, match='modified by an inplace operation'):
+        torch.autograd.grad(with_x, layer.weight, dout)
