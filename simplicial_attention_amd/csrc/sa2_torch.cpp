@@ -119,8 +119,9 @@ Tensor counted_buffer(int64_t bytes, const Tensor &like, int64_t counted) {
         .make_tensor();
 }
 
-Forward run_forward(const Tensor &q, const Tensor &k1, const Tensor &k2, const Tensor &v1, const Tensor &v2, const Geometry &g, bool needs_grad,
-                    bool save) {
+// `admit` (given where a backward may follow): called with the bytes of the per-offset value partials, says whether they may be
+// kept for the backward, in which dV2 then needs no recomputation of the attention weights
+Forward run_forward(const Tensor &q, const Tensor &k1, const Tensor &k2, const Tensor &v1, const Tensor &v2, const Geometry &g, const py::object *admit) {
     Forward f;
     const c10::DeviceGuard guard(q.device());
     void *stream = stream_of(q);
@@ -136,11 +137,14 @@ Forward run_forward(const Tensor &q, const Tensor &k1, const Tensor &k2, const T
     f.out = at::empty({g.batch, g.seq, g.heads, g.dim}, bf16);
     f.lse = at::empty({g.batch, g.heads, g.seq}, q.options().dtype(at::kFloat));
     // bf16 residual of the fp32 accumulator, kept only when a backward may follow
-    if (needs_grad) f.residual = at::empty({g.batch, g.seq, g.heads, g.dim}, bf16);
+    if (admit) f.residual = at::empty({g.batch, g.seq, g.heads, g.dim}, bf16);
     const sa2_problem prob = g.problem();
     sa2_saved saved{};
+    // (a size of 0: the kernels of this head dimension keep none; asked last, so that nothing that fails stands between the
+    // admission and the buffer that reports its end)
+    const int64_t t_bytes = sa2_saved_t_bytes(&prob), m_bytes = sa2_saved_m_bytes(&prob);
+    const bool save = admit && t_bytes + m_bytes > 0 && (*admit)(t_bytes + m_bytes, (int)q.device().index()).cast<bool>();
     if (save) {
-        const int64_t t_bytes = sa2_saved_t_bytes(&prob), m_bytes = sa2_saved_m_bytes(&prob);
         try {
             f.t_save = counted_buffer(t_bytes, q, t_bytes + m_bytes);
         } catch (...) {
@@ -155,8 +159,8 @@ Forward run_forward(const Tensor &q, const Tensor &k1, const Tensor &k2, const T
     if (ws_bytes > 0) ws = at::empty({ws_bytes}, q.options().dtype(at::kByte));
     const sa2_tensor aq = arg(f.q), ak1 = arg(f.k1), ak2 = arg(f.k2), av1 = arg(f.v1), av2 = arg(f.v2), ao = arg(f.out);
     sa2_tensor ar{};
-    if (needs_grad) ar = arg(f.residual);
-    check(sa2_fwd_ws(&prob, &aq, &ak1, &ak2, &av1, &av2, &ao, needs_grad ? &ar : nullptr, static_cast<float *>(f.lse.data_ptr()),
+    if (admit) ar = arg(f.residual);
+    check(sa2_fwd_ws(&prob, &aq, &ak1, &ak2, &av1, &av2, &ao, admit ? &ar : nullptr, static_cast<float *>(f.lse.data_ptr()),
                      save ? &saved : nullptr, ws_bytes > 0 ? ws.data_ptr() : nullptr, ws_bytes, stream));
     if (q.scalar_type() == at::kBFloat16 && g.dim_v == g.dim) {
         f.result = f.out;
@@ -171,8 +175,8 @@ Forward run_forward(const Tensor &q, const Tensor &k1, const Tensor &k2, const T
 
 struct Attend : public torch::autograd::Function<Attend> {
     static Tensor forward(AutogradContext *ctx, const Tensor &q, const Tensor &k1, const Tensor &k2, const Tensor &v1, const Tensor &v2,
-                          const Geometry &g, bool save) {
-        Forward f = run_forward(q, k1, k2, v1, v2, g, true, save);
+                          const Geometry &g, const py::object &admit) {
+        Forward f = run_forward(q, k1, k2, v1, v2, g, &admit);
         ctx->save_for_backward(saved_of(f));
         ctx->saved_data["geometry"] = c10::List<int64_t>(sizes_of(g, {&q, &k1, &k2, &v1, &v2}));
         ctx->saved_data["scale"] = g.scale;
@@ -260,15 +264,6 @@ Geometry geometry_of(const Tensor &q, const Tensor &k1, const Tensor &v1, int64_
     return g;
 }
 
-// Per-offset value partials, kept for the backward when they fit the budget: dV2 then needs no recomputation of the
-// attention weights (a size of 0: the kernels of this head dimension keep none).  `admit`: called with their bytes, says
-// whether they may be kept
-bool keep_partials(const Geometry &g, const Tensor &q, const py::object &admit) {
-    const sa2_problem prob = g.problem();
-    const int64_t bytes = sa2_saved_t_bytes(&prob) + sa2_saved_m_bytes(&prob);
-    return bytes > 0 && admit(bytes, (int)q.device().index()).cast<bool>();
-}
-
 // a call that autograd has to see: a backward may follow, or an input carries a forward-mode tangent (which the node refuses,
 // also without a graph: the derivative would be lost without a word)
 bool in_autograd(std::initializer_list<const Tensor *> inputs) {
@@ -278,8 +273,8 @@ bool in_autograd(std::initializer_list<const Tensor *> inputs) {
 }
 
 Tensor attend(const Tensor &q, const Tensor &k1, const Tensor &k2, const Tensor &v1, const Tensor &v2, const Geometry &g, const py::object &admit) {
-    if (!in_autograd({&q, &k1, &k2, &v1, &v2})) return run_forward(q, k1, k2, v1, v2, g, false, false).result;
-    return Attend::apply(q, k1, k2, v1, v2, g, keep_partials(g, q, admit));
+    if (!in_autograd({&q, &k1, &k2, &v1, &v2})) return run_forward(q, k1, k2, v1, v2, g, nullptr).result;
+    return Attend::apply(q, k1, k2, v1, v2, g, admit);
 }
 
 // shapes, types and windows of the Function and the wrapper; `pads`: other head dimensions and types than the kernels' are welcome
@@ -329,7 +324,7 @@ std::tuple<Tensor, MaybeTensors, std::vector<int64_t>, double> attend_forward(co
                                                                               const Tensor &v2, int64_t w1, int64_t w2, std::optional<double> scale,
                                                                               bool needs_grad, const py::object &admit) {
     const Geometry g = checked(q, k1, k2, v1, v2, w1, w2, scale, false);
-    const Forward f = run_forward(q, k1, k2, v1, v2, g, needs_grad, needs_grad && keep_partials(g, q, admit));
+    const Forward f = run_forward(q, k1, k2, v1, v2, g, needs_grad ? &admit : nullptr);
     return {f.result, maybe(Attend::saved_of(f)), Attend::sizes_of(g, {&q, &k1, &k2, &v1, &v2}), g.scale};
 }
 

@@ -73,3 +73,30 @@ def test_the_python_form_of_the_nodes_gives_the_same_gradients():
         grads = ext.attend_backward(saved, sizes, scale, dout)
     assert torch.equal(out, want_out)
     assert all(torch.equal(a, b) for a, b in zip(grads, want))
+
+
+@pytest.mark.parametrize('python_form', [False, True])
+def test_a_forward_that_fails_leaves_the_budget_of_saved_partials_whole(python_form):
+    """An allocation that fails (the device's share for this process is taken up to a few MiB): the bytes admitted for partials are
+    given back, or were not admitted yet."""
+    from simplicial_attention_amd import _native
+    from simplicial_attention_amd.two_simplicial_attention import partials_budget, sliding_two_simplicial_attn
+    n = 4096                           # q: 8 MiB of bf16
+    ts = [torch.randn(1, n, h, 128, device='cuda', dtype=torch.bfloat16).requires_grad_() for h in (8, 8, 8, 8, 8)]
+    live = lambda: partials_budget.live.get(0, 0) - _native.torch_ext().released_bytes(0)
+    out = sliding_two_simplicial_attn(ts[0], (ts[1], ts[2]), (ts[3], ts[4]), w1=32, w2=2)
+    del out
+    before = live()
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    try:
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (4 << 20)) / total)
+        with pytest.raises(torch.OutOfMemoryError):
+            if python_form:
+                _native.torch_ext().attend_forward(*ts, 32, 2, None, True, partials_budget.admit)
+            else:
+                sliding_two_simplicial_attn(ts[0], (ts[1], ts[2]), (ts[3], ts[4]), w1=32, w2=2)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert live() == before
