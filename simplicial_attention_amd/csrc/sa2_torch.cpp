@@ -100,22 +100,18 @@ struct Geometry {
 
 struct Forward {
     Tensor q, k1, k2, v1, v2;          // the kernels' operands
-    Tensor out, lse, residual, t_save, m_save;
+    Tensor out, lse, residual, t_save, m_save, note;
     Tensor result;                     // out in the caller's type and head dimension
 };
 
-// a buffer that reports its bytes as released when its last tensor dies
-Tensor counted_buffer(int64_t bytes, const Tensor &like, int64_t counted) {
-    Tensor base = at::empty({bytes}, like.options().dtype(at::kByte));
-    void *ptr = base.data_ptr();
-    const int device = like.device().index();
-    return at::for_blob(ptr, {bytes})
-        .deleter([base, device, counted](void *) mutable {
-            base.reset();
-            g_released[device].fetch_add(counted);
-        })
-        .options(like.options().dtype(at::kByte))
-        .target_device(like.device())
+// An empty tensor that reports `counted` bytes as released when it dies.  It is saved beside the partials and shares their fate;
+// these are ordinary tensors, whose memory the allocator keeps for other streams where record_stream asks for it.
+Tensor release_note(const Tensor &partials, int64_t counted) {
+    const int device = partials.device().index();
+    return at::for_blob(partials.data_ptr(), {0})
+        .deleter([device, counted](void *) { g_released[device].fetch_add(counted); })
+        .options(partials.options())
+        .target_device(partials.device())
         .make_tensor();
 }
 
@@ -141,17 +137,18 @@ Forward run_forward(const Tensor &q, const Tensor &k1, const Tensor &k2, const T
     const sa2_problem prob = g.problem();
     sa2_saved saved{};
     // (a size of 0: the kernels of this head dimension keep none; asked last, so that nothing that fails stands between the
-    // admission and the buffer that reports its end)
+    // admission and the buffers that it is for)
     const int64_t t_bytes = sa2_saved_t_bytes(&prob), m_bytes = sa2_saved_m_bytes(&prob);
     const bool save = admit && t_bytes + m_bytes > 0 && (*admit)(t_bytes + m_bytes, (int)q.device().index()).cast<bool>();
     if (save) {
         try {
-            f.t_save = counted_buffer(t_bytes, q, t_bytes + m_bytes);
+            f.t_save = at::empty({t_bytes}, q.options().dtype(at::kByte));
+            f.m_save = at::empty({g.batch, g.heads, g.w2, g.seq}, f.lse.options());
+            f.note = release_note(f.t_save, t_bytes + m_bytes);
         } catch (...) {
-            g_released[q.device().index()].fetch_add(t_bytes + m_bytes);      // (no buffer: give the admitted bytes back)
+            g_released[q.device().index()].fetch_add(t_bytes + m_bytes);      // (nothing to hang the report on)
             throw;
         }
-        f.m_save = at::empty({g.batch, g.heads, g.w2, g.seq}, f.lse.options());
         saved = {f.t_save.data_ptr(), static_cast<float *>(f.m_save.data_ptr())};
     }
     const int64_t ws_bytes = sa2_fwd_workspace_bytes(&prob);
@@ -190,7 +187,7 @@ struct Attend : public torch::autograd::Function<Attend> {
     }
 
     // what the backward needs of a forward: tensors, and as numbers the geometry and the types of the inputs
-    static variable_list saved_of(const Forward &f) { return {f.q, f.k1, f.k2, f.v1, f.v2, f.out, f.lse, f.residual, f.t_save, f.m_save}; }
+    static variable_list saved_of(const Forward &f) { return {f.q, f.k1, f.k2, f.v1, f.v2, f.out, f.lse, f.residual, f.t_save, f.m_save, f.note}; }
     static std::vector<int64_t> sizes_of(const Geometry &g, const std::array<const Tensor *, 5> &inputs) {
         std::vector<int64_t> n{g.batch, g.seq, g.heads, g.kv_heads, g.dim_qk, g.dim_v, g.dim, g.w1, g.w2};
         for (const Tensor *t : inputs) n.push_back((int64_t)t->scalar_type());

@@ -100,3 +100,44 @@ def test_a_forward_that_fails_leaves_the_budget_of_saved_partials_whole(python_f
     finally:
         torch.cuda.set_per_process_memory_fraction(1.0)
     assert live() == before
+
+
+def test_saved_partials_outlive_their_use_on_another_stream():
+    """A saved-tensor hook that copies on a stream of its own and calls record_stream: the allocator hands the memory out again only
+    when that stream has got there."""
+    ts = [torch.randn(1, 512, h, 64, device='cuda', dtype=torch.bfloat16).requires_grad_() for h in (2, 2, 2, 2, 2)]
+    side, taken = torch.cuda.Stream(), []
+
+    def pack(t):
+        with torch.cuda.stream(side):
+            torch.cuda._sleep(50_000_000)      # (tens of milliseconds: the stream is behind for the rest of the test)
+        t.record_stream(side)
+        taken.append((t.data_ptr(), t.untyped_storage().nbytes()))
+        return t.shape
+
+    with torch.autograd.graph.saved_tensors_hooks(pack, lambda shape: None):
+        out = _attend(*ts)
+    largest = max(size for _, size in taken)
+    places = {ptr for ptr, size in taken if size == largest}       # (the partials: w2 times the size of q)
+    del out
+    again = [torch.empty(largest, dtype=torch.uint8, device='cuda') for _ in range(3)]
+    assert not side.query()
+    assert not places & {t.data_ptr() for t in again}
+    torch.cuda.synchronize()
+
+
+def test_partials_are_counted_while_they_are_saved():
+    from simplicial_attention_amd import _native
+    from simplicial_attention_amd.two_simplicial_attention import partials_budget
+    live = lambda: partials_budget.live.get(0, 0) - _native.torch_ext().released_bytes(0)
+    ts = _inputs(grad=True)
+    before = live()
+    out = _attend(*ts)
+    assert live() - before == 2 * 9 * 96 * (64 * 2 + 4)            # heads, offsets, rows of 64 bf16 values and a reference each
+    torch.autograd.grad(out.sum(), ts, retain_graph=True)
+    assert live() > before
+    torch.autograd.grad(out.sum(), ts)
+    assert live() == before
+    out = _attend(*ts)
+    del out
+    assert live() == before
