@@ -208,6 +208,17 @@ static double finish_time(double groups, double longest, double total) {
 // took 29 us unsplit.
 static constexpr int kRoundEnd = 3, kQueryCost = 6;
 static constexpr int64_t kQueryPartBytes = 128ll << 20;
+// Every split of the backward has scatter rows of its own, as many as the second window is long even where the sequence is shorter
+// (2 heads of 96 rows, w2 = 10^6, D = 64: 3 GiB each); splits that would take more than this together are not made.
+static constexpr int64_t kScatterPartBytes = 1ll << 30;
+
+// rows below a 32-row query tile that its offsets reach (offsets run in rounds of eight)
+static int q_halo(int w2) { return 8 * ((w2 + 7) / 8) - 1; }
+
+// partial rows of dK2 and dV2 (the dV2 half is not needed with saved forward partials)
+static int64_t partial_rows_bytes(const sa2_problem *prob) {
+    return sa2::qk2_ws_floats(prob->batch, prob->heads, prob->seq_len, prob->dim_head, 32 + q_halo(prob->w2)) * 4;
+}
 
 static int64_t q_parts_bytes(const sa2_problem *prob, int splits) {
     return (int64_t)splits * prob->batch * prob->heads * prob->seq_len * prob->dim_head * 4;
@@ -215,7 +226,8 @@ static int64_t q_parts_bytes(const sa2_problem *prob, int splits) {
 
 // `shared`: two workgroups of the kernel fit a CU and together finish 1.4 times the work of one (the forward at D = 32
 // and 64), so up to two workgroups per CU run at once and each takes 1.45 times as long.
-static int q_splits(const sa2_problem *prob, int merge_cost, bool shared) {
+// `scatter_bytes`: scatter rows of one split
+static int q_splits(const sa2_problem *prob, int merge_cost, bool shared, int64_t scatter_bytes) {
     if (prob->dim_head == kWideDimHead) return 1;
     const int ntile = (prob->seq_len + 31) / 32;
     const double heads = (double)prob->batch * prob->heads;
@@ -237,7 +249,7 @@ static int q_splits(const sa2_problem *prob, int merge_cost, bool shared) {
     int best = 1;
     double best_cost = 0;
     for (int splits = 1; splits <= rounds; ++splits) {
-        if (splits > 1 && q_parts_bytes(prob, splits) > kQueryPartBytes) break;
+        if (splits > 1 && (q_parts_bytes(prob, splits) > kQueryPartBytes || splits * scatter_bytes > kScatterPartBytes)) break;
         double total = 0, longest = 0, groups = 0;
         for (int x = 0; x < ncls; ++x) {
             const int r = cls[x].rounds, n = splits < r ? splits : r;
@@ -258,8 +270,8 @@ static int q_splits(const sa2_problem *prob, int merge_cost, bool shared) {
     return best;
 }
 
-static int fwd_splits(const sa2_problem *prob) { return q_splits(prob, 8, prob->dim_head != 128); }   // (the merge is a launch of its own)
-static int bwd_splits(const sa2_problem *prob) { return q_splits(prob, 2, false); }
+static int fwd_splits(const sa2_problem *prob) { return q_splits(prob, 8, prob->dim_head != 128, 0); }   // (the merge is a launch of its own)
+static int bwd_splits(const sa2_problem *prob) { return q_splits(prob, 2, false, partial_rows_bytes(prob)); }
 
 // dim_head 128: one wave per SIMD with two offsets each; 64 and 32: two workgroups of eight waves per CU
 static void launch_fwd(int dim_head, bool split, int grid, hipStream_t s, const sa2::KParams &k) {
@@ -390,14 +402,6 @@ static int bwd_pass_filter() {
     if (v && std::strcmp(v, "first") == 0) return 1;
 #endif
     return 0;
-}
-
-// rows below a 32-row query tile that its offsets reach (offsets run in rounds of eight)
-static int q_halo(int w2) { return 8 * ((w2 + 7) / 8) - 1; }
-
-// partial rows of dK2 and dV2 (the dV2 half is not needed with saved forward partials)
-static int64_t partial_rows_bytes(const sa2_problem *prob) {
-    return sa2::qk2_ws_floats(prob->batch, prob->heads, prob->seq_len, prob->dim_head, 32 + q_halo(prob->w2)) * 4;
 }
 
 static int64_t max64(int64_t a, int64_t b) { return a > b ? a : b; }

@@ -283,6 +283,19 @@ def test_saved_partials_budget_is_global_per_device(monkeypatch):
     assert not _PartialsBudget().admit(3 * gib, 'cuda:0', total)
 
 
+@pytest.mark.parametrize('shape', [(1, 96, 2, 1, 64, 512, 1_000_000), (1, 256, 8, 8, 128, 256, 40_000), (4, 64, 1, 1, 32, 64, 200_000),
+                                   (1, 4096, 1, 1, 128, 512, 1024), (1, 128, 4, 4, 32, 128, 128)])
+def test_scratch_of_shared_grids_is_bounded(lib, shape):
+    """Workgroups that share a query tile each have scatter rows of their own: together they stay near a GiB where one set is smaller,
+    and long second windows ask for no more than undivided tiles."""
+    b, n, h, hk, d, w1, w2 = shape
+    prob = _native.problem(b, n, h, hk, d, w1, w2, True, d ** -0.5)
+    for with_saved in (0, 1):
+        undivided = lib.sa2_bwd_workspace_bytes_with_saved(prob) if with_saved else lib.sa2_bwd_workspace_bytes(prob)
+        shared = lib.sa2_bwd_split_workspace_bytes(prob, with_saved)
+        assert undivided <= shared <= max(undivided, (1 << 30) + (128 << 20))
+
+
 def test_signed_determinant_is_the_triple_product_of_channel_triples():
     """simplicial_attention.py:36-76: every triple of channels contributes det[q; k1; k2]; pinned against
     torch.linalg.det, with left-over channels contributing their plain trilinear product."""
