@@ -70,7 +70,9 @@ typedef struct sa2_problem {
     int32_t dtype;      /* sa2_dtype of the activations */
 } sa2_problem;
 
-/* A (batch, seq, heads, dim_head) activation: base pointer and element strides. */
+/* A (batch, seq, heads, dim_head) activation: base pointer and element strides.  The rows of an operand that the kernels read
+ * (q, k1, k2, v1, v2, dout, where there is more than one) are 0 to SA2_MOST_STRIDE_N elements apart. */
+#define SA2_MOST_STRIDE_N (1ll << 25)
 typedef struct sa2_tensor {
     void   *ptr;
     int64_t stride_b;

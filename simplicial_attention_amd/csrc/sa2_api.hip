@@ -63,6 +63,15 @@ int check_tensor(const sa2_tensor *t, const char *name) {
     return SA2_OK;
 }
 
+// The kernels address a row inside a 32-row tile of an operand by 32 bits: its stride is bounded (by 64 MiB)
+int check_operand(const sa2_problem *p, const sa2_tensor *t, const char *name) {
+    const int rc = check_tensor(t, name);
+    if (rc == SA2_OK && p->seq_len > 1 && (t->stride_n < 0 || t->stride_n > SA2_MOST_STRIDE_N))
+        return fail(SA2_ERR_BAD_SHAPE, "tensor %s: rows are %lld elements apart, 0 to %lld are supported", name, (long long)t->stride_n,
+                    (long long)SA2_MOST_STRIDE_N);
+    return rc;
+}
+
 sa2::DevTensor dev(const sa2_tensor *t) {
     sa2::DevTensor d;
     d.ptr = static_cast<char *>(t->ptr);
@@ -297,11 +306,11 @@ int sa2_fwd_ws(const sa2_problem *prob, const sa2_tensor *q, const sa2_tensor *k
                float *lse, const sa2_saved *saved, void *workspace, int64_t workspace_bytes, void *hip_stream) {
     SA2_TRY(check_problem(prob));
     if (out_residual) SA2_TRY(check_tensor(out_residual, "out_residual"));
-    SA2_TRY(check_tensor(q, "q"));
-    SA2_TRY(check_tensor(k1, "k1"));
-    SA2_TRY(check_tensor(k2, "k2"));
-    SA2_TRY(check_tensor(v1, "v1"));
-    SA2_TRY(check_tensor(v2, "v2"));
+    SA2_TRY(check_operand(prob, q, "q"));
+    SA2_TRY(check_operand(prob, k1, "k1"));
+    SA2_TRY(check_operand(prob, k2, "k2"));
+    SA2_TRY(check_operand(prob, v1, "v1"));
+    SA2_TRY(check_operand(prob, v2, "v2"));
     SA2_TRY(check_tensor(out, "out"));
     if (!lse) return fail(SA2_ERR_NULL_POINTER, "lse is NULL");
     if ((reinterpret_cast<uintptr_t>(workspace) & 15) != 0) return fail(SA2_ERR_ALIGNMENT, "workspace must be 16-byte aligned");
@@ -373,12 +382,12 @@ static int bwd_common(const sa2_problem *prob, const sa2_tensor *q, const sa2_te
                       const sa2_tensor *v1, const sa2_tensor *v2, const sa2_tensor *dout, const float *lse,
                       const float *delta, sa2::KParams *k) {
     SA2_TRY(check_problem(prob));
-    SA2_TRY(check_tensor(q, "q"));
-    SA2_TRY(check_tensor(k1, "k1"));
-    SA2_TRY(check_tensor(k2, "k2"));
-    SA2_TRY(check_tensor(v1, "v1"));
-    SA2_TRY(check_tensor(v2, "v2"));
-    SA2_TRY(check_tensor(dout, "dout"));
+    SA2_TRY(check_operand(prob, q, "q"));
+    SA2_TRY(check_operand(prob, k1, "k1"));
+    SA2_TRY(check_operand(prob, k2, "k2"));
+    SA2_TRY(check_operand(prob, v1, "v1"));
+    SA2_TRY(check_operand(prob, v2, "v2"));
+    SA2_TRY(check_operand(prob, dout, "dout"));
     if (!lse) return fail(SA2_ERR_NULL_POINTER, "lse is NULL");
     if (!delta) return fail(SA2_ERR_NULL_POINTER, "delta is NULL");
     *k = base_params(prob);

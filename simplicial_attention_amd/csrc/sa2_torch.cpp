@@ -41,9 +41,9 @@ void *stream_of(const Tensor &t) { return c10::hip::getCurrentHIPStreamMasquerad
 
 sa2_tensor arg(const Tensor &t) { return {t.data_ptr(), t.stride(0), t.stride(1), t.stride(2)}; }
 
-// the kernels need a unit innermost stride, 16-byte aligned rows and base
+// the kernels need a unit innermost stride, 16-byte aligned rows and base, rows within reach of each other
 Tensor aligned(const Tensor &t) {
-    const bool ok = t.stride(3) == 1 && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 && t.stride(0) % 8 == 0 && t.stride(1) % 8 == 0 &&
+    const bool ok = t.stride(3) == 1 && (t.size(1) == 1 || t.stride(1) <= SA2_MOST_STRIDE_N) && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 && t.stride(0) % 8 == 0 && t.stride(1) % 8 == 0 &&
                     t.stride(2) % 8 == 0;
     return ok ? t : t.clone(at::MemoryFormat::Contiguous);
 }

@@ -283,6 +283,23 @@ def test_saved_partials_budget_is_global_per_device(monkeypatch):
     assert not _PartialsBudget().admit(3 * gib, 'cuda:0', total)
 
 
+@pytest.mark.parametrize('d', [64, 128, 256])
+def test_rows_beyond_the_reach_of_the_kernels_are_refused(lib, d):
+    """32-bit addresses inside a 32-row tile: operands whose rows lie further apart are refused before a launch."""
+    prob = _native.problem(1, 64, 1, 1, d, 16, 4, True, 0.1)
+    t, lse = _dummy(), ctypes.c_void_p(0x2000)
+    need = lib.sa2_bwd_workspace_bytes(prob)
+    for stride in ((1 << 25) + 8, -8):
+        far = _native.TensorArg(0x1000, 0, stride, 0)
+        for place in range(5):
+            args = [t] * 5
+            args[place] = far
+            assert lib.sa2_fwd(prob, *args, t, None, lse, None, None) == 2
+            assert lib.sa2_bwd_dkv1(prob, *args, t, lse, lse, t, t, None) == 2
+            assert lib.sa2_bwd(prob, *args, t, None, t, lse, None, lse, t, t, t, t, t, lse, need, None) == 2
+        assert lib.sa2_bwd(prob, t, t, t, t, t, t, None, far, lse, None, lse, t, t, t, t, t, lse, need, None) == 2
+
+
 @pytest.mark.parametrize('shape', [(1, 96, 2, 1, 64, 512, 1_000_000), (1, 256, 8, 8, 128, 256, 40_000), (4, 64, 1, 1, 32, 64, 200_000),
                                    (1, 4096, 1, 1, 128, 512, 1024), (1, 128, 4, 4, 32, 128, 128)])
 def test_scratch_of_shared_grids_is_bounded(lib, shape):

@@ -237,6 +237,25 @@ def test_strided_views_need_no_copy():
         assert torch.equal(gpk.view(b, n, h, 5, d)[:, :, :, x], grads_c[x])
 
 
+@pytest.mark.parametrize('d', [64, 256])
+def test_rows_far_apart(d):
+    """Rows further apart than 32 bits reach from the first to the last of a tile: the operands are copied, the result is the same."""
+    from simplicial_attention_amd import sliding_two_simplicial_attn
+    n, stride = 33, (1 << 26) + 64
+    buffer = torch.empty(32 * stride + 6 * d, dtype=torch.bfloat16, device='cuda')          # (4 GiB)
+    near = [t.cuda() for t in U.make_inputs(1, n, 1, 1, d, seed=3)]
+    far = []
+    for x, t in enumerate(near):
+        far.append(buffer.as_strided((1, n, 1, d), (stride * n, stride, d, 1), x * d).copy_(t))
+    results = []
+    for *ts, dout in (near, far):
+        ts = [t.detach().requires_grad_(True) for t in ts]
+        out = sliding_two_simplicial_attn(ts[0], (ts[1], ts[2]), (ts[3], ts[4]), w1=40, w2=5)
+        results.append((out, *torch.autograd.grad(out, ts, dout)))
+    for a, b in zip(*results):
+        assert torch.equal(a, b)
+
+
 def test_each_backward_entry_point_against_the_oracle():
     """sa2_bwd_delta, sa2_bwd_dq_dkv2 (with and without the forward's saved partials) and
     sa2_bwd_dkv1 called one by one through the C ABI, each output against the CPU oracle."""
