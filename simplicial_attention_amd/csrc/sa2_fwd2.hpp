@@ -22,9 +22,10 @@
 // compiler, which is told to keep MFMA results in ordinary registers (-amdgpu-mfma-vgpr-form: the VALU reads the logits at
 // once; left to itself it puts the results of every MFMA of a kernel of this size in accumulation registers and moves the
 // logits).  A row's
-// softmax reference M is fixed by the wave's first tile (the diagonal one, which every valid row attends) and moves only when
-// a row sum says that weights outgrew 2^90 (rare: the tile's logits are then formed again).  Lanes without a valid key
-// row (k < 0, a row beyond the sequence) compute on clamped rows; their sums are never taken.
+// softmax reference M is fixed by the wave's first tile (the diagonal one, which every valid row attends).  Where a row sum
+// says at the end that weights outgrew 2^90 (rare), the workgroup walks its rounds twice more: once for the largest logits of
+// the rows, once for the result.  Lanes without a valid key row (k < 0, a row beyond the sequence) compute on clamped rows;
+// their sums are never taken.
 #pragma once
 
 #include "sa2_acc.hpp"
@@ -526,8 +527,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
         // did a row sum of this workgroup outgrow the safe range?
         if (attempt) break;
         uint32_t *vote = reinterpret_cast<uint32_t *>(lds + C::VOTE);
-        if (lane == 0) vote[wave] = 0;
-        if (!(l < kBig)) vote[wave] = 1;
+        const bool outgrown = wave_any(!(l < kBig));
+        if (lane == 0) vote[wave] = outgrown;
         __syncthreads();
         if (!uniform((int)(vote[0] | vote[1] | vote[2] | vote[3]))) break;
         if (R > r_first + 4) {

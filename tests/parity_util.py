@@ -57,6 +57,31 @@ def hip_fwd_bwd(q, k1, k2, v1, v2, dout, w1, w2):
     return out.detach(), grads
 
 
+def hip_unshared_fwd_bwd(q, k1, k2, v1, v2, dout, w1, w2, use_saved, scale=None):
+    """Output, lse and gradients through sa2_fwd and sa2_bwd: one workgroup per query tile and key slab, however small the grid.
+    Everything that the kernels are to write starts as NaN."""
+    from simplicial_attention_amd import _native
+    lib, arg = _native.load(), _native.tensor_arg
+    b, n, h, d = q.shape
+    q, k1, k2, v1, v2, dout = (t.cuda() for t in (q, k1, k2, v1, v2, dout))
+    prob = _native.problem(b, n, h, k1.shape[2], d, w1, w2, True, d ** -0.5 if scale is None else scale)
+    assert lib.sa2_bwd_workspace_bytes(prob) > 0
+    nan = lambda shape, dtype=torch.bfloat16: torch.full(shape, float('nan'), dtype=dtype, device='cuda')
+    raw = lambda size: torch.full((size,), 0xFF, dtype=torch.uint8, device='cuda')
+    out, res, lse, delta = nan(q.shape), nan(q.shape), nan((b, h, n), torch.float32), nan((b, h, n), torch.float32)
+    grads = [nan(t.shape) for t in (q, k1, k2, v1, v2)]
+    t_save, m_save = raw(lib.sa2_saved_t_bytes(prob)), raw(lib.sa2_saved_m_bytes(prob))
+    saved = _native.saved_arg(t_save, m_save) if use_saved else None
+    ws = raw(lib.sa2_bwd_workspace_bytes(prob))
+    stream = torch.cuda.current_stream().cuda_stream
+    ins = [arg(t) for t in (q, k1, k2, v1, v2)]
+    _native.check(lib.sa2_fwd(prob, *ins, arg(out), arg(res), lse.data_ptr(), saved, stream))
+    _native.check(lib.sa2_bwd(prob, *ins, arg(out), arg(res), arg(dout), lse.data_ptr(), saved, delta.data_ptr(), *(arg(t) for t in grads),
+                              ws.data_ptr(), ws.numel(), stream))
+    torch.cuda.synchronize()
+    return out, lse, grads
+
+
 def compare(name, got, ref):
     got = got.detach().float().cpu()
     ref = ref.detach().float().cpu()

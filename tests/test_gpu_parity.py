@@ -87,9 +87,9 @@ def test_seeded_random_shapes_head_dimension_256(b, n, hq, hk, d, w1, w2):
 
 @pytest.mark.parametrize('d', [128, 256])
 def test_large_and_drifting_logits(d):
-    """Logits that grow along the sequence by far more than 2^64 per window: exercises
-    the paths of the forward that move the softmax reference point while accumulators
-    hold data.  q and k2 hold powers of two and the softmax scale is chosen so that
+    """Logits that grow along the sequence by far more than 2^64 per window: at D = 256 the forward's
+    softmax reference follows them while accumulators hold data, at D = 128 row sums come to 2^82
+    (test_weights_that_outgrow_the_reference goes beyond what the reference stands).  q and k2 hold powers of two and the softmax scale is chosen so that
     scale * log2(e) = 2^-4, so the bf16 operand q * k2 * scale * log2(e) that the kernels feed
     to the MFMA is exact and the large logits carry no operand-rounding error (which would
     otherwise dominate any comparison at this scale, for the reference's kernels as well:
@@ -114,6 +114,72 @@ def test_large_and_drifting_logits(d):
     row = U.compare('out', out, ref_out)
     assert row['bad'] == 0 and row['rel_fro'] <= 1e-2, row
     # gradients reach magnitudes of 30-60 here (k1 is scaled up to 24x): relative check only
+    for name, got, ref in zip(U.NAMES[1:], grads, ref_grads):
+        row = U.compare(name, got, ref)
+        print('  ', row, flush=True)
+        assert row['rel_fro'] <= 3e-2, row
+
+
+def _log2_reference_gap(q, k1, k2, scale, w1, w2, waves, per_wave, rounds_of_a_share):
+    """How far the largest logit of a row lies above the largest one of the tile that fixes its wave's softmax reference (log2):
+    the largest gap over all rows, waves and shares.  A wave's row sum is at least 2^gap there."""
+    import math
+    n = q.shape[1]
+    i, j = torch.arange(n).view(n, 1), torch.arange(n).view(1, n)
+    attended, diagonal = (j <= i) & (i - j < w1), (i // 32) == (j // 32)
+    tops, firsts = [], []
+    for dlt in range(w2):
+        a = q[0].double() * torch.roll(k2[0].double(), dlt, 0)                             # (n, h, d)
+        s = torch.einsum('ihd,jhd->hij', a, k1[0].double()) * scale * math.log2(math.e)
+        s = s.masked_fill(~attended | (i < dlt), float('-inf'))
+        tops.append(s.amax(-1))
+        firsts.append(s.masked_fill(~diagonal, float('-inf')).amax(-1))
+    rounds = (w2 + waves * per_wave - 1) // (waves * per_wave)
+    gap = 0.0
+    for r0 in range(0, rounds, rounds_of_a_share or rounds):
+        for wave in range(waves):
+            mine = [[dlt for dlt in range(r * waves * per_wave + wave * per_wave, r * waves * per_wave + (wave + 1) * per_wave) if dlt < w2]
+                    for r in range(r0, min(rounds, r0 + (rounds_of_a_share or rounds)))]
+            if not mine[0]:
+                continue
+            first = torch.stack([firsts[x] for x in mine[0]]).amax(0)
+            top = torch.stack([tops[x] for r in mine for x in r]).amax(0)
+            gap = max(gap, float((top - first)[first > float('-inf')].max()))
+    return gap
+
+
+@pytest.mark.parametrize('form', ['shared', 'unshared', 'unshared, saved'])
+@pytest.mark.parametrize('d,w2', [(32, 16), (64, 16), (64, 70), (128, 16), (128, 40), (128, 100)])
+def test_weights_that_outgrow_the_reference(d, w2, form):
+    """Logits that fall along the sequence by more than 2^90 between a row's earliest keys and its diagonal tile, which fixes the
+    softmax reference: the forward has to move it (at D = 32 and 64 within the tile that outgrew it, at D = 128 by walking all rounds
+    again, the restaged k2/v2 rows beyond the fourth among them).  Exact operands as in the test above."""
+    import math
+    b, n, h, w1 = 1, 224, 2, 96
+    scale = 2.0 ** -4 / math.log2(math.e)
+    g = torch.Generator().manual_seed(22)
+    q = torch.pow(2.0, torch.randint(-1, 2, (b, n, h, d), generator=g).float()).bfloat16()
+    k2 = torch.pow(2.0, torch.randint(0, 2, (b, n, h, d), generator=g).float()).bfloat16()
+    ramp = torch.linspace(32.0, 0.2, n).view(1, n, 1, 1) * (128 / d)
+    k1 = (torch.randn(b, n, h, d, generator=g).abs() * ramp).bfloat16()
+    v1, v2, dout = [torch.randn(b, n, h, d, generator=g).bfloat16() for _ in range(3)]
+    gap = _log2_reference_gap(q, k1, k2, scale, w1, w2, *((4, 2) if d == 128 else (8, 1)), 1 if form == 'shared' else 0)
+    assert gap > 91.0, gap
+    print(f'\ncase d={d} w2={w2} {form}: 2^{gap:.0f}', flush=True)
+    f64 = lambda t: t.double()
+    ref_out, ref_lse, ref_grads = R.windowed_banded_fwd_bwd(f64(q), f64(k1), f64(k2), f64(v1), f64(v2), f64(dout), w1, w2, scale=scale)
+    if form == 'shared':
+        from simplicial_attention_amd import SlidingTwoSimplicialAttention
+        ts = [t.cuda().requires_grad_(True) for t in (q, k1, k2, v1, v2)]
+        out = SlidingTwoSimplicialAttention.apply(*ts, w1, w2, True, scale)
+        grads = torch.autograd.grad(out, ts, dout.cuda())
+    else:
+        out, lse, grads = U.hip_unshared_fwd_bwd(q, k1, k2, v1, v2, dout, w1, w2, form != 'unshared', scale)
+        assert torch.allclose(lse.cpu().double(), ref_lse, atol=2e-2, rtol=1e-6)
+    row = U.compare('out', out, ref_out)
+    print('  ', row, flush=True)
+    assert row['bad'] == 0 and row['rel_fro'] <= 1e-2, row
+    # (gradients as large as k1: relative check only)
     for name, got, ref in zip(U.NAMES[1:], grads, ref_grads):
         row = U.compare(name, got, ref)
         print('  ', row, flush=True)
