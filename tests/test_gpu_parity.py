@@ -186,6 +186,21 @@ def test_weights_that_outgrow_the_reference(d, w2, form):
         assert row['rel_fro'] <= 3e-2, row
 
 
+@pytest.mark.parametrize('saved', [False, True], ids=['recomputed', 'saved'])
+@pytest.mark.parametrize('d', [32, 64, 128])
+@pytest.mark.parametrize('n,hq,hk,w1,w2', [(200, 2, 1, 70, 65), (260, 1, 1, 40, 100), (290, 2, 2, 290, 128)])
+def test_long_second_windows_in_one_workgroup(n, hq, hk, w1, w2, d, saved):
+    """Grids as small as these are shared out by the wrapper until a workgroup walks a round or three; larger ones are not.  Nine to
+    sixteen rounds in one workgroup: the 64-row k2/v2 buffers refilled several times over, three and four blocks of offsets per
+    key slab."""
+    print(f'\ncase n={n} hq={hq} hk={hk} d={d} w1={w1} w2={w2} saved={saved}', flush=True)
+    ins = U.make_inputs(1, n, hq, hk, d, seed=n + d + w2, std=d ** -0.5)
+    ref_out, ref_lse, ref_grads = U.oracle_fwd_bwd(*ins, w1, w2)
+    out, lse, grads = U.hip_unshared_fwd_bwd(*ins, w1, w2, saved)
+    assert torch.allclose(lse.cpu(), ref_lse, atol=2e-2, rtol=1e-2)
+    U.check_all(out, grads, ref_out, ref_grads)
+
+
 @pytest.mark.parametrize('std', [0.5, 1.0])
 def test_degenerate_windows_attend_only_self(std):
     """w1 = w2 = 1: every row attends (i, i) only, so out_i = v1_i * v2_i and
