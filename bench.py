@@ -132,9 +132,9 @@ def kernel_symbol(entry, D, w2):
     if D == 256:
         return {'fwd': 'sa2::fwd_wide_kernel<256>', 'bwd_dq_dk2_pass': 'sa2::bwd_wide_q_kernel<256, true>', 'bwd_dkv1': 'sa2::bwd_kvr_kernel<256, false>'}.get(entry)
     if entry == 'fwd':
-        return 'sa2::fwd2_kernel<128>' if D == 128 else 'sa2::fwd_kernel<%d>' % D
+        return 'sa2::fwd2_kernel<128, false>' if D == 128 else 'sa2::fwd_kernel<%d, false>' % D
     if entry == 'bwd_dq_dk2_pass':
-        return 'sa2::bwd_q_kernel<%d, true>' % D
+        return 'sa2::bwd_q_kernel<%d, true, false>' % D
     if entry == 'bwd_dkv1':
         # (the entry point sa2_bwd_dkv1 has no workspace and always runs one workgroup per key slab: PARTS = false)
         return 'sa2::bwd_kv8_kernel<%d, %d, false>' % (D, 3 if D == 128 else 2)

@@ -26,22 +26,21 @@ namespace sa2 {
 
 template <int D>
 struct KvrCfg {
+    static_assert(D == 256, "two waves per SIMD are faster at smaller head dimensions (bwd_kv8_kernel)");
     static constexpr int KS = D / 16, DT = D / 32;
     using T = DmaTile<D>;
-    static constexpr int OP = 256 / D;                 // offsets per step
     static constexpr int CPW = T::NCH / 4;             // chunks of a tile that a wave builds
-    static constexpr int NPROD = 2 * OP * CPW;         // products per thread and step
+    static constexpr int NPROD = 2 * CPW;              // products per thread and step
     static constexpr int NSLOT = 48;                   // k2 / v2 rows, circular
     static constexpr int NRC = NSLOT / T::RPC;         // their chunks
-    // staging in the first 64 KiB (direct loads): q pieces, k2 rows, v2 rows, do pieces (D = 256: beyond it)
+    // staging in the first 64 KiB (direct loads): q pieces, k2 rows, v2 rows; do pieces beyond it
     static constexpr int QS = 0;
     static constexpr int RK = QS + T::NCH * 1024;
     static constexpr int RV = RK + NRC * 1024;
     static constexpr int DOS = RV + NRC * 1024;
-    static constexpr int OPS = DOS + T::NCH * 1024;    // operand tiles [offset][A, B]; two buffers
-    static constexpr bool DO_DIRECT = OPS <= 65536;
+    static constexpr int OPS = DOS + T::NCH * 1024;    // operand tiles A, B; two buffers
     static_assert(DOS <= 65536, "the LDS address of a direct load travels in 16 bits of M0");
-    static constexpr int STEP = 2 * OP * T::BYTES;
+    static constexpr int STEP = 2 * T::BYTES;
     static constexpr int TAB = OPS + 2 * STEP;         // -lse log2(e) [32], -delta [32]
     static constexpr int LDS = TAB + 256;
     static_assert(LDS <= 160 * 1024, "LDS of a CU");
@@ -51,8 +50,7 @@ template <int D, bool PARTS>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void bwd_kvr_kernel(KParams p) {
     using C = KvrCfg<D>;
     using T = typename C::T;
-    constexpr int KS = C::KS, DT = C::DT, RPC = T::RPC, CPW = C::CPW, OP = C::OP;
-    constexpr bool ACC = D == 256;                     // dK1 in accumulation registers
+    constexpr int KS = C::KS, DT = C::DT, RPC = T::RPC, CPW = C::CPW;
     __shared__ __attribute__((aligned(16))) char lds[C::LDS];
 
     const int N = p.N;
@@ -100,11 +98,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
             vf[kk] = ld_global16(vrow + 32 * kk);
         }
     }
-    f32x16 dK[DT], dV[DT];
+    f32x16 dK[DT], dV[DT];                             // (dK1 in accumulation registers)
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) {
         dK[dt] = dV[dt] = zero16();
-        if constexpr (ACC) pin_acc(dK[dt]);
+        pin_acc(dK[dt]);
     }
 
     // ---- the walk: query heads of the group, query tiles, offsets
@@ -115,11 +113,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     // to the next step; false behind the last one of this workgroup's share
     auto advance = [&](Step &s) {
         const int top = last_offset(s.it);
-        if (OP > 1 || (s.dlt & 1) || s.dlt == top) {
+        if ((s.dlt & 1) || s.dlt == top) {
             if (--pairs_left == 0) return false;
         }
-        s.dlt += OP;
-        if (s.dlt > top) {
+        if (++s.dlt > top) {
             s.dlt = 0;
             if (++s.it > it_end) {
                 s.it = it_begin;
@@ -142,7 +139,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
         load_to_lds16(uniform(g + (int64_t)base * sn), (uint32_t)((clamp_row(first + l_row) - base) * (int)sn + l_col),
                       uniform((int)(lds0 + ring + chunk * 1024)));
     };
-    // what the builds of query tile s.it from offset s.dlt on read: q (and do) pieces, 48 rows of k2 and v2 (no build may be
+    // what the builds of query tile s.it from offset s.dlt on read: q pieces, 48 rows of k2 and v2 (no build may be
     // reading); the start values of its chains on their way to LDS
     float start = 0.f;
     auto stage = [&](const Step &s) {
@@ -154,15 +151,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
             const int ch = wave + 4 * n;
             load_to_lds16(uniform(qg + (int64_t)base * p.q.sn), (uint32_t)((clamp_row(i0 + ch * RPC + l_row) - base) * (int)p.q.sn + l_col),
                           uniform((int)(lds0 + C::QS + ch * 1024)));
-        }
-        if constexpr (C::DO_DIRECT) {
-            const char *dog = p.dout.ptr + b * p.dout.sb + h * p.dout.sh;
-#pragma unroll
-            for (int n = 0; n < CPW; ++n) {
-                const int ch = wave + 4 * n;
-                load_to_lds16(uniform(dog + (int64_t)base * p.dout.sn), (uint32_t)((clamp_row(i0 + ch * RPC + l_row) - base) * (int)p.dout.sn + l_col),
-                              uniform((int)(lds0 + C::DOS + ch * 1024)));
-            }
         }
         if (tid < 64) {
             const int64_t row = ((int64_t)b * p.H + h) * N + clamp_row(i0 + c);
@@ -177,41 +165,38 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     };
     // the rest of it (every wave has left the tile before)
     auto stage_rest = [&](const Step &s) {
-        if constexpr (!C::DO_DIRECT) {
-            const int h = hk * p.G + s.g, i0 = 32 * s.it;
-            const char *dog = p.dout.ptr + b * p.dout.sb + h * p.dout.sh;
-            u32x4 x[CPW];
+        const int h = hk * p.G + s.g, i0 = 32 * s.it;
+        const char *dog = p.dout.ptr + b * p.dout.sb + h * p.dout.sh;
+        u32x4 x[CPW];
 #pragma unroll
-            for (int n = 0; n < CPW; ++n) x[n] = ld_global16(dog + (int64_t)clamp_row(i0 + (wave + 4 * n) * RPC + l_row) * p.dout.sn + l_col);
+        for (int n = 0; n < CPW; ++n) x[n] = ld_global16(dog + (int64_t)clamp_row(i0 + (wave + 4 * n) * RPC + l_row) * p.dout.sn + l_col);
 #pragma unroll
-            for (int n = 0; n < CPW; ++n) *reinterpret_cast<u32x4 *>(lds + C::DOS + (wave + 4 * n) * 1024 + lane * 16) = x[n];
-        }
+        for (int n = 0; n < CPW; ++n) *reinterpret_cast<u32x4 *>(lds + C::DOS + (wave + 4 * n) * 1024 + lane * 16) = x[n];
         if (tid < 64) reinterpret_cast<float *>(lds + C::TAB)[tid] = start;
     };
     // a step is built: the k2 / v2 rows that no later offset of the tile reaches make room for those 48 below
     auto refill = [&](const Step &s) {
-        if ((s.dlt + OP) % RPC != 0 || wave > 1) return;
-        const int first = 32 * s.it + 32 - (s.dlt + OP) - C::NSLOT;
+        if ((s.dlt + 1) % RPC != 0 || wave > 1) return;
+        const int first = 32 * s.it + 32 - (s.dlt + 1) - C::NSLOT;
         if (wave == 0) load_ring(k2g, p.k2.sn, C::RK, first);
         else load_ring(v2g, p.v2.sn, C::RV, first);
     };
 
-    // ---- operand build: product x of a thread is a piece of A (even x) or B (odd x) of offset x / (2 CPW), chunk
-    // wave + 4 (x / 2 % CPW)
+    // ---- operand build: product x of a thread is a piece of A (even x) or B (odd x), chunk wave + 4 (x / 2)
     const float c2 = p.scale_log2e;
     u32x4 bx, by, bz;
     // place of the lane's piece of chunk `wave`, row - offset, in a circular buffer (chunk wave + 4 n: 4096 n bytes on)
-    int shift = 0;                                     // slot of row 0 of the first offset being built
+    int shift = 0;                                     // slot of row 0 of the offset being built
     uint32_t at = 0;
     auto build_begin = [&](const Step &s) {
         shift = (32 * s.it - s.dlt) % C::NSLOT;
         shift = uniform(shift < 0 ? shift + C::NSLOT : shift);
     };
     auto build_read = [&](auto x_) {
-        constexpr int x = decltype(x_)::value, n = x / 2 % CPW, o = x / (2 * CPW);
+        constexpr int x = decltype(x_)::value, n = x / 2;
         constexpr uint32_t ring = C::NRC * 1024;
-        if constexpr (x % (2 * CPW) == 0) {
-            const int slot = wave * RPC + (shift >= o ? shift - o : shift - o + C::NSLOT) + l_row;      // (below 2 * NSLOT)
+        if constexpr (x == 0) {
+            const int slot = wave * RPC + shift + l_row;      // (below 2 * NSLOT)
             at = (uint32_t)(slot / RPC * 1024 + slot % RPC * 64 + l_seg);
             at = at < at - ring ? at : at - ring;
         }
@@ -225,28 +210,25 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
         else bz[w] = pack_bf16(bf16_lo(bx[w]) * bf16_lo(by[w]), bf16_hi(bx[w]) * bf16_hi(by[w]));
     };
     auto build_write = [&](auto x_, char *dst) {
-        constexpr int x = decltype(x_)::value, n = x / 2 % CPW, o = x / (2 * CPW);
-        *reinterpret_cast<u32x4 *>(dst + (2 * o + (x & 1)) * T::BYTES + (wave + 4 * n) * T::CP + lane * 16) = bz;
+        constexpr int x = decltype(x_)::value, n = x / 2;
+        *reinterpret_cast<u32x4 *>(dst + (x & 1) * T::BYTES + (wave + 4 * n) * T::CP + lane * 16) = bz;
     };
-    auto build = [&](auto from, auto to, char *dst) {
-        static_for<decltype(from)::value, decltype(to)::value>([&](auto x) {
+    auto build = [&](char *dst) {
+        static_for<0, C::NPROD>([&](auto x) {
             build_read(x);
 #pragma unroll
             for (int w = 0; w < 4; ++w) build_word(x, w);
             build_write(x, dst);
         });
     };
-    constexpr std::integral_constant<int, 0> all_from{};
-    constexpr std::integral_constant<int, C::NPROD> all_to{};
 
     const int r_lane = T::row_lane(lane), t_lane = T::tr_lane(lane);
-    // offset s.dlt + O of a step; `dst`: where the operand tiles of the next step are built meanwhile (this offset's share of them)
-    auto compute = [&](auto o_, const Step &s, const char *ops, char *dst) {
-        constexpr int O = decltype(o_)::value;
+    // one step; `dst`: where the operand tiles of the next one are built meanwhile
+    auto compute = [&](const Step &s, const char *ops, char *dst) {
         constexpr int W = 6, NROW = 2 * KS, TRA = NROW + 2 * DT, NFR = TRA + 2 * DT;
-        constexpr int PROD0 = O * C::NPROD / OP, EVERY = NFR * OP / C::NPROD;
-        static_assert(EVERY == 8 && NFR * OP == C::NPROD * EVERY, "a product rides behind eight MFMAs");
-        const char *ra = ops + 2 * O * T::BYTES + r_lane, *rb = ra + T::BYTES, *ta = ops + 2 * O * T::BYTES + t_lane, *tb = ta + T::BYTES;
+        constexpr int EVERY = NFR / C::NPROD;
+        static_assert(EVERY == 8 && NFR == C::NPROD * EVERY, "a product rides behind eight MFMAs");
+        const char *ra = ops + r_lane, *rb = ra + T::BYTES, *ta = ops + t_lane, *tb = ta + T::BYTES;
         // A rows, B rows, B transposed, A transposed
         auto fragment = [&](auto idx) {
             constexpr int x = decltype(idx)::value;
@@ -277,7 +259,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
             Y[4 * q4 + 3] = d.w;
         }
         static_for<0, W>([&](auto x) { f[x] = fragment(x); });
-        const int i0 = 32 * s.it, dlt = s.dlt + O;
+        const int i0 = 32 * s.it, dlt = s.dlt;
         if (!(i0 >= jw + 31 && i0 + 31 - jw < w1 && i0 >= dlt)) {
             // attended rows i: max(j, dlt) <= i < j + w1 (register e holds row i0 + 4 hf + 8 (e / 4) + e % 4)
             const int from = j > dlt ? j : dlt, span = j + w1 > from ? j + w1 - from : 0;
@@ -299,13 +281,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
             if constexpr (x < KS) X = mfma32(f[x % W], kf[x], X);
             else if constexpr (x < NROW) Y = mfma32(f[x % W], vf[x - KS], Y);
             else if constexpr (x < TRA) dV[(x - NROW) % DT] = mfma32(f[x % W], pb[(x - NROW) / DT], dV[(x - NROW) % DT]);
-            else if constexpr (ACC) mfma32_acc(dK[(x - TRA) % DT], f[x % W], sb[(x - TRA) / DT]);
-            else dK[(x - TRA) % DT] = mfma32(f[x % W], sb[(x - TRA) / DT], dK[(x - TRA) % DT]);
+            else mfma32_acc(dK[(x - TRA) % DT], f[x % W], sb[(x - TRA) / DT]);
             if constexpr (x + W < NFR) f[x % W] = fragment(std::integral_constant<int, x + W>{});
             // the exponentials behind the chain of Y, dS behind the products of dV
             if constexpr (x >= KS + 2 && x < KS + 10) weights(2 * (x - KS - 2));
             if constexpr (x >= NROW + 2 && x < NROW + 10) slopes(2 * (x - NROW - 2));
-            constexpr std::integral_constant<int, PROD0 + x / EVERY> prod{};
+            constexpr std::integral_constant<int, x / EVERY> prod{};
             if constexpr (x % EVERY == 0) build_read(prod);
             if constexpr (x % EVERY >= 4) build_word(prod, x % EVERY - 4);
             if constexpr (x % EVERY == 7) build_write(prod, dst);
@@ -326,7 +307,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     wait_loads<0>();
     __syncthreads();
     build_begin(nb);
-    build(all_from, all_to, lds + C::OPS);
+    build(lds + C::OPS);
     __syncthreads();
     int buf = 0;
     bool more = true;
@@ -339,23 +320,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
         const char *ops = lds + C::OPS + (buf ? C::STEP : 0);
         char *dst = lds + C::OPS + (buf ? 0 : C::STEP);
         // (behind the last step and where the tile changes, what is built here is of no use: it is built again or not read)
-        if constexpr (decltype(on_)::value) {
-            const int top = last_offset(cur.it);
-            static_for<0, OP>([&](auto o) {
-                constexpr int O = decltype(o)::value, SHARE = C::NPROD / OP;
-                if (O == 0 || cur.dlt + O <= top) compute(o, cur, ops, dst);
-                else build(std::integral_constant<int, O * SHARE>{}, std::integral_constant<int, (O + 1) * SHARE>{}, dst);
-            });
-        } else {
-            build(all_from, all_to, dst);
-        }
+        if constexpr (decltype(on_)::value) compute(cur, ops, dst);
+        else build(dst);
         if (!more) return;
         wait_loads<0>();
         __syncthreads();
         if (turn) {
             stage_rest(nb);
             __syncthreads();
-            build(all_from, all_to, dst);
+            build(dst);
             __syncthreads();
         }
         buf ^= 1;
@@ -378,11 +351,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
         }
     }
 
-    if constexpr (ACC) {
-        acc_done();
+    acc_done();
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt) pin_acc(dK[dt]);
-    }
+    for (int dt = 0; dt < DT; ++dt) pin_acc(dK[dt]);
     if (!j_ok) return;
     // (A carried scale log2(e): times ln 2 gives the softmax scale)
     if constexpr (PARTS) {

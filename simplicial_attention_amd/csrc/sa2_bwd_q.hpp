@@ -170,16 +170,12 @@ __global__ __launch_bounds__(512) void bwd_q_kernel(KParams p, float *ws, int ha
             const u32x4 fd = ld_global16(dog + (int64_t)ii * p.dout.sn + col);
             *reinterpret_cast<u32x4 *>(lds + C::DOS + row * PITCH + col) = fd;
             if constexpr (DQ && SPLIT) {
-                if (p.o.ptr) {
-                    const u32x4 fo = ld_global16(p.o.ptr + b * p.o.sb + (int64_t)ii * p.o.sn + h * p.o.sh + col);
-                    const float part = delta_piece(fo, fd, p.o_lo.ptr ? p.o_lo.ptr + b * p.o_lo.sb + (int64_t)ii * p.o_lo.sn + h * p.o_lo.sh + col : nullptr);
-                    const float dsum = delta_row_sum<PPR>(part);
-                    if (col == 0) {
-                        delta_s[row] = dsum;
-                        if (split == 0 && i0 + row < N) p.delta[((int64_t)b * p.H + h) * N + i0 + row] = dsum;
-                    }
-                } else if (col == 0) {
-                    delta_s[row] = p.delta[((int64_t)b * p.H + h) * N + ii];
+                const u32x4 fo = ld_global16(p.o.ptr + b * p.o.sb + (int64_t)ii * p.o.sn + h * p.o.sh + col);
+                const float part = delta_piece(fo, fd, p.o_lo.ptr ? p.o_lo.ptr + b * p.o_lo.sb + (int64_t)ii * p.o_lo.sn + h * p.o_lo.sh + col : nullptr);
+                const float dsum = delta_row_sum<PPR>(part);
+                if (col == 0) {
+                    delta_s[row] = dsum;
+                    if (split == 0 && i0 + row < N) p.delta[((int64_t)b * p.H + h) * N + i0 + row] = dsum;
                 }
             }
         }

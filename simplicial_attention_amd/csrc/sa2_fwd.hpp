@@ -21,9 +21,9 @@
 //     value chain.
 // The output accumulator is shared: an fp32 [32][D] LDS buffer relative to a common reference
 // Mc.  At the end of a round the waves publish their references, agree on Mc = max, and add
-// v2_{i-dlt} * T * 2^(M - Mc) (formed in place in T first) in eight barrier-separated phases; in phase ph wave w owns the
-// d-slice (w + ph) mod 8, so concurrent waves never touch the same element and every element
-// sees its additions in a fixed order (bitwise reproducible, no atomics).
+// v2_{i-dlt} * T * 2^(M - Mc) in eight barrier-separated phases, in which groups of as many waves as there are slices
+// (D / 16) take turns: in its phases wave w of a group owns the d-slice (w + phase) mod (D / 16), so concurrent waves never touch
+// the same element and every element sees its additions in a fixed order (bitwise reproducible, no atomics).
 // The k2/v2 rows live in a 64-row circular LDS buffer (row k in slot (k - i0) mod 64), filled before the first round
 // with the rows k - i0 = -32 .. 31, which is all that second windows up to 32 ever read; a round needs 39 rows, and
 // from the fourth round on the 8 rows that the next round adds are fetched while the round's results are added to
@@ -241,12 +241,6 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(FwdCfg<D>::
         }
     };
 
-    // accumulator clears: as 64-bit moves where registers are plentiful (at four waves per SIMD the register pairs
-    // they need cost more in spilled registers than the moves save)
-    auto clear16 = [] {
-        if constexpr (C::WPE == 2) return zero16_pairs();
-        else return zero16();
-    };
     f32x16 T[DT];
     u32x4 A[KS];
     // Fragments travel through rolling windows of FW register sets: fragment f of a chain sits in set f % FW and is
@@ -315,7 +309,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(FwdCfg<D>::
                 }
             }
 #pragma unroll
-            for (int dt = 0; dt < DT; ++dt) T[dt] = clear16();
+            for (int dt = 0; dt < DT; ++dt) T[dt] = zero16();
         }
 
         // exponentials and row sums of the tile whose referenced logits are in X
@@ -411,7 +405,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(FwdCfg<D>::
                 // ---- the wave's very first step, the diagonal tile of its first offset: every valid row
                 // attends an entry of it, so this is where the rows get their softmax reference M
                 open_step();
-                f32x16 X = clear16();
+                f32x16 X = zero16();
                 logit_chain(X, std::false_type{});
                 {
                     // row j = 32 t + 4 hf + e (e = 8 (rr / 4) + rr % 4) is attended iff 0 <= i - j < w1;
@@ -442,14 +436,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(FwdCfg<D>::
             // subtraction code follows it.  A row's reference moves only if its row sum says that weights
             // outgrew the safe range.
             float nm = col_ok ? -M : -INFINITY;
-            // the chains' start value, kept in registers where they are plentiful (eight moves per step instead of sixteen)
-            f32x16 NMv;
-            if constexpr (C::WPE == 2) NMv = splat16(nm);
             u32x4 pb[2];
             for (; n < NT; ++n) {
-                f32x16 X;
-                if constexpr (C::WPE == 2) X = NMv;
-                else X = splat16(nm);
+                f32x16 X = splat16(nm);
                 if (n < n_masked) {
                     const char *mk = lds + C::MASKS + n * C::MASK + lane * 16;
 #pragma unroll
@@ -478,7 +467,6 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(FwdCfg<D>::
                     const float shift = over ? fmaxf(fmaxf(tmax, e_old), 0.f) : 0.f;
                     shift_reference(shift, fast_exp2(-shift), X);
                     nm = col_ok ? -M : -INFINITY;
-                    if constexpr (C::WPE == 2) NMv = splat16(nm);
                     exponentials(X, pb);
                 }
                 value_products(pb);
@@ -541,7 +529,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(FwdCfg<D>::
             // phases 2 DT g .. 2 DT g + 2 DT - 1 and its wave w the slice (w + ph) mod 2 DT in phase ph
             for (int ph = 0; ph < 8; ++ph) {
                 constexpr int NS = 2 * DT;
-                if (NS == 8 || ph / NS == wave / NS) with_slice<NS>(wave + ph, [&](auto tag) { add_slice(tag, ph % NS == 0 && (NS == 8 || wave / NS == 0)); });
+                if (ph / NS == wave / NS) with_slice<NS>(wave + ph, [&](auto tag) { add_slice(tag, ph % NS == 0 && wave / NS == 0); });
                 if (ph == 7 && adds_rows(r)) write_rows(r);  // (their slots are not in use in this round)
                 __syncthreads();
             }

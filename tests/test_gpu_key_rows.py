@@ -1,6 +1,6 @@
-"""The dK1/dV1 kernel of head dimensions 128 and 256 at the edges of its walk: second windows around the chunks and the 48 rows of
-its circular buffers, first windows around a tile, ragged last tiles and slabs, several query heads per key/value head, one
-workgroup per key slab and several."""
+"""The dK1/dV1 kernels of head dimensions 128 and 256 at the edges of their walks: second windows around the chunks and the 48 rows
+of the circular buffers (bwd_kvr_kernel, D = 256) and around blocks of 32 offsets (bwd_kv8_kernel, D = 128), first windows around a
+tile, ragged last tiles and slabs, several query heads per key/value head, one workgroup per key slab and several."""
 import pytest
 import torch
 
@@ -33,7 +33,8 @@ def test_against_oracle(b, n, hq, hk, w1, w2, d):
 
 @pytest.mark.parametrize('d', [32, 64, 128, 256])
 def test_several_workgroups_per_slab_against_one(d):
-    """The same sums in shares: fp32 partial sums in another order, rounded to bf16 once."""
+    """The same sums in shares (all gradients at D = 32 to 128, dK1 and dV1 at 256): fp32 partial sums in another order, rounded to
+    bf16 once."""
     from simplicial_attention_amd import _native
     lib = _native.load()
     b, n, h, hk, w1, w2 = 1, 700, 2, 1, 200, 21
@@ -55,7 +56,7 @@ def test_several_workgroups_per_slab_against_one(d):
         _native.check(call(prob, *(arg(t) for t in (q, k1, k2, v1, v2, out)), arg(lo), arg(dout), lse.data_ptr(), None, delta.data_ptr(),
                            *(arg(t) for t in (dq, dk1, dk2, dv1, dv2)), ws.data_ptr(), size, stream))
         torch.cuda.synchronize()
-        results.append((dk1.float(), dv1.float()))
+        results.append([t.float() for t in grads])
     for one, shares in zip(*results):
         # both are the bf16 rounding of fp32 sums that agree to about 1e-5: one bf16 step (2^-7) apart at most, 2^-9 on average
         assert bool(torch.isfinite(shares).all())
