@@ -42,7 +42,9 @@ extern "C" {
 /* 101: saved->t is kept in blocks of 32 rows (sa2_saved_t_bytes), the workspace rules of sa2_bwd_workspace_bytes*
  * cover the split key slabs, sa2_bwd checks every size before its first launch
  * 102: dim_head 256 (its kernels keep no forward partials: the sa2_saved_*_bytes queries return 0 and a non-NULL
- * `saved` is refused) */
+ * `saved` is refused)
+ * The number stands for what existing calls do.  Functions added beside them (sa2_fwd_ws, sa2_bwd_split, sa2_convert, sa2_wgrad and
+ * their size queries) leave it as it is: look them up by name. */
 #define SA2_VERSION 102
 
 typedef enum sa2_status {

@@ -485,8 +485,9 @@ static Kv8Plan kv8_plan(const sa2_problem *prob) {
             best_cost = cost;
         }
     }
-    // (the estimate charges whole rounds of the longest walk: short sequences whose last slabs meet fewer tiles end earlier in halves.
-    // 8 sequences of 2048 rows, 4 key/value heads, D = 64: forward and backward 3.04 ms in halves, 3.06 undivided)
+    // (where the estimate sees no gain, slabs are divided as sa2_bwd divides them, so that both entry points give the same bits there.  Not
+    // for speed: 8 sequences of 2048 rows, 4 key/value heads, D = 64, forward and backward take 3.04 ms in halves and 3.06 undivided, which is
+    // less than two runs differ by)
     return best.parts == 1 ? two_part_plan(prob) : best;
 }
 
