@@ -118,10 +118,9 @@ __global__ __launch_bounds__(512) void bwd_kv8_kernel(KParams p) {
     const int tile = item % ntile;
     const int bh = item / ntile;
     // this workgroup's share of the slab's walk: pairs pair0 .. pair0 + npairs - 1
-    const int head_pairs = kv8_walk_pairs(tile, N, p.w1, p.w2);
-    int pair0 = 0;
-    int npairs = head_pairs * p.G;
+    int head_pairs = 0, pair0 = 0, npairs = 0;
     if constexpr (PARTS) {
+        head_pairs = kv8_walk_pairs(tile, N, p.w1, p.w2);
         const int64_t all = (int64_t)head_pairs * p.G;
         const int parts = uniform(kv8_parts_of(all, p.kv_chunk, p.kv_max_parts));
         if (part >= parts) return;                    // (a slab with a short walk: the combine kernel knows)
@@ -202,6 +201,14 @@ __global__ __launch_bounds__(512) void bwd_kv8_kernel(KParams p) {
     auto next_pair = [&](Pair &s) {
         if (2 * (++s.m) > dmax_of(s.it, s.blk)) next_unit(s);
     };
+    // The whole walk is counted here, behind the loads of the prologue, by a loop of 32-bit steps: with the closed form (64 bits) the
+    // scalar registers run out and the D = 128 kernel spills 24 vector registers instead of 12 (5.05 against 4.96 ms at 4 x 8 x 8192
+    // rows, w1 512, w2 32)
+    if constexpr (!PARTS) {
+        for (int it = it_begin; it <= it_end; ++it)
+            for (int blk = 0; 32 * blk <= dtop_of(it); ++blk) npairs += dmax_of(it, blk) / 2 + 1;
+        npairs *= p.G;
+    }
     // ---- row staging: per (query head, query tile) the q/do rows and the k2/v2 rows go
     // global -> registers (a whole tile ahead) -> LDS
     u32x4 rows[L::RPT];
