@@ -132,7 +132,7 @@ def kernel_symbol(entry, D, w2):
     if D == 256:
         return {'fwd': 'sa2::fwd_wide_kernel<256>', 'bwd_dq_dk2_pass': 'sa2::bwd_wide_q_kernel<256, true>', 'bwd_dkv1': 'sa2::bwd_kvr_kernel<256, false>'}.get(entry)
     if entry == 'fwd':
-        return 'sa2::fwd2_kernel<128, false>' if D == 128 else 'sa2::fwd_kernel<%d, false>' % D
+        return 'sa2::fwd2_kernel<128, false>' if D == 128 and w2 > 12 else 'sa2::fwd_kernel<%d, false>' % D
     if entry == 'bwd_dq_dk2_pass':
         return 'sa2::bwd_q_kernel<%d, true, false>' % D
     if entry == 'bwd_dkv1':

@@ -282,10 +282,15 @@ static int q_splits(const sa2_problem *prob, int merge_cost, bool shared, int64_
 static int fwd_splits(const sa2_problem *prob) { return q_splits(prob, 8, prob->dim_head != 128, 0); }   // (the merge is a launch of its own)
 static int bwd_splits(const sa2_problem *prob) { return q_splits(prob, 2, false, partial_rows_bytes(prob)); }
 
-// dim_head 128: one wave per SIMD with two offsets each; 64 and 32: two workgroups of eight waves per CU
+// dim_head 64 and 32: two workgroups of eight waves per CU, an offset per wave.  128: one wave per SIMD with two offsets each, unless the second
+// window leaves so many waves of the last round without one that eight waves are faster.  4 x 8 x 8192 rows, w1 512, the eight-wave form
+// and the other (us): w2 2 506, 613; 4 511, 620; 9 971, 1028; 12 1032, 1050; 32 2253, 2107.  (Shared rounds are another matter: kernels there are
+// short of workgroups, not of waves, and one form serves.)
+static constexpr int kShortWindow = 12;
 static void launch_fwd(int dim_head, bool split, int grid, hipStream_t s, const sa2::KParams &k) {
     if (dim_head == 128) {
-        sa2::launch_fwd2(split, grid, s, k);
+        if (!split && k.w2 <= kShortWindow) hipLaunchKernelGGL((sa2::fwd_kernel<128>), dim3(grid), dim3(512), 0, s, k);
+        else sa2::launch_fwd2(split, grid, s, k);
     } else if (dim_head == 64) {
         if (split) hipLaunchKernelGGL((sa2::fwd_kernel<64, true>), dim3(grid), dim3(512), 0, s, k);
         else hipLaunchKernelGGL((sa2::fwd_kernel<64>), dim3(grid), dim3(512), 0, s, k);

@@ -57,11 +57,12 @@ struct FwdCfg {
     // LDS and 128 registers: two workgroups per CU)
     static constexpr bool QF = D != 64;
     // waves per SIMD: D = 64 is held to 128 registers (a few spills outside the step's MFMA blocks) so that two workgroups
-    // share a CU, which is worth 20 % at D = 64; D = 32 fits by itself
-    static constexpr int WPE = 4;
+    // share a CU, which is worth 20 % at D = 64; D = 32 fits by itself; D = 128 (short second windows, launch_fwd in sa2_api.hip
+    // has the rule) has one workgroup per CU
+    static constexpr int WPE = D == 128 ? 2 : 4;
     // fragments in flight per operand and chain: two of the four at D = 64, where four waves per SIMD cover the latency
-    // and the registers are the scarcer resource; both at D = 32
-    static constexpr int FW = 2;
+    // and the registers are the scarcer resource; both at D = 32; four of the eight at D = 128
+    static constexpr int FW = D == 128 ? 4 : 2;
     static constexpr int QS = RING + ACC + 2 * EXCH;
     static constexpr int QPITCH = QF ? D * 4 + 16 : tile_pitch<D>();
     static constexpr int KSLOTS = 64;                 // circular k2 / v2 rows
@@ -70,7 +71,7 @@ struct FwdCfg {
     static constexpr int MASKS = V2S + KSLOTS * PITCH; // additive masks (0 / -inf) of the diagonal tile and of up to two lower-edge tiles
     static constexpr int MASK = 16 * 64 * 4;          // one table: [4 quarters][64 lanes][4 floats]
     static constexpr int LDS = MASKS + 3 * MASK;
-    static_assert(D <= 64 && 2 * LDS <= 160 * 1024, "two workgroups per CU need half the LDS each");
+    static_assert((WPE == 4 ? 2 : 1) * LDS <= 160 * 1024, "two workgroups per CU need half the LDS each");
     static_assert(RING - CP < 65536, "the LDS address of a direct load travels in 16 bits of M0");
     static constexpr int PPR = D / 8;                 // 16-byte pieces per row
     static constexpr int PIECES = 32 * PPR;           // ... per tile
@@ -241,6 +242,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(FwdCfg<D>::
         }
     };
 
+    // accumulator clears: as 64-bit moves where registers are plentiful (at four waves per SIMD the register pairs
+    // they need cost more in spilled registers than the moves save)
+    auto clear16 = [] {
+        if constexpr (C::WPE == 2) return zero16_pairs();
+        else return zero16();
+    };
     f32x16 T[DT];
     u32x4 A[KS];
     // Fragments travel through rolling windows of FW register sets: fragment f of a chain sits in set f % FW and is
@@ -309,7 +316,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(FwdCfg<D>::
                 }
             }
 #pragma unroll
-            for (int dt = 0; dt < DT; ++dt) T[dt] = zero16();
+            for (int dt = 0; dt < DT; ++dt) T[dt] = clear16();
         }
 
         // exponentials and row sums of the tile whose referenced logits are in X
@@ -405,7 +412,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(FwdCfg<D>::
                 // ---- the wave's very first step, the diagonal tile of its first offset: every valid row
                 // attends an entry of it, so this is where the rows get their softmax reference M
                 open_step();
-                f32x16 X = zero16();
+                f32x16 X = clear16();
                 logit_chain(X, std::false_type{});
                 {
                     // row j = 32 t + 4 hf + e (e = 8 (rr / 4) + rr % 4) is attended iff 0 <= i - j < w1;
@@ -436,9 +443,14 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(FwdCfg<D>::
             // subtraction code follows it.  A row's reference moves only if its row sum says that weights
             // outgrew the safe range.
             float nm = col_ok ? -M : -INFINITY;
+            // the chains' start value, kept in registers where they are plentiful (eight moves per step instead of sixteen)
+            f32x16 NMv;
+            if constexpr (C::WPE == 2) NMv = splat16(nm);
             u32x4 pb[2];
             for (; n < NT; ++n) {
-                f32x16 X = splat16(nm);
+                f32x16 X;
+                if constexpr (C::WPE == 2) X = NMv;
+                else X = splat16(nm);
                 if (n < n_masked) {
                     const char *mk = lds + C::MASKS + n * C::MASK + lane * 16;
 #pragma unroll
@@ -467,6 +479,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(FwdCfg<D>::
                     const float shift = over ? fmaxf(fmaxf(tmax, e_old), 0.f) : 0.f;
                     shift_reference(shift, fast_exp2(-shift), X);
                     nm = col_ok ? -M : -INFINITY;
+                    if constexpr (C::WPE == 2) NMv = splat16(nm);
                     exponentials(X, pb);
                 }
                 value_products(pb);
@@ -529,7 +542,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(FwdCfg<D>::
             // phases 2 DT g .. 2 DT g + 2 DT - 1 and its wave w the slice (w + ph) mod 2 DT in phase ph
             for (int ph = 0; ph < 8; ++ph) {
                 constexpr int NS = 2 * DT;
-                if (ph / NS == wave / NS) with_slice<NS>(wave + ph, [&](auto tag) { add_slice(tag, ph % NS == 0 && wave / NS == 0); });
+                if (NS == 8 || ph / NS == wave / NS) with_slice<NS>(wave + ph, [&](auto tag) { add_slice(tag, ph % NS == 0 && (NS == 8 || wave / NS == 0)); });
                 if (ph == 7 && adds_rows(r)) write_rows(r);  // (their slots are not in use in this round)
                 __syncthreads();
             }
@@ -575,7 +588,16 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(FwdCfg<D>::
             o[x] = v.x * inv;
             o[x + 1] = v.y * inv;
         }
-        if constexpr (SEG == 4) {
+        if constexpr (SEG == 8) {
+            u32x4 ov, rv;
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                ov[w] = pack_bf16(o[2 * w], o[2 * w + 1]);
+                rv[w] = pack_bf16(o[2 * w] - bf16_lo(ov[w]), o[2 * w + 1] - bf16_hi(ov[w]));
+            }
+            st_global16(orow, ov);
+            if (rrow) st_global16(rrow, rv);
+        } else if constexpr (SEG == 4) {
             u32x2 ov, rv;
 #pragma unroll
             for (int w = 0; w < 2; ++w) {
@@ -585,7 +607,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(FwdCfg<D>::
             *reinterpret_cast<u32x2 *>(orow) = ov;
             if (rrow) *reinterpret_cast<u32x2 *>(rrow) = rv;
         } else {
-            static_assert(SEG == 2, "head dimension 32 or 64");
+            static_assert(SEG == 2, "head dimension 32, 64 or 128");
             const uint32_t ov = pack_bf16(o[0], o[1]);
             *reinterpret_cast<uint32_t *>(orow) = ov;
             if (rrow) *reinterpret_cast<uint32_t *>(rrow) = pack_bf16(o[0] - bf16_lo(ov), o[1] - bf16_hi(ov));
