@@ -57,6 +57,10 @@ struct QCfg {
     static constexpr int LDS = MASKS + 3 * MASK;
     static constexpr int PPR = D / 8;                 // 16-byte pieces per row
     static constexpr int PIECES = 32 * PPR;           // ... per tile
+    // dQ pass at D <= 64: the start values of the logit chains stay in 16 registers for a round (198 of 256 at D = 64; at
+    // D = 128 none are left) instead of being copied together at every step.  At D = 64 a step has 12 MFMAs, and what it issues
+    // beside them is the bound: 948 -> 929 us at 8 x 8 x 2048 rows, w1 512, w2 32.
+    static constexpr bool KEEP_NL = DQ && D <= 64;
 };
 
 // SPLIT: the rounds of a query tile are shared by p.q_splits workgroups (fwd_split_round); each leaves its dq rows in
@@ -278,6 +282,8 @@ __global__ __launch_bounds__(512) void bwd_q_kernel(KParams p, float *ws, int ha
         }
         const float nl = col_ok ? -lse2 : -INFINITY;  // where the logit chains start
         const f32x2 nl2 = {nl, nl};
+        f32x16 nl_reg;                                // (KEEP_NL)
+        if constexpr (C::KEEP_NL) nl_reg = splat16(nl);
 
         for (int n = 0; n < NT; ++n) {
             open_step();
@@ -304,8 +310,11 @@ __global__ __launch_bounds__(512) void bwd_q_kernel(KParams p, float *ws, int ha
                 // while they are in flight, not in front of them)
                 u32x4 f[W];
                 static_for<0, (W < NFR ? W : NFR)>([&](auto s) { f[s] = fragment(s); });
-                f32x16 X = splat16_pairs(nl2);
-                if (t == t_hi || n < n_head) {
+                f32x16 X;
+                if constexpr (!C::KEEP_NL) X = splat16_pairs(nl2);
+                const bool masked = t == t_hi || n < n_head;
+                if (masked) {
+                    if constexpr (C::KEEP_NL) X = nl_reg;
                     const char *mk = lds + C::MASKS + (t == t_hi ? 0 : 1 + n) * C::MASK + lane * 16;
 #pragma unroll
                     for (int qq = 0; qq < 4; ++qq) {
@@ -316,11 +325,18 @@ __global__ __launch_bounds__(512) void bwd_q_kernel(KParams p, float *ws, int ha
                         X[4 * qq + 3] += m4.w;
                     }
                 }
+                if constexpr (C::KEEP_NL) {
+                    // (the first product in both branches: an unmasked one takes the start values from where they are)
+                    if (masked) X = mfma32(f[0], A[0], X);
+                    else X = mfma32(f[0], A[0], nl_reg);
+                }
                 f32x16 dP = neg_delta;      // DQ: the chain starts from -delta_i, so dP - delta costs no VALU work
                 __builtin_amdgcn_sched_barrier(0);
                 static_for<0, NROW>([&](auto sc_) {
                     constexpr int s = decltype(sc_)::value;
-                    if constexpr (s < KS) X = mfma32(f[s % W], A[s], X);
+                    if constexpr (s < KS) {
+                        if constexpr (s > 0 || !C::KEEP_NL) X = mfma32(f[s % W], A[s], X);
+                    }
                     else dP = mfma32(f[s % W], Bv[DQ ? s - KS : 0], dP);
                     if constexpr (s + W < NFR) f[s % W] = fragment(std::integral_constant<int, s + W>{});
                     __builtin_amdgcn_sched_barrier(0);
