@@ -591,17 +591,25 @@ static int launch_q_mfma(const sa2_problem *prob, const QLaunch &L, int pass, hi
     return after_launch("dq/dk2/dv2");
 }
 
+static int dv2_blocks(const sa2_problem *prob) { return prob->batch * prob->kv_heads * ((prob->seq_len + 31) / 32); }
+
 static int launch_dv2_from_saved(const sa2_problem *prob, const QLaunch &L, hipStream_t s) {
-    const int dgrid = prob->batch * prob->kv_heads * ((prob->seq_len + 31) / 32);
-    // up to two workgroups per CU the chain of loads of one workgroup is what the kernel takes: split it inside the workgroup
-    const bool grouped = prob->dim_head < 128 && dgrid <= 2 * kComputeUnits;
-    if (grouped && prob->dim_head == 64)
-        hipLaunchKernelGGL((sa2::dv2_from_saved_kernel<64, true>), dim3(dgrid), dim3((sa2::Dv2Cfg<64, true>::THREADS)), 0, s, L.k);
-    else if (grouped)
-        hipLaunchKernelGGL((sa2::dv2_from_saved_kernel<32, true>), dim3(dgrid), dim3((sa2::Dv2Cfg<32, true>::THREADS)), 0, s, L.k);
-    else
-        SA2_FOR_DIM_HEAD(prob->dim_head, hipLaunchKernelGGL((sa2::dv2_from_saved_kernel<DH, false>), dim3(dgrid), dim3((sa2::Dv2Cfg<DH, false>::THREADS)), 0, s, L.k));
+    SA2_FOR_DIM_HEAD(prob->dim_head,
+                     hipLaunchKernelGGL(sa2::dv2_from_saved_kernel<DH>, dim3(dv2_blocks(prob)), dim3((sa2::Dv2Cfg<DH, false>::THREADS)), 0, s, L.k));
     return after_launch("dv2 from saved partials");
+}
+
+// Up to two dV2 blocks per CU the chains of loads of single workgroups are what dV2, dK2 and dQ take: one launch, with the chains
+// split inside the workgroups
+static int launch_small_grid_merge(const sa2_problem *prob, const QLaunch &L, hipStream_t s) {
+    const int64_t k_rows = (int64_t)prob->batch * prob->kv_heads * prob->seq_len, q_rows = (int64_t)prob->batch * prob->heads * prob->seq_len;
+    SA2_FOR_DIM_HEAD(prob->dim_head, {
+        using C = sa2::MergeCfg<DH>;
+        const int k_blocks = (int)((k_rows + C::DK2_ROWS - 1) / C::DK2_ROWS);
+        const int q_blocks = L.k.q_splits > 1 ? (int)((q_rows + C::DQ_ROWS - 1) / C::DQ_ROWS) : 0;
+        hipLaunchKernelGGL(sa2::small_grid_merge_kernel<DH>, dim3(dv2_blocks(prob) + k_blocks + q_blocks), dim3(C::THREADS), 0, s, L.k, L.ws, 32 + L.halo, dv2_blocks(prob), k_blocks);
+    });
+    return after_launch("dv2, dk2 and dq of a small grid");
 }
 
 static int launch_q_combine(const sa2_problem *prob, const QLaunch &L, hipStream_t s) {
@@ -615,6 +623,12 @@ static int launch_q_combine(const sa2_problem *prob, const QLaunch &L, hipStream
     return after_launch("dk2/dv2 combine");
 }
 
+static int launch_q_merge(const sa2_problem *prob, const QLaunch &L, hipStream_t s) {
+    if (L.use_saved && dv2_blocks(prob) <= 2 * kComputeUnits) return launch_small_grid_merge(prob, L, s);
+    if (L.use_saved) SA2_TRY(launch_dv2_from_saved(prob, L, s));
+    return launch_q_combine(prob, L, s);
+}
+
 int sa2_bwd_dq_dkv2(const sa2_problem *prob, const sa2_tensor *q, const sa2_tensor *k1, const sa2_tensor *k2,
                     const sa2_tensor *v1, const sa2_tensor *v2, const sa2_tensor *dout, const float *lse,
                     const float *delta, const sa2_saved *saved, const sa2_tensor *dq, const sa2_tensor *dk2,
@@ -625,8 +639,7 @@ int sa2_bwd_dq_dkv2(const sa2_problem *prob, const sa2_tensor *q, const sa2_tens
     const int pass = bwd_pass_filter();
     SA2_TRY(launch_q_mfma(prob, L, pass, s));
     if (pass == 1) return SA2_OK;    // profiling build, one pass: leave the reductions out of its timing
-    if (L.use_saved) SA2_TRY(launch_dv2_from_saved(prob, L, s));
-    return launch_q_combine(prob, L, s);
+    return launch_q_merge(prob, L, s);
 }
 
 static int launch_dkv1(const sa2_problem *prob, const sa2_tensor *q, const sa2_tensor *k1, const sa2_tensor *k2,
@@ -702,8 +715,7 @@ static int bwd_all(bool split, const sa2_problem *prob, const sa2_tensor *q, con
         if (out_residual) L.k.o_lo = dev(out_residual);
     }
     SA2_TRY(launch_q_mfma(prob, L, 0, s));
-    if (L.use_saved) SA2_TRY(launch_dv2_from_saved(prob, L, s));
-    SA2_TRY(launch_q_combine(prob, L, s));
+    SA2_TRY(launch_q_merge(prob, L, s));
     // the partial rows of dK2/dV2 are spent by now: the partial results of split key slabs reuse the workspace
     return launch_dkv1(prob, q, k1, k2, v1, v2, dout, lse, delta_ws, dk1, dv1, plan, static_cast<float *>(workspace), hip_stream);
 }

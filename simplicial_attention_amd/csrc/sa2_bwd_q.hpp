@@ -470,8 +470,8 @@ __global__ __launch_bounds__(512) void bwd_q_kernel(KParams p, float *ws, int ha
 // (h = hk*G + g).  Streams T once from HBM.  A workgroup owns 32 rows k, a thread 8 d of one row; consecutive
 // threads own consecutive rows, whose pieces are consecutive in the blocked layout of T (saved_t_offset).  The do
 // rows k0 .. k0 + 62 that 32 offsets reach and the 32 x 32 weights are staged in LDS per block of 32 offsets.
-// GROUPS: at D = 32 and 64 the threads of a workgroup form OG groups that take every OG-th offset and meet through LDS.  The
-// loop over the offsets is a chain of loads, which few workgroups do not hide (launch_dv2_from_saved has the rule); a large grid does
+// GROUPS (small_grid_merge_kernel): at D = 32 and 64 the threads of a workgroup form OG groups that take every OG-th offset and meet
+// through LDS.  The loop over the offsets is a chain of loads, which few workgroups do not hide; a large grid does
 // and loses by the larger workgroups (152 us instead of 130 at 8 x 8 x 2048 rows of 64).
 template <int D, bool GROUPS>
 struct Dv2Cfg {
@@ -482,7 +482,7 @@ struct Dv2Cfg {
 };
 
 template <int D, bool GROUPS>
-__global__ __launch_bounds__((Dv2Cfg<D, GROUPS>::THREADS)) void dv2_from_saved_kernel(KParams p) {
+__device__ __forceinline__ void dv2_from_saved_block(const KParams &p, const int block) {
     using C = Dv2Cfg<D, GROUPS>;
     constexpr int LP = C::LP, NTH = C::THREADS, PITCH = C::PITCH, OG = C::OG;
     __shared__ __attribute__((aligned(16))) char dos[63 * PITCH];
@@ -490,8 +490,8 @@ __global__ __launch_bounds__((Dv2Cfg<D, GROUPS>::THREADS)) void dv2_from_saved_k
     __shared__ float4 red[OG > 1 ? (OG - 1) * 32 * LP * 2 : 1];
     const int N = p.N;
     const int ntile = (N + 31) / 32;
-    const int kt = blockIdx.x % ntile;
-    const int bh = blockIdx.x / ntile;
+    const int kt = block % ntile;
+    const int bh = block / ntile;
     const int hk = bh % p.HK, b = bh / p.HK;
     const int tid = threadIdx.x;
     const int og = GROUPS ? tid / (32 * LP) : 0, t_in = GROUPS ? tid % (32 * LP) : tid;
@@ -506,6 +506,21 @@ __global__ __launch_bounds__((Dv2Cfg<D, GROUPS>::THREADS)) void dv2_from_saved_k
         const char *dog = p.dout.ptr + b * p.dout.sb + h * p.dout.sh;
         const float *lse = p.lse + bh_row * N;
         for (int d0 = 0; d0 < nd; d0 += 32) {
+            // (rows past the end have weight 0; their T is read from the last row, which every offset has written)
+            auto t_of = [&](int dl) {
+                const int i = k + d0 + dl < N ? k + d0 + dl : N - 1;
+                const int64_t sbh = bh_row * p.w2 + d0 + dl;
+                return ld_global16(p.t_save + (sbh * ntile + (i >> 5)) * saved_t_block<D>() + t_piece + (i & 31) * 16);
+            };
+            const int nl = nd - d0 < 32 ? nd - d0 : 32;
+            // GROUPS: the first eight T pieces of the block are requested in front of the staging, whose latency they then share
+            // (offsets past the last one are read from it and not used)
+            u32x4 ahead[GROUPS ? 8 : 1];
+            auto request = [&](int x0) {
+#pragma unroll
+                for (int x = 0; x < 8; ++x) ahead[GROUPS ? x : 0] = t_of(og + (x0 + x) * OG < nl ? og + (x0 + x) * OG : nl - 1);
+            };
+            if constexpr (GROUPS) request(0);
             __syncthreads();
             for (int x = tid; x < 63 * LP; x += NTH) {
                 const int row = x / LP, pc = x % LP;
@@ -520,13 +535,7 @@ __global__ __launch_bounds__((Dv2Cfg<D, GROUPS>::THREADS)) void dv2_from_saved_k
                 wsh[x] = w;
             }
             __syncthreads();
-            const int nl = nd - d0 < 32 ? nd - d0 : 32;
-#pragma unroll 8
-            for (int dl = og; dl < nl; dl += OG) {
-                // (rows past the end have weight 0; their T is read from the last row, which every offset has written)
-                const int i = k + d0 + dl < N ? k + d0 + dl : N - 1;
-                const int64_t sbh = bh_row * p.w2 + d0 + dl;
-                const u32x4 t = ld_global16(p.t_save + (sbh * ntile + (i >> 5)) * saved_t_block<D>() + t_piece + (i & 31) * 16);
+            auto add = [&](int dl, const u32x4 &t) {
                 const u32x4 o = ld_lds16(dos + (c + dl) * PITCH + piece * 16);
                 const float w = wsh[dl * 32 + c];
 #pragma unroll
@@ -534,6 +543,18 @@ __global__ __launch_bounds__((Dv2Cfg<D, GROUPS>::THREADS)) void dv2_from_saved_k
                     acc[2 * x] += bf16_lo(o[x]) * bf16_lo(t[x]) * w;
                     acc[2 * x + 1] += bf16_hi(o[x]) * bf16_hi(t[x]) * w;
                 }
+            };
+            if constexpr (GROUPS) {
+#pragma unroll
+                for (int x0 = 0; x0 < 32 / OG; x0 += 8) {
+                    if (x0 > 0) request(x0);
+#pragma unroll
+                    for (int x = 0; x < 8; ++x)
+                        if (og + (x0 + x) * OG < nl) add(og + (x0 + x) * OG, ahead[x]);
+                }
+            } else {
+#pragma unroll 8
+                for (int dl = 0; dl < nl; ++dl) add(dl, t_of(dl));
             }
         }
     }
@@ -563,39 +584,30 @@ __global__ __launch_bounds__((Dv2Cfg<D, GROUPS>::THREADS)) void dv2_from_saved_k
     st_global16(p.dv2.ptr + b * p.dv2.sb + (int64_t)k * p.dv2.sn + hk * p.dv2.sh + piece * 16, r);
 }
 
+template <int D>
+__global__ __launch_bounds__((Dv2Cfg<D, false>::THREADS)) void dv2_from_saved_kernel(KParams p) {
+    dv2_from_saved_block<D, false>(p, blockIdx.x);
+}
+
 // dK2 / dV2 from the partial rows of the workspace: sums the tiles that reach a row and the query heads of a group.
 // Workspace rows of a tile with first query row i0: index x <-> k = i0 - halo + x, so
 // rows 0..halo-1 are the halo below the tile and rows halo..halo+31 its own rows.
 // With split query tiles (p.q_splits > 1) the shares of a tile are added in split order (a share has written the rows its
-// rounds reach, k - i0 = -8 R + 1 .. 31 - 8 r_first) and the blocks of grid row 1 form dq from the shares' fp32 rows.
-template <int D>
-__global__ __launch_bounds__(256) void dk2_dv2_combine_kernel(KParams p, const float *ws, int srows, int with_dv2) {
+// rounds reach, k - i0 = -8 R + 1 .. 31 - 8 r_first); dq_from_shares forms dq from the shares' fp32 rows.
+// CG > 1 (no dV2 rows): CG groups of threads take every CG-th share that reaches a row (an undivided tile counts as one share) and
+// meet through LDS, in a fixed order.
+template <int D, int NTH, int CG>
+__device__ __forceinline__ void combine_rows(const KParams &p, const float *ws, const int srows, const int with_dv2, const int block) {
     constexpr int LP = D / 8;   // threads per row, 8 d each
+    constexpr int RPB = NTH / (LP * CG);
     const int N = p.N, ntile = (N + 31) / 32;
     const int halo = srows - 32;
     const int piece = threadIdx.x % LP;
-    const int64_t row = (int64_t)blockIdx.x * (256 / LP) + threadIdx.x / LP;
-    if (blockIdx.y == 1) {
-        const int64_t rows = (int64_t)p.B * p.H * N;
-        if (row >= rows) return;
-        const int i = (int)(row % N), h = (int)((row / N) % p.H), b = (int)(row / ((int64_t)N * p.H));
-        const int rounds = fwd_rounds(i / 32, p.w2);
-        const int splits = p.q_splits < rounds ? p.q_splits : rounds;
-        float a[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-        for (int s = 0; s < splits; ++s) {
-            const float *src = p.q_parts + (s * rows + row) * D + piece * 8;
-#pragma unroll
-            for (int x = 0; x < 8; ++x) a[x] += src[x];
-        }
-        u32x4 o;
-#pragma unroll
-        for (int w = 0; w < 4; ++w) o[w] = pack_bf16(a[2 * w] * p.scale, a[2 * w + 1] * p.scale);
-        st_global16(p.dq.ptr + b * p.dq.sb + (int64_t)i * p.dq.sn + h * p.dq.sh + piece * 16, o);
-        return;
-    }
+    const int cg = CG > 1 ? threadIdx.x / (LP * RPB) : 0, t_in = threadIdx.x % (LP * RPB);
     const int64_t rows = (int64_t)p.B * p.HK * N;
-    if (row >= rows) return;
+    const int64_t row_raw = (int64_t)block * RPB + t_in / LP;
+    if (CG == 1 && row_raw >= rows) return;
+    const int64_t row = row_raw < rows ? row_raw : rows - 1;      // (CG > 1: every thread reaches the barrier)
     const int k = (int)(row % N);
     const int hk = (int)((row / N) % p.HK);
     const int b = (int)(row / ((int64_t)N * p.HK));
@@ -604,24 +616,27 @@ __global__ __launch_bounds__(256) void dk2_dv2_combine_kernel(KParams p, const f
     float ak[8], av[8];
 #pragma unroll
     for (int x = 0; x < 8; ++x) ak[x] = av[x] = 0.f;
+    int turn = 0;                // shares seen (CG > 1)
     for (int g = 0; g < p.G; ++g) {
         const int h = hk * p.G + g;
         const float *base = ws + (((int64_t)b * p.H + h) * ntile) * srows * D;
         for (int m = 0; tile + m < ntile && kl + halo - 32 * m >= 0; ++m) {
             const float *src = base + ((int64_t)(tile + m) * srows + (kl + halo - 32 * m)) * D + piece * 8;
-            if (p.q_splits > 1) {
+            if (CG > 1 || p.q_splits > 1) {
                 // the shares whose rounds r0 .. r1 - 1 reach the row: 1 - 8 r1 <= rel <= 31 - 8 r0
                 const int rounds = fwd_rounds(tile + m, p.w2), rel = kl - 32 * m;
                 const int r_lo = rel >= 0 ? 0 : (-rel) / 8, r_hi = (31 - rel) / 8;        // rounds that reach it
-                for (int s = fwd_split_of(r_lo, p.q_splits, rounds); s < p.q_splits; ++s) {
-                    const int r0 = fwd_split_round(s, p.q_splits, rounds), r1 = fwd_split_round(s + 1, p.q_splits, rounds);
+                int s = fwd_split_of(r_lo, p.q_splits, rounds);
+                for (int r0 = fwd_split_round(s, p.q_splits, rounds), r1; s < p.q_splits; ++s, r0 = r1) {
+                    r1 = fwd_split_round(s + 1, p.q_splits, rounds);
                     if (r0 >= r1 || r0 > r_hi) break;
                     if (rel < 1 - 8 * r1) continue;
+                    if (CG > 1 && turn++ % CG != cg) continue;
                     const float *ss = src + s * p.q_ws_stride;
 #pragma unroll
                     for (int x = 0; x < 8; ++x) {
                         ak[x] += ss[x];
-                        if (with_dv2) av[x] += ss[per_tensor + x];
+                        if (CG == 1 && with_dv2) av[x] += ss[per_tensor + x];
                     }
                 }
                 continue;
@@ -633,6 +648,27 @@ __global__ __launch_bounds__(256) void dk2_dv2_combine_kernel(KParams p, const f
             }
         }
     }
+    if constexpr (CG > 1) {
+        __shared__ float4 red[(CG - 1) * RPB * LP * 2];
+        if (cg > 0) {
+            red[((cg - 1) * RPB * LP + t_in) * 2] = make_float4(ak[0], ak[1], ak[2], ak[3]);
+            red[((cg - 1) * RPB * LP + t_in) * 2 + 1] = make_float4(ak[4], ak[5], ak[6], ak[7]);
+        }
+        __syncthreads();
+        if (cg > 0 || row_raw >= rows) return;
+#pragma unroll
+        for (int x = 0; x < CG - 1; ++x) {
+            const float4 a = red[(x * RPB * LP + t_in) * 2], e = red[(x * RPB * LP + t_in) * 2 + 1];
+            ak[0] += a.x;
+            ak[1] += a.y;
+            ak[2] += a.z;
+            ak[3] += a.w;
+            ak[4] += e.x;
+            ak[5] += e.y;
+            ak[6] += e.z;
+            ak[7] += e.w;
+        }
+    }
     u32x4 ok, ov;
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
@@ -640,7 +676,57 @@ __global__ __launch_bounds__(256) void dk2_dv2_combine_kernel(KParams p, const f
         ov[w] = pack_bf16(av[2 * w], av[2 * w + 1]);
     }
     st_global16(p.dk2.ptr + b * p.dk2.sb + (int64_t)k * p.dk2.sn + hk * p.dk2.sh + piece * 16, ok);
-    if (with_dv2) st_global16(p.dv2.ptr + b * p.dv2.sb + (int64_t)k * p.dv2.sn + hk * p.dv2.sh + piece * 16, ov);
+    if (CG == 1 && with_dv2) st_global16(p.dv2.ptr + b * p.dv2.sb + (int64_t)k * p.dv2.sn + hk * p.dv2.sh + piece * 16, ov);
+}
+
+// dq from the fp32 rows that the shares of split query tiles leave
+template <int D, int NTH>
+__device__ __forceinline__ void dq_from_shares(const KParams &p, const int block) {
+    constexpr int LP = D / 8;
+    const int N = p.N, piece = threadIdx.x % LP;
+    const int64_t row = (int64_t)block * (NTH / LP) + threadIdx.x / LP;
+    const int64_t rows = (int64_t)p.B * p.H * N;
+    if (row >= rows) return;
+    const int i = (int)(row % N), h = (int)((row / N) % p.H), b = (int)(row / ((int64_t)N * p.H));
+    const int rounds = fwd_rounds(i / 32, p.w2);
+    const int splits = p.q_splits < rounds ? p.q_splits : rounds;
+    float a[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+    for (int s = 0; s < splits; ++s) {
+        const float *src = p.q_parts + (s * rows + row) * D + piece * 8;
+#pragma unroll
+        for (int x = 0; x < 8; ++x) a[x] += src[x];
+    }
+    u32x4 o;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) o[w] = pack_bf16(a[2 * w] * p.scale, a[2 * w + 1] * p.scale);
+    st_global16(p.dq.ptr + b * p.dq.sb + (int64_t)i * p.dq.sn + h * p.dq.sh + piece * 16, o);
+}
+
+// (grid row 1, with split query tiles: dq)
+template <int D>
+__global__ __launch_bounds__(256) void dk2_dv2_combine_kernel(KParams p, const float *ws, int srows, int with_dv2) {
+    if (blockIdx.y == 1) dq_from_shares<D, 256>(p, blockIdx.x);
+    else combine_rows<D, 256, 1>(p, ws, srows, with_dv2, blockIdx.x);
+}
+
+// Small grids with saved forward partials: dV2, dK2 and, of split query tiles, dQ in one launch.  Blocks 0 .. dv2_blocks - 1 form dV2,
+// the next dk2_blocks dK2, the rest dQ.  Each is a chain of dependent loads in a few workgroups, so one behind the other they cost
+// the sum of their latencies, side by side the longest.  As two launches and as one (us): 1 x 4 x 128 rows of 32, w2 128: 38.8, 13.0;
+// 1 x 8 (4 kv) x 1000 rows of 64, w2 32: 20.4, 13.7; 2 x 6 (2 kv) x 2999 rows of 128, w2 20: 68.3, 55.0.
+template <int D>
+struct MergeCfg {
+    static constexpr int THREADS = 512, CG = 4;
+    static constexpr int DK2_ROWS = THREADS / (D / 8 * CG), DQ_ROWS = THREADS / (D / 8);      // rows per block
+    static_assert(Dv2Cfg<D, (D < 128)>::THREADS == THREADS, "one block size");
+};
+template <int D>
+__global__ __launch_bounds__(512) void small_grid_merge_kernel(KParams p, const float *ws, int srows, int dv2_blocks, int dk2_blocks) {
+    using C = MergeCfg<D>;
+    const int x = blockIdx.x;
+    if (x < dv2_blocks) dv2_from_saved_block<D, (D < 128)>(p, x);
+    else if (x < dv2_blocks + dk2_blocks) combine_rows<D, C::THREADS, C::CG>(p, ws, srows, 0, x - dv2_blocks);
+    else dq_from_shares<D, C::THREADS>(p, x - dv2_blocks - dk2_blocks);
 }
 
 }  // namespace sa2

@@ -39,6 +39,25 @@ def test_forward_in_shares(b, n, h, hk, w1, w2, d):
     assert float((o0 - o1).norm() / o0.norm()) <= 2.0 ** -8
 
 
+@pytest.mark.parametrize('d', [32, 64, 128])
+@pytest.mark.parametrize('shared', [True, False], ids=['shared', 'unshared'])
+@pytest.mark.parametrize('b,n,h,hk,w1,w2', [
+    (1, 1, 1, 1, 4, 3), (1, 33, 3, 1, 16, 9), (1, 70, 4, 2, 70, 33), (1, 257, 2, 2, 40, 128),
+    (8, 33, 32, 32, 8, 5),         # 512 blocks of dV2 rows: the last grid that takes one launch
+    (8, 33, 33, 33, 8, 5),         # 528: the first that takes two
+])
+def test_second_set_gradients_of_small_grids(b, n, h, hk, w1, w2, d, shared):
+    """dV2, dK2 and dQ merged in one launch: single rows, remainders of tiles, groups, offsets beyond one block of 32."""
+    print(f'\ncase b={b} n={n} h={h} hk={hk} d={d} w1={w1} w2={w2} shared={shared}', flush=True)
+    ins = U.make_inputs(b, n, h, hk, d, seed=7 * n + d, std=d ** -0.5)
+    ref_out, _, ref_grads = U.oracle_fwd_bwd(*ins, w1, w2)
+    if shared:
+        out, grads = U.hip_fwd_bwd(*ins, w1, w2)
+    else:
+        out, _, grads = U.hip_unshared_fwd_bwd(*ins, w1, w2, use_saved=True)
+    U.check_all(out, grads, ref_out, ref_grads)
+
+
 @pytest.mark.parametrize('src_type,dst_type', [(torch.float32, torch.bfloat16), (torch.float16, torch.bfloat16), (torch.bfloat16, torch.float32),
                                                (torch.bfloat16, torch.float16), (torch.bfloat16, torch.bfloat16)])
 @pytest.mark.parametrize('src_dim,dst_dim,vector', [(96, 128, True), (128, 96, True), (33, 64, False), (64, 33, False), (5, 32, False), (64, 64, True)])
