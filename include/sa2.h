@@ -202,6 +202,18 @@ int sa2_bwd_split(const sa2_problem *prob,
                   const sa2_tensor *dv1, const sa2_tensor *dv2,
                   void *workspace, int64_t workspace_bytes, void *hip_stream);
 
+/* The same for heads of fewer channels padded to dim_head: the channels from `channels` on are zero in q, k1, k2, v1, v2, out and
+ * dout, and kernels may leave the products over them out.  The gradients are written with dim_head channels; those of the
+ * padding mean nothing. */
+int sa2_bwd_split_padded(const sa2_problem *prob, int32_t channels,
+                         const sa2_tensor *q, const sa2_tensor *k1, const sa2_tensor *k2,
+                         const sa2_tensor *v1, const sa2_tensor *v2,
+                         const sa2_tensor *out, const sa2_tensor *out_residual, const sa2_tensor *dout,
+                         const float *lse, const sa2_saved *saved, float *delta_ws,
+                         const sa2_tensor *dq, const sa2_tensor *dk1, const sa2_tensor *dk2,
+                         const sa2_tensor *dv1, const sa2_tensor *dv2,
+                         void *workspace, int64_t workspace_bytes, void *hip_stream);
+
 /* Whole backward for callers that cannot allocate (code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc): sa2_bwd without the delta_ws and workspace arguments.
  * No counterpart in the reference.  The delta rows and the dK2/dV2 partial rows live in a

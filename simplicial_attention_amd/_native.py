@@ -29,7 +29,7 @@ STATUS_NAMES = {
 
 EXPORTS = ('sa2_version', 'sa2_last_error', 'sa2_supported', 'sa2_saved_t_bytes', 'sa2_saved_m_bytes', 'sa2_fwd', 'sa2_fwd_ws', 'sa2_fwd_workspace_bytes',
            'sa2_bwd_delta', 'sa2_bwd_workspace_bytes', 'sa2_bwd_workspace_bytes_with_saved',
-           'sa2_bwd_split', 'sa2_bwd_split_workspace_bytes', 'sa2_bwd_dq_dkv2', 'sa2_bwd_dkv1', 'sa2_bwd',
+           'sa2_bwd_split', 'sa2_bwd_split_padded', 'sa2_bwd_split_workspace_bytes', 'sa2_bwd_dq_dkv2', 'sa2_bwd_dkv1', 'sa2_bwd',
            'sa2_bwd_noalloc_scratch_bytes', 'sa2_bwd_noalloc',
            'sa2_convert', 'sa2_qkv_norm_fwd', 'sa2_qkv_norm_bwd_workspace_bytes', 'sa2_qkv_norm_bwd',
            'sa2_wgrad_workspace_bytes', 'sa2_wgrad')
@@ -101,6 +101,8 @@ def _declare(lib: ctypes.CDLL) -> ctypes.CDLL:
     lib.sa2_bwd.argtypes = [P, T, T, T, T, T, T, T, T, F, S, F, T, T, T, T, T, V, I64, V]
     lib.sa2_bwd_split.restype = ctypes.c_int
     lib.sa2_bwd_split.argtypes = lib.sa2_bwd.argtypes
+    lib.sa2_bwd_split_padded.restype = ctypes.c_int
+    lib.sa2_bwd_split_padded.argtypes = [P, ctypes.c_int32, *lib.sa2_bwd.argtypes[1:]]
     lib.sa2_bwd_noalloc.restype = ctypes.c_int
     lib.sa2_bwd_noalloc.argtypes = [P, T, T, T, T, T, T, T, T, F, S, T, T, T, T, T, V]
     lib.sa2_qkv_norm_fwd.restype = ctypes.c_int

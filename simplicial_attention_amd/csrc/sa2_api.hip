@@ -529,6 +529,7 @@ struct QLaunch {
     float *ws;
     int grid, halo;
     bool use_saved;
+    int channels = 256;      // channels of a head that are not zero padding, at most
 };
 
 static int prepare_dq_dkv2(const sa2_problem *prob, const sa2_tensor *q, const sa2_tensor *k1, const sa2_tensor *k2,
@@ -577,6 +578,13 @@ static int launch_q_mfma(const sa2_problem *prob, const QLaunch &L, int pass, hi
         sa2::launch_bwd_wide_q(true, L.grid, s, L.k, L.ws, L.halo);
         if (pass != 1) sa2::launch_bwd_wide_q(false, L.grid, s, L.k, L.ws, L.halo);
         return after_launch("dq/dk2/dv2");
+    }
+    // (heads of 65 to 96 channels padded to 128, with partials saved for dV2)
+    const bool narrow = prob->dim_head == 128 && L.channels <= 96 && L.use_saved;
+    if (narrow) {
+        if (L.k.q_splits > 1) hipLaunchKernelGGL((sa2::bwd_q_kernel<128, true, true, 96>), dim3(L.k.q_splits * L.grid), dim3(512), 0, s, L.k, L.ws, L.halo);
+        else hipLaunchKernelGGL((sa2::bwd_q_kernel<128, true, false, 96>), dim3(L.grid), dim3(512), 0, s, L.k, L.ws, L.halo);
+        return after_launch("dq/dk2 of narrow heads");
     }
     if (L.k.q_splits > 1) {
         const dim3 sgrid(L.k.q_splits * L.grid);
@@ -687,7 +695,7 @@ int sa2_bwd_dkv1(const sa2_problem *prob, const sa2_tensor *q, const sa2_tensor 
     return launch_dkv1(prob, q, k1, k2, v1, v2, dout, lse, delta, dk1, dv1, Kv8Plan{0, 1}, nullptr, hip_stream);
 }
 
-static int bwd_all(bool split, const sa2_problem *prob, const sa2_tensor *q, const sa2_tensor *k1, const sa2_tensor *k2,
+static int bwd_all(bool split, int channels, const sa2_problem *prob, const sa2_tensor *q, const sa2_tensor *k1, const sa2_tensor *k2,
             const sa2_tensor *v1, const sa2_tensor *v2, const sa2_tensor *out, const sa2_tensor *out_residual,
             const sa2_tensor *dout, const float *lse, const sa2_saved *saved, float *delta_ws, const sa2_tensor *dq,
             const sa2_tensor *dk1, const sa2_tensor *dk2, const sa2_tensor *dv1, const sa2_tensor *dv2, void *workspace,
@@ -706,6 +714,7 @@ static int bwd_all(bool split, const sa2_problem *prob, const sa2_tensor *q, con
     SA2_TRY(check_tensor(dv1, "dv1"));
     QLaunch L;
     SA2_TRY(prepare_dq_dkv2(prob, q, k1, k2, v1, v2, dout, lse, delta_ws, saved, dq, dk2, dv2, workspace, workspace_bytes, split, &L));
+    L.channels = channels;
     hipStream_t s = static_cast<hipStream_t>(hip_stream);
     if (L.k.q_splits <= 1) {
         SA2_TRY(sa2_bwd_delta(prob, out, out_residual, dout, delta_ws, hip_stream));
@@ -725,7 +734,7 @@ int sa2_bwd(const sa2_problem *prob, const sa2_tensor *q, const sa2_tensor *k1, 
             const sa2_tensor *dout, const float *lse, const sa2_saved *saved, float *delta_ws, const sa2_tensor *dq,
             const sa2_tensor *dk1, const sa2_tensor *dk2, const sa2_tensor *dv1, const sa2_tensor *dv2, void *workspace,
             int64_t workspace_bytes, void *hip_stream) {
-    return bwd_all(false, prob, q, k1, k2, v1, v2, out, out_residual, dout, lse, saved, delta_ws, dq, dk1, dk2, dv1, dv2, workspace,
+    return bwd_all(false, 256, prob, q, k1, k2, v1, v2, out, out_residual, dout, lse, saved, delta_ws, dq, dk1, dk2, dv1, dv2, workspace,
                    workspace_bytes, hip_stream);
 }
 
@@ -734,7 +743,17 @@ int sa2_bwd_split(const sa2_problem *prob, const sa2_tensor *q, const sa2_tensor
                   const sa2_tensor *dout, const float *lse, const sa2_saved *saved, float *delta_ws, const sa2_tensor *dq,
                   const sa2_tensor *dk1, const sa2_tensor *dk2, const sa2_tensor *dv1, const sa2_tensor *dv2, void *workspace,
                   int64_t workspace_bytes, void *hip_stream) {
-    return bwd_all(true, prob, q, k1, k2, v1, v2, out, out_residual, dout, lse, saved, delta_ws, dq, dk1, dk2, dv1, dv2, workspace,
+    return bwd_all(true, 256, prob, q, k1, k2, v1, v2, out, out_residual, dout, lse, saved, delta_ws, dq, dk1, dk2, dv1, dv2, workspace,
+                   workspace_bytes, hip_stream);
+}
+
+int sa2_bwd_split_padded(const sa2_problem *prob, int32_t channels, const sa2_tensor *q, const sa2_tensor *k1, const sa2_tensor *k2,
+                         const sa2_tensor *v1, const sa2_tensor *v2, const sa2_tensor *out, const sa2_tensor *out_residual,
+                         const sa2_tensor *dout, const float *lse, const sa2_saved *saved, float *delta_ws, const sa2_tensor *dq,
+                         const sa2_tensor *dk1, const sa2_tensor *dk2, const sa2_tensor *dv1, const sa2_tensor *dv2, void *workspace,
+                         int64_t workspace_bytes, void *hip_stream) {
+    if (channels < 1) return fail(SA2_ERR_BAD_SHAPE, "channels = %d: at least one", (int)channels);
+    return bwd_all(true, channels, prob, q, k1, k2, v1, v2, out, out_residual, dout, lse, saved, delta_ws, dq, dk1, dk2, dv1, dv2, workspace,
                    workspace_bytes, hip_stream);
 }
 

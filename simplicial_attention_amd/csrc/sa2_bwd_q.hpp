@@ -35,8 +35,6 @@ namespace sa2 {
 
 template <int D, bool DQ>
 struct QCfg {
-    static constexpr int KS = D / 16;
-    static constexpr int DT = D / 32;
     static constexpr int PITCH = tile_pitch<D>();     // staged q / do / k2 / v2 rows
     static constexpr int TILE = 32 * PITCH;
     // ring buffer: a K1 tile and a V1 tile, written by direct-to-LDS loads (layout: DmaTile; DQ reads K1 both ways)
@@ -71,10 +69,15 @@ __host__ __device__ inline int64_t qk2_ws_floats(int B, int H, int N, int D, int
     return 2ll * B * H * ((N + 31) / 32) * srows * D;
 }
 
-template <int D, bool DQ, bool SPLIT = false>
+// CH < D: the channels from CH on are zero in every operand (rows of narrower heads padded to D), and the products over them
+// are left out: their k-slots add zeros to S and dP, their rows of G are zero.  2 x 6 (2 kv) x 2999 rows of 96 channels,
+// w1 300, w2 20: @FIG@.
+template <int D, bool DQ, bool SPLIT = false, int CH = D>
 __global__ __launch_bounds__(512) void bwd_q_kernel(KParams p, float *ws, int halo) {
     using C = QCfg<D, DQ>;
-    constexpr int KS = C::KS, DT = C::DT, PPR = C::PPR, PITCH = C::PITCH;
+    constexpr int KS = CH / 16, DT = CH / 32, PPR = C::PPR, PITCH = C::PITCH;
+    static_assert(CH % 32 == 0, "whole tiles of channels");
+    constexpr bool KEEP_NL = C::KEEP_NL || CH < D;    // (218 registers at CH = 96 without them)
     __shared__ __attribute__((aligned(16))) char lds[C::LDS];
 
     const int N = p.N;
@@ -283,7 +286,7 @@ __global__ __launch_bounds__(512) void bwd_q_kernel(KParams p, float *ws, int ha
         const float nl = col_ok ? -lse2 : -INFINITY;  // where the logit chains start
         const f32x2 nl2 = {nl, nl};
         f32x16 nl_reg;                                // (KEEP_NL)
-        if constexpr (C::KEEP_NL) nl_reg = splat16(nl);
+        if constexpr (KEEP_NL) nl_reg = splat16(nl);
 
         for (int n = 0; n < NT; ++n) {
             open_step();
@@ -311,10 +314,10 @@ __global__ __launch_bounds__(512) void bwd_q_kernel(KParams p, float *ws, int ha
                 u32x4 f[W];
                 static_for<0, (W < NFR ? W : NFR)>([&](auto s) { f[s] = fragment(s); });
                 f32x16 X;
-                if constexpr (!C::KEEP_NL) X = splat16_pairs(nl2);
+                if constexpr (!KEEP_NL) X = splat16_pairs(nl2);
                 const bool masked = t == t_hi || n < n_head;
                 if (masked) {
-                    if constexpr (C::KEEP_NL) X = nl_reg;
+                    if constexpr (KEEP_NL) X = nl_reg;
                     const char *mk = lds + C::MASKS + (t == t_hi ? 0 : 1 + n) * C::MASK + lane * 16;
 #pragma unroll
                     for (int qq = 0; qq < 4; ++qq) {
@@ -325,7 +328,7 @@ __global__ __launch_bounds__(512) void bwd_q_kernel(KParams p, float *ws, int ha
                         X[4 * qq + 3] += m4.w;
                     }
                 }
-                if constexpr (C::KEEP_NL) {
+                if constexpr (KEEP_NL) {
                     // (the first product in both branches: an unmasked one takes the start values from where they are)
                     if (masked) X = mfma32(f[0], A[0], X);
                     else X = mfma32(f[0], A[0], nl_reg);
@@ -335,7 +338,7 @@ __global__ __launch_bounds__(512) void bwd_q_kernel(KParams p, float *ws, int ha
                 static_for<0, NROW>([&](auto sc_) {
                     constexpr int s = decltype(sc_)::value;
                     if constexpr (s < KS) {
-                        if constexpr (s > 0 || !C::KEEP_NL) X = mfma32(f[s % W], A[s], X);
+                        if constexpr (s > 0 || !KEEP_NL) X = mfma32(f[s % W], A[s], X);
                     }
                     else dP = mfma32(f[s % W], Bv[DQ ? s - KS : 0], dP);
                     if constexpr (s + W < NFR) f[s % W] = fragment(std::integral_constant<int, s + W>{});
@@ -359,9 +362,9 @@ __global__ __launch_bounds__(512) void bwd_q_kernel(KParams p, float *ws, int ha
                     acc[s % DT] = mfma32(f[(NROW + s) % W], pb[s / DT], acc[s % DT]);
                     if constexpr (NROW + s + W < NFR) f[(NROW + s) % W] = fragment(std::integral_constant<int, NROW + s + W>{});
                     if constexpr (s < DT) {
-                        // (DT = 4: one pair of weights per MFMA; DT = 2: two pairs)
+                        // (four pairs of weights behind the first DT MFMAs)
 #pragma unroll
-                        for (int x = 0; x < 4 / DT; ++x) weights(8 + 2 * ((4 / DT) * s + x));
+                        for (int x = 4 * s / DT; x < 4 * (s + 1) / DT; ++x) weights(8 + 2 * x);
                     }
                     __builtin_amdgcn_sched_barrier(0);
                 });
@@ -417,10 +420,14 @@ __global__ __launch_bounds__(512) void bwd_q_kernel(KParams p, float *ws, int ha
                     *reinterpret_cast<float4 *>(dd + 4) = b1;
                 }
             };
+            auto add_slice_of = [&](auto slice_tag) {     // (CH < D: nothing to add to the slices of the zero channels)
+                if constexpr (decltype(slice_tag)::value < 2 * DT) add_slice(slice_tag);
+            };
             for (int ph = 0; ph < 8; ++ph) {
-                // 2 DT slices: the waves form 8 / (2 DT) groups that take turns, group g owns the phases 2 DT g ..
-                // 2 DT g + 2 DT - 1 (D = 128: one group, every wave works in every phase)
-                if (DT == 4 || ph / (2 * DT) == wave / (2 * DT)) with_slice<2 * DT>(wave + ph, add_slice);
+                // D / 16 slices: the waves form 8 / (D / 16) groups that take turns, group g owns the phases D / 16 g ..
+                // D / 16 g + D / 16 - 1 (D = 128: one group, every wave works in every phase)
+                constexpr int SL = D / 16;
+                if (SL == 8 || ph / SL == wave / SL) with_slice<SL>(wave + ph, add_slice_of);
                 if (ph == 7 && r + 1 < R) write_rows(r);    // (their slots are not in use in this round)
                 __syncthreads();
             }

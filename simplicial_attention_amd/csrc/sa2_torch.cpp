@@ -220,8 +220,8 @@ struct Attend : public torch::autograd::Function<Attend> {
         const sa2_tensor aq = arg(q), ak1 = arg(k1), ak2 = arg(k2), av1 = arg(v1), av2 = arg(v2), ao = arg(out), ar = arg(residual), ad = arg(dout);
         sa2_tensor ag[5];
         for (int x = 0; x < 5; ++x) ag[x] = arg(grads[x]);
-        check(sa2_bwd_split(&prob, &aq, &ak1, &ak2, &av1, &av2, &ao, &ar, &ad, static_cast<float *>(lse.data_ptr()), have_saved ? &saved : nullptr,
-                            reinterpret_cast<float *>(base), &ag[0], &ag[1], &ag[2], &ag[3], &ag[4], base + delta_bytes, ws_bytes, stream));
+        check(sa2_bwd_split_padded(&prob, (int32_t)std::max(g.dim_qk, g.dim_v), &aq, &ak1, &ak2, &av1, &av2, &ao, &ar, &ad,
+                                   static_cast<float *>(lse.data_ptr()), have_saved ? &saved : nullptr, reinterpret_cast<float *>(base), &ag[0], &ag[1], &ag[2], &ag[3], &ag[4], base + delta_bytes, ws_bytes, stream));
         // back to the types and head dimensions of the inputs
         Conversions back;
         variable_list result(5);

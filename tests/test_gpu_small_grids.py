@@ -58,6 +58,18 @@ def test_second_set_gradients_of_small_grids(b, n, h, hk, w1, w2, d, shared):
     U.check_all(out, grads, ref_out, ref_grads)
 
 
+@pytest.mark.parametrize('d', [65, 80, 96, 97])
+@pytest.mark.parametrize('b,n,h,hk,w1,w2', [(1, 1, 1, 1, 4, 3), (1, 75, 4, 2, 40, 41),
+                                            (8, 40, 66, 33, 16, 9)])     # the last: more query tiles than are shared out
+def test_narrow_heads_on_the_kernels_of_wide_ones(b, n, h, hk, w1, w2, d):
+    """Up to 96 channels padded to 128 leave the products over the last 32 out; 97 takes them all."""
+    print(f'\ncase b={b} n={n} h={h} hk={hk} d={d} w1={w1} w2={w2}', flush=True)
+    ins = U.make_inputs(b, n, h, hk, d, seed=3 * n + d, std=d ** -0.5)
+    ref_out, _, ref_grads = U.oracle_fwd_bwd(*ins, w1, w2)
+    out, grads = U.hip_fwd_bwd(*ins, w1, w2)
+    U.check_all(out, grads, ref_out, ref_grads)
+
+
 @pytest.mark.parametrize('src_type,dst_type', [(torch.float32, torch.bfloat16), (torch.float16, torch.bfloat16), (torch.bfloat16, torch.float32),
                                                (torch.bfloat16, torch.float16), (torch.bfloat16, torch.bfloat16)])
 @pytest.mark.parametrize('src_dim,dst_dim,vector', [(96, 128, True), (128, 96, True), (33, 64, False), (64, 33, False), (5, 32, False), (64, 64, True)])
