@@ -55,10 +55,11 @@ struct QCfg {
     static constexpr int LDS = MASKS + 3 * MASK;
     static constexpr int PPR = D / 8;                 // 16-byte pieces per row
     static constexpr int PIECES = 32 * PPR;           // ... per tile
-    // dQ pass at D <= 64: the start values of the logit chains stay in 16 registers for a round (198 of 256 at D = 64; at
-    // D = 128 none are left) instead of being copied together at every step.  At D = 64 a step has 12 MFMAs, and what it issues
-    // beside them is the bound: 948 -> 929 us at 8 x 8 x 2048 rows, w1 512, w2 32.
-    static constexpr bool KEEP_NL = DQ && D <= 64;
+    // dQ pass at D = 64: the start values of the logit chains stay in 16 registers for a round (198 of 256; at D = 128 none are
+    // left) instead of being copied together at every step.  A step has 12 MFMAs there, and what it issues beside them is the
+    // bound: 926 -> 895 us at 8 x 8 (4 kv) x 2048 rows, w1 512, w2 32.  At D = 32 it is no gain: 694 us there either way, and 2533 us
+    // copied, 2580 kept at 2 x 4 x 30000 rows, w1 200, w2 100, where many rounds have few steps each.
+    static constexpr bool KEEP_NL = DQ && D == 64;
 };
 
 // SPLIT: the rounds of a query tile are shared by p.q_splits workgroups (fwd_split_round); each leaves its dq rows in
