@@ -607,14 +607,16 @@ static int launch_dv2_from_saved(const sa2_problem *prob, const QLaunch &L, hipS
     return after_launch("dv2 from saved partials");
 }
 
-// Up to two dV2 blocks per CU the chains of loads of single workgroups are what dV2, dK2 and dQ take: one launch, with the chains
-// split inside the workgroups
+// Up to two dV2 blocks per CU the chains of loads of single workgroups are what dV2, dK2 and dQ take: one launch.  Measured against
+// two at 1 to 512 dV2 blocks, 1 to 16 query heads per key/value head, w2 1 to 500 and D = 32, 64, 128, it takes 0.4 to 0.9 of their time; at
+// 512 blocks (1 x 16 (4 kv) x 4096 rows), us, two and one: D = 64 w2 2 25.2, 22.5; w2 16 46.2, 39.2; w2 128 301, 258; D = 128 w2 2 42, 25; w2 128
+// 498, 453.  Beyond 512 the grids are long enough for blocks of one size each.
 static int launch_small_grid_merge(const sa2_problem *prob, const QLaunch &L, hipStream_t s) {
     const int64_t k_rows = (int64_t)prob->batch * prob->kv_heads * prob->seq_len, q_rows = (int64_t)prob->batch * prob->heads * prob->seq_len;
     SA2_FOR_DIM_HEAD(prob->dim_head, {
         using C = sa2::MergeCfg<DH>;
-        const int k_blocks = (int)((k_rows + C::DK2_ROWS - 1) / C::DK2_ROWS);
-        const int q_blocks = L.k.q_splits > 1 ? (int)((q_rows + C::DQ_ROWS - 1) / C::DQ_ROWS) : 0;
+        const int k_blocks = (int)((k_rows + C::ROWS - 1) / C::ROWS);
+        const int q_blocks = L.k.q_splits > 1 ? (int)((q_rows + C::ROWS - 1) / C::ROWS) : 0;
         hipLaunchKernelGGL(sa2::small_grid_merge_kernel<DH>, dim3(dv2_blocks(prob) + k_blocks + q_blocks), dim3(C::THREADS), 0, s, L.k, L.ws, 32 + L.halo, dv2_blocks(prob), k_blocks);
     });
     return after_launch("dv2, dk2 and dq of a small grid");

@@ -601,21 +601,17 @@ __global__ __launch_bounds__((Dv2Cfg<D, false>::THREADS)) void dv2_from_saved_ke
 // Workspace rows of a tile with first query row i0: index x <-> k = i0 - halo + x, so
 // rows 0..halo-1 are the halo below the tile and rows halo..halo+31 its own rows.
 // With split query tiles (p.q_splits > 1) the shares of a tile are added in split order (a share has written the rows its
-// rounds reach, k - i0 = -8 R + 1 .. 31 - 8 r_first); dq_from_shares forms dq from the shares' fp32 rows.
-// CG > 1 (no dV2 rows): CG groups of threads take every CG-th share that reaches a row (an undivided tile counts as one share) and
-// meet through LDS, in a fixed order.
-template <int D, int NTH, int CG>
+// rounds reach, k - i0 = -8 R + 1 .. 31 - 8 r_first); dq_from_shares forms dq from the shares' fp32 rows.  One chain of sums per
+// element, whichever kernel runs it: dK2 has the same bits with saved partials and without.
+template <int D, int NTH>
 __device__ __forceinline__ void combine_rows(const KParams &p, const float *ws, const int srows, const int with_dv2, const int block) {
     constexpr int LP = D / 8;   // threads per row, 8 d each
-    constexpr int RPB = NTH / (LP * CG);
     const int N = p.N, ntile = (N + 31) / 32;
     const int halo = srows - 32;
     const int piece = threadIdx.x % LP;
-    const int cg = CG > 1 ? threadIdx.x / (LP * RPB) : 0, t_in = threadIdx.x % (LP * RPB);
+    const int64_t row = (int64_t)block * (NTH / LP) + threadIdx.x / LP;
     const int64_t rows = (int64_t)p.B * p.HK * N;
-    const int64_t row_raw = (int64_t)block * RPB + t_in / LP;
-    if (CG == 1 && row_raw >= rows) return;
-    const int64_t row = row_raw < rows ? row_raw : rows - 1;      // (CG > 1: every thread reaches the barrier)
+    if (row >= rows) return;
     const int k = (int)(row % N);
     const int hk = (int)((row / N) % p.HK);
     const int b = (int)(row / ((int64_t)N * p.HK));
@@ -624,13 +620,12 @@ __device__ __forceinline__ void combine_rows(const KParams &p, const float *ws, 
     float ak[8], av[8];
 #pragma unroll
     for (int x = 0; x < 8; ++x) ak[x] = av[x] = 0.f;
-    int turn = 0;                // shares seen (CG > 1)
     for (int g = 0; g < p.G; ++g) {
         const int h = hk * p.G + g;
         const float *base = ws + (((int64_t)b * p.H + h) * ntile) * srows * D;
         for (int m = 0; tile + m < ntile && kl + halo - 32 * m >= 0; ++m) {
             const float *src = base + ((int64_t)(tile + m) * srows + (kl + halo - 32 * m)) * D + piece * 8;
-            if (CG > 1 || p.q_splits > 1) {
+            if (p.q_splits > 1) {
                 // the shares whose rounds r0 .. r1 - 1 reach the row: 1 - 8 r1 <= rel <= 31 - 8 r0
                 const int rounds = fwd_rounds(tile + m, p.w2), rel = kl - 32 * m;
                 const int r_lo = rel >= 0 ? 0 : (-rel) / 8, r_hi = (31 - rel) / 8;        // rounds that reach it
@@ -639,12 +634,11 @@ __device__ __forceinline__ void combine_rows(const KParams &p, const float *ws, 
                     r1 = fwd_split_round(s + 1, p.q_splits, rounds);
                     if (r0 >= r1 || r0 > r_hi) break;
                     if (rel < 1 - 8 * r1) continue;
-                    if (CG > 1 && turn++ % CG != cg) continue;
                     const float *ss = src + s * p.q_ws_stride;
 #pragma unroll
                     for (int x = 0; x < 8; ++x) {
                         ak[x] += ss[x];
-                        if (CG == 1 && with_dv2) av[x] += ss[per_tensor + x];
+                        if (with_dv2) av[x] += ss[per_tensor + x];
                     }
                 }
                 continue;
@@ -656,27 +650,6 @@ __device__ __forceinline__ void combine_rows(const KParams &p, const float *ws, 
             }
         }
     }
-    if constexpr (CG > 1) {
-        __shared__ float4 red[(CG - 1) * RPB * LP * 2];
-        if (cg > 0) {
-            red[((cg - 1) * RPB * LP + t_in) * 2] = make_float4(ak[0], ak[1], ak[2], ak[3]);
-            red[((cg - 1) * RPB * LP + t_in) * 2 + 1] = make_float4(ak[4], ak[5], ak[6], ak[7]);
-        }
-        __syncthreads();
-        if (cg > 0 || row_raw >= rows) return;
-#pragma unroll
-        for (int x = 0; x < CG - 1; ++x) {
-            const float4 a = red[(x * RPB * LP + t_in) * 2], e = red[(x * RPB * LP + t_in) * 2 + 1];
-            ak[0] += a.x;
-            ak[1] += a.y;
-            ak[2] += a.z;
-            ak[3] += a.w;
-            ak[4] += e.x;
-            ak[5] += e.y;
-            ak[6] += e.z;
-            ak[7] += e.w;
-        }
-    }
     u32x4 ok, ov;
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
@@ -684,7 +657,7 @@ __device__ __forceinline__ void combine_rows(const KParams &p, const float *ws, 
         ov[w] = pack_bf16(av[2 * w], av[2 * w + 1]);
     }
     st_global16(p.dk2.ptr + b * p.dk2.sb + (int64_t)k * p.dk2.sn + hk * p.dk2.sh + piece * 16, ok);
-    if (CG == 1 && with_dv2) st_global16(p.dv2.ptr + b * p.dv2.sb + (int64_t)k * p.dv2.sn + hk * p.dv2.sh + piece * 16, ov);
+    if (with_dv2) st_global16(p.dv2.ptr + b * p.dv2.sb + (int64_t)k * p.dv2.sn + hk * p.dv2.sh + piece * 16, ov);
 }
 
 // dq from the fp32 rows that the shares of split query tiles leave
@@ -715,17 +688,18 @@ __device__ __forceinline__ void dq_from_shares(const KParams &p, const int block
 template <int D>
 __global__ __launch_bounds__(256) void dk2_dv2_combine_kernel(KParams p, const float *ws, int srows, int with_dv2) {
     if (blockIdx.y == 1) dq_from_shares<D, 256>(p, blockIdx.x);
-    else combine_rows<D, 256, 1>(p, ws, srows, with_dv2, blockIdx.x);
+    else combine_rows<D, 256>(p, ws, srows, with_dv2, blockIdx.x);
 }
 
 // Small grids with saved forward partials: dV2, dK2 and, of split query tiles, dQ in one launch.  Blocks 0 .. dv2_blocks - 1 form dV2,
 // the next dk2_blocks dK2, the rest dQ.  Each is a chain of dependent loads in a few workgroups, so one behind the other they cost
-// the sum of their latencies, side by side the longest.  As two launches and as one (us): 1 x 4 x 128 rows of 32, w2 128: 38.8, 13.0;
-// 1 x 8 (4 kv) x 1000 rows of 64, w2 32: 20.4, 13.7; 2 x 6 (2 kv) x 2999 rows of 128, w2 20: 68.3, 55.0.
+// the sum of their latencies, side by side the longest.  As two launches; as one; as one with the first T pieces of dV2 requested
+// ahead of the staging (GROUPS), in us: 1 x 4 x 128 rows of 32, w2 128: 40.9, 22.7, 15.9; 1 x 8 (4 kv) x 1000 rows of 64, w2 32: 27.5,
+// 20.7, 16.9; 2 x 6 (2 kv) x 2999 rows of 128, w2 20 (nothing ahead at D = 128): 71, 54.  (dK2's shares dealt out to four groups of
+// threads that meet through LDS: 15.9, 16.9, 58, and 30.0 instead of 22.5 at 1 x 16 (4 kv) x 4096 rows of 64, w2 2.)
 template <int D>
 struct MergeCfg {
-    static constexpr int THREADS = 512, CG = 4;
-    static constexpr int DK2_ROWS = THREADS / (D / 8 * CG), DQ_ROWS = THREADS / (D / 8);      // rows per block
+    static constexpr int THREADS = 512, ROWS = THREADS / (D / 8);      // rows of dK2 or dQ per block
     static_assert(Dv2Cfg<D, (D < 128)>::THREADS == THREADS, "one block size");
 };
 template <int D>
@@ -733,7 +707,7 @@ __global__ __launch_bounds__(512) void small_grid_merge_kernel(KParams p, const 
     using C = MergeCfg<D>;
     const int x = blockIdx.x;
     if (x < dv2_blocks) dv2_from_saved_block<D, (D < 128)>(p, x);
-    else if (x < dv2_blocks + dk2_blocks) combine_rows<D, C::THREADS, C::CG>(p, ws, srows, 0, x - dv2_blocks);
+    else if (x < dv2_blocks + dk2_blocks) combine_rows<D, C::THREADS>(p, ws, srows, 0, x - dv2_blocks);
     else dq_from_shares<D, C::THREADS>(p, x - dv2_blocks - dk2_blocks);
 }
 

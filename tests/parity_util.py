@@ -58,8 +58,13 @@ def hip_fwd_bwd(q, k1, k2, v1, v2, dout, w1, w2):
 
 
 def hip_unshared_fwd_bwd(q, k1, k2, v1, v2, dout, w1, w2, use_saved, scale=None):
-    """Output, lse and gradients through sa2_fwd and sa2_bwd: one workgroup per query tile and key slab, however small the grid.
-    Everything that the kernels are to write starts as NaN."""
+    """Output, lse and gradients through sa2_fwd and sa2_bwd: one workgroup per query tile and key slab, however small the grid."""
+    return hip_abi_fwd_bwd(q, k1, k2, v1, v2, dout, w1, w2, use_saved, scale)
+
+
+def hip_abi_fwd_bwd(q, k1, k2, v1, v2, dout, w1, w2, use_saved, scale=None, shared=False, channels=None):
+    """Output, lse and gradients through the C ABI: sa2_fwd and, `shared`, sa2_bwd_split (with `channels` sa2_bwd_split_padded), else
+    sa2_bwd.  Everything that the kernels are to write starts as NaN."""
     from simplicial_attention_amd import _native
     lib, arg = _native.load(), _native.tensor_arg
     b, n, h, d = q.shape
@@ -72,12 +77,13 @@ def hip_unshared_fwd_bwd(q, k1, k2, v1, v2, dout, w1, w2, use_saved, scale=None)
     grads = [nan(t.shape) for t in (q, k1, k2, v1, v2)]
     t_save, m_save = raw(lib.sa2_saved_t_bytes(prob)), raw(lib.sa2_saved_m_bytes(prob))
     saved = _native.saved_arg(t_save, m_save) if use_saved else None
-    ws = raw(lib.sa2_bwd_workspace_bytes(prob))
+    ws = raw(lib.sa2_bwd_split_workspace_bytes(prob, use_saved) if shared else lib.sa2_bwd_workspace_bytes(prob))
     stream = torch.cuda.current_stream().cuda_stream
     ins = [arg(t) for t in (q, k1, k2, v1, v2)]
     _native.check(lib.sa2_fwd(prob, *ins, arg(out), arg(res), lse.data_ptr(), saved, stream))
-    _native.check(lib.sa2_bwd(prob, *ins, arg(out), arg(res), arg(dout), lse.data_ptr(), saved, delta.data_ptr(), *(arg(t) for t in grads),
-                              ws.data_ptr(), ws.numel(), stream))
+    call = lib.sa2_bwd_split_padded if channels is not None else lib.sa2_bwd_split if shared else lib.sa2_bwd
+    _native.check(call(prob, *([] if channels is None else [channels]), *ins, arg(out), arg(res), arg(dout), lse.data_ptr(), saved,
+                       delta.data_ptr(), *(arg(t) for t in grads), ws.data_ptr(), ws.numel(), stream))
     torch.cuda.synchronize()
     return out, lse, grads
 

@@ -58,6 +58,18 @@ def test_second_set_gradients_of_small_grids(b, n, h, hk, w1, w2, d, shared):
     U.check_all(out, grads, ref_out, ref_grads)
 
 
+@pytest.mark.parametrize('d', [32, 64, 128])
+@pytest.mark.parametrize('shared', [True, False], ids=['shared', 'unshared'])
+@pytest.mark.parametrize('b,n,h,hk,w1,w2', [(1, 70, 4, 2, 70, 33), (1, 257, 2, 2, 40, 128), (1, 300, 8, 2, 64, 20)])
+def test_partials_do_not_reach_the_other_gradients(b, n, h, hk, w1, w2, d, shared):
+    """Whether partials are saved decides how dV2 is formed and nothing else: the other gradients have the same bits."""
+    print(f'\ncase b={b} n={n} h={h} hk={hk} d={d} w1={w1} w2={w2} shared={shared}', flush=True)
+    ins = U.make_inputs(b, n, h, hk, d, seed=n + d, std=1.0)
+    with_saved, without = (U.hip_abi_fwd_bwd(*ins, w1, w2, use_saved, shared=shared)[2] for use_saved in (True, False))
+    for name, x, y in zip(('dq', 'dk1', 'dk2', 'dv1'), with_saved, without):
+        assert bool(torch.isfinite(x).all()) and torch.equal(x, y), name
+
+
 @pytest.mark.parametrize('d', [65, 80, 96, 97])
 @pytest.mark.parametrize('b,n,h,hk,w1,w2', [(1, 1, 1, 1, 4, 3), (1, 75, 4, 2, 40, 41),
                                             (8, 40, 66, 33, 16, 9)])     # the last: more query tiles than are shared out
