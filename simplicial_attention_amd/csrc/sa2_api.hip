@@ -609,8 +609,9 @@ static int launch_dv2_from_saved(const sa2_problem *prob, const QLaunch &L, hipS
 
 // Up to two dV2 blocks per CU the chains of loads of single workgroups are what dV2, dK2 and dQ take: one launch.  Measured against
 // two at 1 to 512 dV2 blocks, 1 to 16 query heads per key/value head, w2 1 to 500 and D = 32, 64, 128, it takes 0.4 to 0.9 of their time; at
-// 512 blocks (1 x 16 (4 kv) x 4096 rows), us, two and one: D = 64 w2 2 25.2, 22.5; w2 16 46.2, 39.2; w2 128 301, 258; D = 128 w2 2 42, 25; w2 128
-// 498, 453.  Beyond 512 the grids are long enough for blocks of one size each.
+// 512 blocks (1 x 16 (4 kv) x 4096 rows), us, two and one: D = 64 w2 2 25.2, 18.7; w2 16 46.2, 36.9; w2 128 301, 258; D = 128 w2 2 42, 25; w2 128
+// 498, 453.  The line lies on the safe side: at 2048 blocks one launch of D = 32 and 64 loses at the shortest second windows (w2 2, 1 x 4 x 16384
+// rows of 32: 17.3, 19.8), at 1024 it does not (13.8, 13.0; D = 128 w2 32, 1 x 16 (4 kv) x 8192 rows: 292, 253).
 static int launch_small_grid_merge(const sa2_problem *prob, const QLaunch &L, hipStream_t s) {
     const int64_t k_rows = (int64_t)prob->batch * prob->kv_heads * prob->seq_len, q_rows = (int64_t)prob->batch * prob->heads * prob->seq_len;
     SA2_FOR_DIM_HEAD(prob->dim_head, {

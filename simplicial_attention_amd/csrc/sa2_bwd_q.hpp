@@ -555,7 +555,10 @@ __device__ __forceinline__ void dv2_from_saved_block(const KParams &p, const int
             if constexpr (GROUPS) {
 #pragma unroll
                 for (int x0 = 0; x0 < 32 / OG; x0 += 8) {
-                    if (x0 > 0) request(x0);
+                    if (x0 > 0) {
+                        if (x0 * OG >= nl) break;         // (D = 64, up to 16 offsets: there are no second eight)
+                        request(x0);
+                    }
 #pragma unroll
                     for (int x = 0; x < 8; ++x)
                         if (og + (x0 + x) * OG < nl) add(og + (x0 + x) * OG, ahead[x]);

@@ -43,6 +43,7 @@ def test_forward_in_shares(b, n, h, hk, w1, w2, d):
 @pytest.mark.parametrize('shared', [True, False], ids=['shared', 'unshared'])
 @pytest.mark.parametrize('b,n,h,hk,w1,w2', [
     (1, 1, 1, 1, 4, 3), (1, 33, 3, 1, 16, 9), (1, 70, 4, 2, 70, 33), (1, 257, 2, 2, 40, 128),
+    (1, 70, 2, 1, 33, 16), (1, 70, 2, 1, 33, 17), (1, 113, 2, 2, 33, 49),      # eight offsets per group and one more, in either block of 32
     (8, 33, 32, 32, 8, 5),         # 512 blocks of dV2 rows: the last grid that takes one launch
     (8, 33, 33, 33, 8, 5),         # 528: the first that takes two
 ])
