@@ -202,8 +202,8 @@ int sa2_bwd_split(const sa2_problem *prob,
                   const sa2_tensor *dv1, const sa2_tensor *dv2,
                   void *workspace, int64_t workspace_bytes, void *hip_stream);
 
-/* The same for heads of fewer channels padded to dim_head: the channels from `channels` on are zero in q, k1, k2, v1, v2, out and
- * dout, and kernels may leave the products over them out.  The gradients are written with dim_head channels; those of the
+/* The same for heads of fewer channels padded to dim_head: the channels from `channels` (1 to dim_head) on are zero in q, k1, k2, v1,
+ * v2, out and dout, and kernels may leave the products over them out.  The gradients are written with dim_head channels; those of the
  * padding mean nothing. */
 int sa2_bwd_split_padded(const sa2_problem *prob, int32_t channels,
                          const sa2_tensor *q, const sa2_tensor *k1, const sa2_tensor *k2,

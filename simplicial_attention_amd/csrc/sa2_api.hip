@@ -755,7 +755,9 @@ int sa2_bwd_split_padded(const sa2_problem *prob, int32_t channels, const sa2_te
                          const sa2_tensor *dout, const float *lse, const sa2_saved *saved, float *delta_ws, const sa2_tensor *dq,
                          const sa2_tensor *dk1, const sa2_tensor *dk2, const sa2_tensor *dv1, const sa2_tensor *dv2, void *workspace,
                          int64_t workspace_bytes, void *hip_stream) {
-    if (channels < 1) return fail(SA2_ERR_BAD_SHAPE, "channels = %d: at least one", (int)channels);
+    SA2_TRY(check_problem(prob));
+    if (channels < 1 || channels > prob->dim_head)
+        return fail(SA2_ERR_BAD_SHAPE, "channels=%d: 1 to dim_head=%d of them are not padding", (int)channels, prob->dim_head);
     return bwd_all(true, channels, prob, q, k1, k2, v1, v2, out, out_residual, dout, lse, saved, delta_ws, dq, dk1, dk2, dv1, dv2, workspace,
                    workspace_bytes, hip_stream);
 }

@@ -283,6 +283,26 @@ def test_saved_partials_budget_is_global_per_device(monkeypatch):
     assert not _PartialsBudget().admit(3 * gib, 'cuda:0', total)
 
 
+@pytest.mark.parametrize('d', [32, 64, 128, 256])
+def test_channel_counts_that_no_padded_head_has_are_refused(lib, d):
+    """sa2_bwd_split_padded takes 1 to dim_head channels; the problem itself is checked before them."""
+    prob = _native.problem(1, 64, 2, 1, d, 16, 4, True, 0.1)
+    t, lse = _dummy(), ctypes.c_void_p(0x2000)
+    need = lib.sa2_bwd_split_workspace_bytes(prob, 0)
+
+    def call(prob, channels, ws_bytes):
+        return lib.sa2_bwd_split_padded(prob, channels, t, t, t, t, t, t, None, t, lse, None, lse, t, t, t, t, t, lse, ws_bytes, None)
+
+    for channels in (0, -1, d + 1, 2 ** 31 - 1):
+        assert call(prob, channels, need) == 2
+        assert b'channels' in lib.sa2_last_error()
+    assert call(None, 1, need) == 1
+    assert call(_native.problem(1, 64, 2, 1, 96, 16, 4, True, 0.1), 97, need) == 3
+    for channels in (1, d):                  # (as far as the workspace, which is a byte short)
+        assert call(prob, channels, need - 1) == 2
+        assert b'workspace' in lib.sa2_last_error()
+
+
 @pytest.mark.parametrize('d', [64, 128, 256])
 def test_rows_beyond_the_reach_of_the_kernels_are_refused(lib, d):
     """32-bit addresses inside a 32-row tile: operands whose rows lie further apart are refused before a launch."""
