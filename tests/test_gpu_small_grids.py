@@ -73,7 +73,9 @@ def test_partials_do_not_reach_the_other_gradients(b, n, h, hk, w1, w2, d, share
 
 @pytest.mark.parametrize('d', [65, 80, 96, 97])
 @pytest.mark.parametrize('b,n,h,hk,w1,w2', [(1, 1, 1, 1, 4, 3), (1, 75, 4, 2, 40, 41),
-                                            (8, 40, 66, 33, 16, 9)])     # the last: more query tiles than are shared out
+                                            (8, 40, 66, 33, 16, 9),      # more query tiles than are shared out
+                                            (1, 200, 4, 2, 100, 12),     # lower edge, interior and diagonal tiles: shared out,
+                                            (8, 200, 20, 10, 100, 3)])   # and in undivided walks
 def test_narrow_heads_on_the_kernels_of_wide_ones(b, n, h, hk, w1, w2, d):
     """Up to 96 channels padded to 128 leave the products over the last 32 out; 97 takes them all."""
     print(f'\ncase b={b} n={n} h={h} hk={hk} d={d} w1={w1} w2={w2}', flush=True)
@@ -81,6 +83,64 @@ def test_narrow_heads_on_the_kernels_of_wide_ones(b, n, h, hk, w1, w2, d):
     ref_out, _, ref_grads = U.oracle_fwd_bwd(*ins, w1, w2)
     out, grads = U.hip_fwd_bwd(*ins, w1, w2)
     U.check_all(out, grads, ref_out, ref_grads)
+
+
+@pytest.mark.parametrize('dtype,dim_qk,dim_v', [(torch.float16, 96, 70), (torch.float16, 65, 96), (torch.float32, 40, 80), (torch.bfloat16, 96, 97)])
+@pytest.mark.parametrize('b,n,h,hk,w1,w2', [(1, 200, 4, 2, 100, 12), (8, 200, 20, 10, 100, 3)])
+def test_narrow_heads_with_values_of_another_width(b, n, h, hk, w1, w2, dtype, dim_qk, dim_v):
+    """The wider of the two head dimensions decides which products are left out.  The output gradients are scaled up by a power of two, as
+    float16 training scales its loss, and the gradients back down: the rms of dq is about 1e-6 here, of which the rounding to float16's
+    subnormal spacing, 2^-24 / sqrt(12) = 1.7e-8, would alone be more than 1 %."""
+    from simplicial_attention_amd import sliding_two_simplicial_attn
+    print(f'\ncase b={b} n={n} h={h} hk={hk} dim_qk={dim_qk} dim_v={dim_v} w1={w1} w2={w2} {dtype}', flush=True)
+    q, k1, k2 = U.make_inputs(b, n, h, hk, dim_qk, seed=dim_qk, std=dim_qk ** -0.5)[:3]
+    _, v1, v2, _, _, dout = U.make_inputs(b, n, h, hk, dim_v, seed=1000 + dim_v, std=dim_v ** -0.5)
+    ref_out, _, ref_grads = U.oracle_fwd_bwd(q, k1, k2, v1, v2, dout, w1, w2)
+    loss_scale = 2.0 ** 10
+    ts = [t.to(dtype).cuda().requires_grad_(True) for t in (q, k1, k2, v1, v2)]
+    out = sliding_two_simplicial_attn(ts[0], (ts[1], ts[2]), (ts[3], ts[4]), w1=w1, w2=w2)
+    grads = torch.autograd.grad(out, ts, (dout * loss_scale).to(dtype).cuda())
+    U.check_all(out, [g.float() / loss_scale for g in grads], ref_out, ref_grads)
+
+
+@pytest.mark.parametrize('channels', [1, 40, 65, 96, 97])
+@pytest.mark.parametrize('use_saved', [True, False], ids=['saved', 'recomputed'])
+@pytest.mark.parametrize('b,n,h,hk,w1,w2', [(1, 200, 4, 2, 100, 12), (8, 200, 20, 10, 100, 3)])
+def test_products_over_padding_add_nothing(b, n, h, hk, w1, w2, use_saved, channels):
+    """sa2_bwd_split_padded on heads of 128 with zero channels: what is left out would have added zeros to fp32 sums, so every gradient
+    has the bits of the call that takes all channels."""
+    print(f'\ncase b={b} n={n} h={h} hk={hk} channels={channels} w1={w1} w2={w2} saved={use_saved}', flush=True)
+    ins = U.make_inputs(b, n, h, hk, 128, seed=channels, std=1.0)
+    for t in ins:
+        t[..., channels:] = 0
+    scale = channels ** -0.5
+    few, every = (U.hip_abi_fwd_bwd(*ins, w1, w2, use_saved, scale, shared=True, channels=c)[2] for c in (channels, 128))
+    for name, x, y in zip(('dq', 'dk1', 'dk2', 'dv1', 'dv2'), few, every):
+        x, y = x[..., :channels], y[..., :channels]
+        assert bool(torch.isfinite(x).all()) and torch.equal(x, y), name
+
+
+@pytest.mark.parametrize('d', [32, 64, 128])
+@pytest.mark.parametrize('b,n,h,hk,w1,w2', [(1, 128, 8, 1, 40, 33), (1, 70, 4, 2, 70, 128), (1, 200, 8, 1, 128, 64)])
+def test_shares_merged_from_a_poisoned_workspace(b, n, h, hk, w1, w2, d):
+    """Shared query tiles with saved partials, every byte of scratch and results NaN before the call: a share's row that is read has been
+    written, twice the same bits, and the sums are those of sa2_bwd in another order."""
+    from simplicial_attention_amd import _native
+    lib = _native.load()
+    print(f'\ncase b={b} n={n} h={h} hk={hk} d={d} w1={w1} w2={w2}', flush=True)
+    prob = _native.problem(b, n, h, hk, d, w1, w2, True, d ** -0.5)
+    # (scatter rows and fp32 dq rows of several shares: the query tiles are shared out)
+    sets, rest = divmod(lib.sa2_bwd_split_workspace_bytes(prob, 1), lib.sa2_bwd_workspace_bytes(prob) // 2 + b * h * n * d * 4)
+    assert sets > 1 and rest == 0
+    ins = U.make_inputs(b, n, h, hk, d, seed=5, std=d ** -0.5)
+    one = U.hip_abi_fwd_bwd(*ins, w1, w2, True)[2]
+    shares, again = (U.hip_abi_fwd_bwd(*ins, w1, w2, True, shared=True)[2] for _ in range(2))
+    for name, x, y, z in zip(('dq', 'dk1', 'dk2', 'dv1', 'dv2'), one, shares, again):
+        assert torch.equal(y, z), name
+        x, y = x.float(), y.float()
+        # bf16 roundings of fp32 sums that agree to about 1e-5: one bf16 step (2^-7) apart at most, 2^-9 on average
+        assert bool(torch.isfinite(y).all()) and float((x - y).norm() / x.norm()) <= 2.0 ** -9, name
+        assert bool(((x - y).abs() <= 2.0 ** -7 * x.abs() + 1e-5 * float(x.abs().max())).all()), name
 
 
 @pytest.mark.parametrize('src_type,dst_type', [(torch.float32, torch.bfloat16), (torch.float16, torch.bfloat16), (torch.bfloat16, torch.float32),
