@@ -134,7 +134,7 @@ def kernel_symbol(entry, D, w2):
     if entry == 'fwd':
         return 'sa2::fwd2_kernel<128, false>' if D == 128 and w2 > 12 else 'sa2::fwd_kernel<%d, false>' % D
     if entry == 'bwd_dq_dk2_pass':
-        return 'sa2::bwd_q_kernel<%d, true, false>' % D
+        return 'sa2::bwd_q_kernel<%d, true, false, %d>' % (D, D)
     if entry == 'bwd_dkv1':
         # (the entry point sa2_bwd_dkv1 has no workspace and always runs one workgroup per key slab: PARTS = false)
         return 'sa2::bwd_kv8_kernel<%d, %d, false>' % (D, 3 if D == 128 else 2)

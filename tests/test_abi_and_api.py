@@ -223,6 +223,20 @@ def test_naive_attend_matches_oracle_restatement():
     assert S.TwoSimplicialMHA(dim=512, causal=True)(t).shape == t.shape   # tests/test_attn.py:49-55 in the reference
 
 
+@pytest.mark.parametrize('w2', [12, 32])
+@pytest.mark.parametrize('d', [32, 64, 128, 256])
+@pytest.mark.parametrize('entry', ['fwd', 'bwd_dq_dk2_pass', 'bwd_dkv1'])
+def test_bench_names_kernels_that_the_library_holds(lib, entry, d, w2):
+    import importlib.util
+    spec = importlib.util.spec_from_file_location('bench', os.path.join(ROOT, 'bench.py'))
+    bench = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(bench)
+    name, args = re.fullmatch(r'sa2::(\w+)<(.*)>', bench.kernel_symbol(entry, d, w2)).groups()
+    coded = {'true': 'Lb1E', 'false': 'Lb0E'}
+    mangled = '_ZN3sa2%d%sI%sEE' % (len(name), name, ''.join(coded.get(a) or 'Li%sE' % a for a in args.split(', ')))
+    assert mangled.encode() in open(_native.LIB_PATH, 'rb').read()
+
+
 def test_bench_refuses_more_than_one_gpu():
     import subprocess, sys
     r = subprocess.run([sys.executable, os.path.join(ROOT, 'bench.py'), '--gpus', '2'], capture_output=True, text=True)
