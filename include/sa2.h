@@ -43,8 +43,8 @@ extern "C" {
  * cover the split key slabs, sa2_bwd checks every size before its first launch
  * 102: dim_head 256 (its kernels keep no forward partials: the sa2_saved_*_bytes queries return 0 and a non-NULL
  * `saved` is refused)
- * The number stands for what existing calls do.  Functions added beside them (sa2_fwd_ws, sa2_bwd_split, sa2_convert, sa2_wgrad and
- * their size queries) leave it as it is: look them up by name. */
+ * The number stands for what existing calls do.  Functions added beside them (sa2_fwd_ws, sa2_bwd_split, sa2_bwd_split_padded,
+ * sa2_convert, sa2_wgrad and their size queries) leave it as it is: look them up by name. */
 #define SA2_VERSION 102
 
 typedef enum sa2_status {
@@ -158,7 +158,9 @@ int64_t sa2_bwd_workspace_bytes_with_saved(const sa2_problem *prob);
  * dK2/dV2 as partial rows in the workspace), a second one sums the partial rows and
  * the query heads of a group.  No atomics; results are bitwise reproducible.
  * saved may be NULL; if it holds what sa2_fwd wrote for these inputs, dV2 is formed from it
- * instead of from a recomputation of the attention weights. */
+ * instead of from a recomputation of the attention weights: by a kernel in front of the one that
+ * sums, on small grids (up to 512 blocks of 32 rows of the key/value heads) by the same one.  dQ and dK2 have the
+ * same bits with and without it. */
 int sa2_bwd_dq_dkv2(const sa2_problem *prob,
                     const sa2_tensor *q, const sa2_tensor *k1, const sa2_tensor *k2,
                     const sa2_tensor *v1, const sa2_tensor *v2, const sa2_tensor *dout,

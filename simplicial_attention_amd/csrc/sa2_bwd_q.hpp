@@ -20,9 +20,10 @@
 // barrier-separated phases in which wave w owns the d-slice (w + phase) mod 8, so no two waves touch
 // one element at a time and the order is fixed (bitwise reproducible, no atomics).  The rows k that
 // the offsets scatter to live in a 64-row circular buffer (row k in slot (k - i0) mod 64); the eight
-// rows that a round completes go to the fp32 workspace that dk2_dv2_combine_kernel reduces:
+// rows that a round completes go to the fp32 workspace:
 // [tensor 0: dk2, 1: dv2][b][h][tile][32 + halo][D], row x of a tile <-> k = i0 - halo + x, with
-// halo = 8 ceil(w2 / 8) - 1.
+// halo = 8 ceil(w2 / 8) - 1.  combine_rows reduces it, in dk2_dv2_combine_kernel or, on small grids with
+// saved forward partials, in small_grid_merge_kernel, beside dV2.
 #pragma once
 
 #include <type_traits>
