@@ -579,7 +579,7 @@ static int launch_q_mfma(const sa2_problem *prob, const QLaunch &L, int pass, hi
         return after_launch("dq/dk2/dv2");
     }
     // At most 96 channels that are not padding (the package: heads of 65 to 96), with partials saved for dV2.  2 x 6 (2 kv) x 2999
-    // rows of 96 channels, w1 300, w2 20: 253 us with the general instance, 214 with this one.  Without partials both passes are general.
+    // rows of 96 channels, w1 300, w2 20: 243 us with the general instance, 207 with this one.  Without partials both passes are general.
     const bool narrow = prob->dim_head == 128 && L.channels <= 96 && L.use_saved;
     if (narrow) {
         if (L.k.q_splits > 1) hipLaunchKernelGGL((sa2::bwd_q_kernel<128, true, true, 96>), dim3(L.k.q_splits * L.grid), dim3(512), 0, s, L.k, L.ws, L.halo);
