@@ -579,7 +579,7 @@ static int launch_q_mfma(const sa2_problem *prob, const QLaunch &L, int pass, hi
         return after_launch("dq/dk2/dv2");
     }
     // At most 96 channels that are not padding (the package: heads of 65 to 96), with partials saved for dV2.  2 x 6 (2 kv) x 2999
-    // rows of 96 channels, w1 300, w2 20: 243 us with the general instance, 207 with this one.  Without partials both passes are general.
+    // rows of 96 channels, w1 300, w2 20: 243 us with the general instance, 204 with this one.  Without partials both passes are general.
     const bool narrow = prob->dim_head == 128 && L.channels <= 96 && L.use_saved;
     if (narrow) {
         if (L.k.q_splits > 1) hipLaunchKernelGGL((sa2::bwd_q_kernel<128, true, true, 96>), dim3(L.k.q_splits * L.grid), dim3(512), 0, s, L.k, L.ws, L.halo);
@@ -609,9 +609,10 @@ static int launch_dv2_from_saved(const sa2_problem *prob, const QLaunch &L, hipS
 
 // Up to two dV2 blocks per CU the chains of loads of single workgroups are what dV2, dK2 and dQ take: one launch.  Measured against
 // two at 1 to 512 dV2 blocks, 1 to 16 query heads per key/value head, w2 1 to 500 and D = 32, 64, 128, it takes 0.4 to 0.9 of their time; at
-// 512 blocks (1 x 16 (4 kv) x 4096 rows), us, two and one: D = 64 w2 2 25.2, 18.7; w2 16 46.2, 36.9; w2 128 301, 258; D = 128 w2 2 42, 25; w2 128
-// 498, 453.  The line lies on the safe side: at 2048 blocks one launch of D = 32 and 64 loses at the shortest second windows (w2 2, 1 x 4 x 16384
-// rows of 32: 17.3, 19.8), at 1024 it does not (13.8, 13.0; D = 128 w2 32, 1 x 16 (4 kv) x 8192 rows: 292, 253).
+// 512 blocks (1 x 16 (4 kv) x 4096 rows), us in a trace, two and one: D = 32 w2 2 17.6, 15.0; D = 64 w2 2 28.2, 16.2; w2 16 48.2, 33.5; w2 128
+// 328, 254; D = 128 w2 2 39.2, 21.3; w2 128 493, 448.  The line lies on the safe side: at 2048 blocks one launch of D = 32 and 64 loses at the
+// shortest second windows (w2 2, 1 x 4 x 16384 rows of 32: 17.3, 19.8), at 1024 it does not (13.8, 13.0; D = 128 w2 32, 1 x 16 (4 kv) x 8192
+// rows: 292, 253).
 static int launch_small_grid_merge(const sa2_problem *prob, const QLaunch &L, hipStream_t s) {
     const int64_t k_rows = (int64_t)prob->batch * prob->kv_heads * prob->seq_len, q_rows = (int64_t)prob->batch * prob->heads * prob->seq_len;
     SA2_FOR_DIM_HEAD(prob->dim_head, {

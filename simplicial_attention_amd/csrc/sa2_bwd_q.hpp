@@ -58,7 +58,7 @@ struct QCfg {
     static constexpr int PIECES = 32 * PPR;           // ... per tile
     // dQ pass at D = 64: the start values of the logit chains stay in 16 registers for a round (198 of 256; at D = 128 none are
     // left) instead of being copied together at every step.  A step has 12 MFMAs there, and what it issues beside them is the
-    // bound: 918 -> 892 us at 8 x 8 (4 kv) x 2048 rows, w1 512, w2 32.  At D = 32 it is no gain: 694 us there either way, and 2533 us
+    // bound: 919 -> 890 us at 8 x 8 (4 kv) x 2048 rows, w1 512, w2 32.  At D = 32 it is no gain: 694 us there either way, and 2533 us
     // copied, 2580 kept at 2 x 4 x 30000 rows, w1 200, w2 100, where many rounds have few steps each.
     static constexpr bool KEEP_NL = DQ && D == 64;
 };
@@ -73,7 +73,7 @@ __host__ __device__ inline int64_t qk2_ws_floats(int B, int H, int N, int D, int
 
 // CH < D: the channels from CH on are zero in every operand (rows of narrower heads padded to D), and the products over them
 // are left out: their k-slots add zeros to S and dP, their rows of G are zero.  2 x 6 (2 kv) x 2999 rows of 96 channels,
-// w1 300, w2 20: 243 -> 207 us.
+// w1 300, w2 20: 243 -> 204 us.
 template <int D, bool DQ, bool SPLIT = false, int CH = D>
 __global__ __launch_bounds__(512) void bwd_q_kernel(KParams p, float *ws, int halo) {
     using C = QCfg<D, DQ>;
@@ -700,8 +700,8 @@ __global__ __launch_bounds__(256) void dk2_dv2_combine_kernel(KParams p, const f
 // the sum of their latencies, side by side the longest.  As two launches; as one; as one with the first T pieces of dV2 requested
 // ahead of the staging (GROUPS), in us between events around the launches (a kernel trace has 3 us less for the last of each): 1 x 4 x 128
 // rows of 32, w2 128: 40.9, 22.7, 15.9; 1 x 8 (4 kv) x 1000 rows of 64, w2 32: 27.5, 20.7, 16.9; 2 x 6 (2 kv) x 2999 rows of 128, w2 20
-// (nothing ahead at D = 128): 71, 54.  (dK2's shares dealt out to four groups of
-// threads that meet through LDS: 15.9, 16.9, 58, and 30.0 instead of 22.5 at 1 x 16 (4 kv) x 4096 rows of 64, w2 2.)
+// (nothing ahead at D = 128): 71, 54.  (dK2's shares dealt out to four groups of threads that meet through LDS: 15.9, 16.9, 58, and
+// 30.0 instead of 22.5 at 1 x 16 (4 kv) x 4096 rows of 64, w2 2.)
 template <int D>
 struct MergeCfg {
     static constexpr int THREADS = 512, ROWS = THREADS / (D / 8);      // rows of dK2 or dQ per block
